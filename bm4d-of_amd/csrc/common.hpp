@@ -38,11 +38,9 @@ struct StepConst {
 // counted from tb0.
 struct AggRegion { int RX, RY, RT, tb0; };
 
-// Binned ordered aggregation: bins of 8 x 8 pixels x AGG_TB frames; a bin
-// gathers the rows of at most AGG_BPOS patch positions ((7 + sPx)^2 x
-// (AGG_TB + sPt - 1)).
-#define AGG_TB 4
-#define AGG_BPOS 1024
+// Binned ordered aggregation: bins (regions) of 2^lx x 2^ly pixels x 2^lt
+// frames; a patch overlaps at most 8 of them.
+struct BinShape { int lx, ly, lt; };
 
 // stable radix sort passes (sortscan.hip): threads per block, pairs per
 // thread and per block (tile)

@@ -97,16 +97,19 @@ template <int CC> __global__ void agg_exact_kernel(AGG_ARGS);
 __global__ void pack_rows_kernel(const uint32_t *, const uint32_t *, const float *, int64_t, uint32_t, uint32_t,
                                  uint4 *);
 template <int CC, int CAP, int WP> __global__ void agg_chunk_kernel(AGG2_ARGS);
-__global__ void bin_hist1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, int, int, int, uint32_t *);
-__global__ void bin_scatter1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, int, int, int,
+__global__ void bin_hist1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int,
+                                 uint32_t *);
+__global__ void bin_scatter1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int,
                                     const uint32_t *, uint32_t *, uint32_t *);
 __global__ void bin_bounds_kernel(const uint32_t *, const uint32_t *, int64_t, int, uint32_t *);
 __global__ void rs_hist_kernel(const uint32_t *, const uint32_t *, int, int, uint32_t *);
 __global__ void rs_scatter_kernel(const uint32_t *, const uint32_t *, const uint32_t *, int, int, const uint32_t *,
                                   uint32_t *, uint32_t *);
-#define AGGB_ARGS const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, StepConst, \
-	int, int, int, float *, float *
-template <int CC, int NBR, int PQ, int SQ> __global__ void agg_bin_fold_kernel(AGGB_ARGS);
+#define AGGB_ARGS const uint32_t *, const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, \
+	StepConst, int, int, float *, float *
+__global__ void bin_order_kernel(const uint32_t *, int, uint32_t *);
+template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS>
+__global__ void agg_region_fold_kernel(AGGB_ARGS);
 __global__ void band_bounds_kernel(const uint32_t *, const uint32_t *, int, int, uint32_t *);
 __global__ void normalize_kernel(const float *, const float *, const float *, StepConst,
                                  float *);
@@ -665,26 +668,73 @@ void dscan(bm4dof_ctx *ctx, int op, const uint32_t *in, int64_t n_in, int64_t n,
 	HIPCHK(hipGetLastError());
 }
 
-// Binned aggregation: shapes it takes (64-sample patches 4x4x4 or 8x8x1,
-// one block overlapping at most 2 x 2 tile interiors) and the list sizes
-// (at most 8 bins per row, pair counts in 32 bits; rows and frames below
-// 2^16, as the row records hold them in 16 bits each).
+// Binned aggregation: shapes it takes (4x4x4 patches and patches of one
+// frame, tiles of at least 8 x 8 pixels) and the list sizes (at most 8 bins
+// per row, pair counts in 32 bits; rows and frames below 2^16, as the row
+// records hold them in 16 bits each).
 bool agg_binned_ok(const bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
 {
 	return ctx->agg_binned && ctx->agg_chunked && sc.wTmp >= 8 && sc.hTmp >= 8 &&
-	       ((sc.sPx == 4 && sc.sPt == 4) || (sc.sPx == 8 && sc.sPt == 1)) &&
+	       ((sc.sPx == 4 && sc.sPt == 4) || (sc.sPt == 1 && sc.sPx <= 16)) &&
 	       (sc.C == 1 || sc.C == 3 || sc.C == 4) && sc.H < 65536 && sc.F < 65536 &&
 	       8 * Mub < ((int64_t)1 << 32) - RS_TILE;
 }
 
-struct BinGrid { int nbx, nby, nbins; };
-BinGrid bin_grid(const StepConst &sc)
+struct BinGrid {
+	BinShape s;
+	int nbx, nby, nbins;
+};
+BinGrid bin_grid_of(const StepConst &sc, BinShape s)
 {
 	BinGrid g;
-	g.nbx = (sc.W + 7) / 8;
-	g.nby = (sc.H + 7) / 8;
-	g.nbins = g.nbx * g.nby * ((sc.F + AGG_TB - 1) / AGG_TB);
+	g.s = s;
+	g.nbx = (sc.W + (1 << s.lx) - 1) >> s.lx;
+	g.nby = (sc.H + (1 << s.ly) - 1) >> s.ly;
+	g.nbins = g.nbx * g.nby * ((sc.F + (1 << s.lt) - 1) >> s.lt);
 	return g;
+}
+
+// One wave folds a region.  4x4x4 patches: 8 x 8 pixels over 32 frames list
+// a row 1.9 times instead of 3.3 times over 4 frames (960x540x20, step 2:
+// 7.5 against 10.0 ms), as long as they give the chip about six waves per CU
+// (480x270x12, 2040 regions: 1.80 against 1.86 ms; 64x48x6, 48 regions: no
+// difference); 16 x 8 and 16 x 16 pixels were slower (10.1 ms, 10.7 ms: their
+// sums leave fewer waves per CU).  Colour stops at 16 frames: its sums take
+// two to four times the LDS.  8x8x1 patches gain nothing from more frames.
+// Other one-frame patches may overlap three bins of 8.
+constexpr int BIN_LONG_MIN = 1536;
+BinGrid bin_grid(const StepConst &sc)
+{
+	if (sc.sPx == 4 && sc.sPt == 4) {
+		const BinGrid g = bin_grid_of(sc, {3, 3, sc.C == 1 ? 5 : 4});
+		return g.nbins >= BIN_LONG_MIN ? g : bin_grid_of(sc, {3, 3, 2});
+	}
+	return bin_grid_of(sc, sc.sPx == 8 ? BinShape{3, 3, 2} : BinShape{4, 4, 0});
+}
+
+// The fold of a step's bins and its LDS bytes (one frame of sums per frame
+// of the region the video has).
+struct Fold {
+	void (*kernel)(AGGB_ARGS);
+	size_t lds;
+};
+template <int CC> Fold fold_of(const StepConst &sc, const BinShape &s)
+{
+	Fold f;
+	int fs = 384;
+	if (sc.sPx == 4 && sc.sPt == 4) {
+		f.kernel = s.lt > 2 ? agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68>
+		                    : agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68>;
+		fs = 68;
+	} else if (sc.sPx == 8) {
+		f.kernel = agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64>;
+		fs = 64;
+	} else
+		f.kernel = sc.P <= 64    ? agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384>
+		           : sc.P <= 128 ? agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384>
+		                         : agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384>;
+	f.lds = (size_t)std::min(1 << s.lt, sc.F) * fs * (CC == 1 ? 8 : CC == 3 ? 16 : 32);
+	return f;
 }
 
 // Device buffers of the bin lists for Mub rows: the first pass's digit
@@ -692,7 +742,7 @@ BinGrid bin_grid(const StepConst &sc)
 // value buffers, 8 Mub each), digit counts per radix tile, list starts per
 // bin.  The sorted values end in bin_list (v0).
 struct BinBufs {
-	uint32_t *off1, *k0, *v0, *k1, *v1, *hist, *hoff, *boff;
+	uint32_t *off1, *k0, *v0, *k1, *v1, *hist, *hoff, *boff, *order;
 	int nt1, nblk;   // tiles of the first pass (rows) and of the later ones (pairs)
 };
 BinBufs bin_bufs(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
@@ -709,7 +759,8 @@ BinBufs bin_bufs(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
 	q.v1 = ctx->bin_v1.as<uint32_t>(npair);
 	q.hist = ctx->bin_hist.as<uint32_t>((size_t)256 * q.nblk);
 	q.hoff = ctx->bin_hoff.as<uint32_t>((size_t)256 * q.nblk + 1);
-	q.boff = ctx->bin_off.as<uint32_t>((size_t)bg.nbins + 1);
+	q.boff = ctx->bin_off.as<uint32_t>((size_t)2 * bg.nbins + 1);
+	q.order = q.boff + bg.nbins + 1;
 	return q;
 }
 
@@ -726,12 +777,12 @@ void agg_bin_lists(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub, const uint
 	// the passes alternate between the buffers and end in bin_k0 / bin_list
 	uint32_t *kout = passes % 2 ? q.k0 : q.k1, *vout = passes % 2 ? q.v0 : q.v1;
 	// pass 0 from the rows; off1[256 nt1] = the pair count
-	hipLaunchKernelGGL(bin_hist1_kernel, dim3(side_grid(ctx, q.nt1)), dim3(64), 0, st, epos, Mp, Mub, sc, bg.nbx,
-	                   bg.nby, q.nt1, q.hist);
+	hipLaunchKernelGGL(bin_hist1_kernel, dim3(side_grid(ctx, q.nt1)), dim3(64), 0, st, epos, Mp, Mub, sc, bg.s,
+	                   bg.nbx, bg.nby, q.nt1, q.hist);
 	dscan(ctx, 0, q.hist, (int64_t)256 * q.nt1, (int64_t)256 * q.nt1 + 1, q.off1, true);
 	const uint32_t *np = q.off1 + (size_t)256 * q.nt1;
 	hipLaunchKernelGGL(bin_scatter1_kernel, dim3(side_grid(ctx, q.nt1)), dim3(64), 0, st, epos, Mp, Mub, sc,
-	                   bg.nbx, bg.nby, q.nt1, q.off1, kout, vout);
+	                   bg.s, bg.nbx, bg.nby, q.nt1, q.off1, kout, vout);
 	HIPCHK(hipGetLastError());
 	uint32_t *kin = kout, *vin = vout;
 	kout = kin == q.k0 ? q.k1 : q.k0;
@@ -749,6 +800,7 @@ void agg_bin_lists(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub, const uint
 	const int64_t nub = 8 * Mub;
 	hipLaunchKernelGGL(bin_bounds_kernel, dim3(side_grid(ctx, (nub + 1 + 1023) / 1024)), dim3(64), 0, st,
 	                   q.k0, np, nub, bg.nbins, q.boff);
+	hipLaunchKernelGGL(bin_order_kernel, dim3(1), dim3(1024), 0, st, q.boff, bg.nbins, q.order);
 	HIPCHK(hipGetLastError());
 }
 
@@ -775,23 +827,14 @@ void aggregate_chunk(bm4dof_ctx *ctx, const StepConst &sc, const std::vector<uin
 			// the bin lists were built on the side stream (agg_bin_lists)
 			const BinGrid bg = bin_grid(sc);
 			const BinBufs q = bin_bufs(ctx, sc, Mub);
-			const uint32_t *boff = q.boff, *blist = q.v0;
-			auto fold = agg_bin_fold_kernel<1, 32, 16, 4>;
-			if (sc.sPx == 4) {
-				if (sc.C == 3) fold = agg_bin_fold_kernel<3, 16, 16, 4>;
-				else if (sc.C == 4) fold = agg_bin_fold_kernel<4, 16, 16, 4>;
-			} else {
-				fold = sc.C == 1 ? agg_bin_fold_kernel<1, 32, 16, 16>
-				                 : sc.C == 3 ? agg_bin_fold_kernel<3, 16, 16, 16> : agg_bin_fold_kernel<4, 16, 16, 16>;
-			}
-			const unsigned nb8 = (unsigned)(((size_t)bg.nbins + 7) / 8 * 8);
-			hipLaunchKernelGGL(fold, dim3(nb8), dim3(64), 0, ctx->stream, boff, blist, d_erec, est, win, sc, bg.nbx,
-			                   bg.nby, bg.nbins, num, wsum);
+			const Fold f = sc.C == 1 ? fold_of<1>(sc, bg.s) : sc.C == 3 ? fold_of<3>(sc, bg.s) : fold_of<4>(sc, bg.s);
+			hipLaunchKernelGGL(f.kernel, dim3((unsigned)bg.nbins), dim3(64), f.lds, ctx->stream, q.boff, q.order, q.v0,
+			                   d_erec, est, win, sc, bg.nbx, bg.nby, num, wsum);
 			HIPCHK(hipGetLastError());
 			ctx->agg_blocks += (uint64_t)bg.nbins;
-			ctx->agg_region[0] = 8;
-			ctx->agg_region[1] = 8;
-			ctx->agg_region[2] = AGG_TB;
+			ctx->agg_region[0] = 1 << bg.s.lx;
+			ctx->agg_region[1] = 1 << bg.s.ly;
+			ctx->agg_region[2] = 1 << bg.s.lt;
 			return;
 		}
 		const dim3 cgrid((unsigned)(((size_t)(t1c - t0c) * ((sc.W + 7) / 8) * ((sc.H + 7) / 8) + 7) / 8 * 8));

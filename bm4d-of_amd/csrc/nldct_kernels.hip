@@ -3184,35 +3184,26 @@ __global__ void band_bounds_kernel(const uint32_t *__restrict__ base, const uint
 
 // computeWeightedAggregation, nldct.cpp:2436-2448.
 // ---------------------------------------------------------------------------
-// Ordered aggregation by bins of 8 x 8 pixels x AGG_TB frames.
-//
-// bin_hist1_kernel / bin_scatter1_kernel (side stream, beside the filter):
-// every row e gives one (bin, e) pair per bin its patch overlaps, in
-// increasing e, sorted stably by the bin's low 8 bits straight from the
-// rows; the further 8-bit passes (sortscan.hip) then leave each bin's rows
-// in increasing e, and bin_bounds_kernel marks where each bin's list
-// starts.  agg_bin_fold_kernel: one wave per bin, lane = pixel
-// of the 8 x 8 block, AGG_TB running sums per lane (one per frame of the
-// bin).  The bin's list is read in chunks of NBR rows; each row's slices at
-// the bin's frames are staged once in LDS and added, frame by frame, into
-// the lanes whose pixel the row covers, in increasing e: for every pixel the
-// rows come in the order computeAggregationStep{1,2} adds them
-// (nldct.cpp:2284-2300, 2376-2393), one float addition at a time, so the
-// sums are those of the per-frame kernels above.
+// Ordered aggregation by bins (regions of a BinShape).  The rows of every
+// bin are listed in increasing e beside the filter: (bin, e) pairs, one per
+// bin a row's patch overlaps, in increasing e, sorted stably by bin
+// (bin_hist1 / bin_scatter1_kernel, then rs_hist / rs_scatter_kernel); one
+// wave then folds a bin's list into the bin's sums in list order
+// (agg_region_fold_kernel).
 // ---------------------------------------------------------------------------
 
 // bins of row e's patch (x blocks, y blocks, frame bins)
-__device__ __forceinline__ void bin_span(uint32_t q, const StepConst &sc, int &bx0, int &bx1, int &by0, int &by1,
-                                         int &bt0, int &bt1)
+__device__ __forceinline__ void bin_span(uint32_t q, const StepConst &sc, const BinShape &bs, int &bx0, int &bx1,
+                                         int &by0, int &by1, int &bt0, int &bt1)
 {
 	int qx, qy, qt;
 	pos_decode(q, sc.W, sc.WH, qx, qy, qt);
-	bx0 = qx >> 3;
-	bx1 = (qx + sc.sPx - 1) >> 3;
-	by0 = qy >> 3;
-	by1 = (qy + sc.sPx - 1) >> 3;
-	bt0 = qt / AGG_TB;
-	bt1 = (qt + sc.sPt - 1) / AGG_TB;
+	bx0 = qx >> bs.lx;
+	bx1 = (qx + sc.sPx - 1) >> bs.lx;
+	by0 = qy >> bs.ly;
+	by1 = (qy + sc.sPx - 1) >> bs.ly;
+	bt0 = qt >> bs.lt;
+	bt1 = (qt + sc.sPt - 1) >> bs.lt;
 }
 
 // bin key of the pairs of a row, in the order they are listed: frame bins,
@@ -3220,7 +3211,7 @@ __device__ __forceinline__ void bin_span(uint32_t q, const StepConst &sc, int &b
 #define BIN_FOR_PAIRS(q, KEY, BODY)                                                                  \
 	{                                                                                                \
 		int bx0_, bx1_, by0_, by1_, bt0_, bt1_;                                                      \
-		bin_span(q, sc, bx0_, bx1_, by0_, by1_, bt0_, bt1_);                                         \
+		bin_span(q, sc, bs, bx0_, bx1_, by0_, by1_, bt0_, bt1_);                                         \
 		for (int bt_ = bt0_; bt_ <= bt1_; bt_++)                                                     \
 			for (int by_ = by0_; by_ <= by1_; by_++)                                                 \
 				for (int bx_ = bx0_; bx_ <= bx1_; bx_++) {                                           \
@@ -3235,7 +3226,7 @@ __device__ __forceinline__ void bin_span(uint32_t q, const StepConst &sc, int &b
 // (hist[d * ntiles + tile]).
 __global__ __launch_bounds__(64)
 void bin_hist1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restrict__ Mp, int64_t Mub,
-                      StepConst sc, int nbx, int nby, int ntiles, uint32_t *__restrict__ hist)
+                      StepConst sc, BinShape bs, int nbx, int nby, int ntiles, uint32_t *__restrict__ hist)
 {
 	__shared__ uint32_t h[256];
 	const int lane = threadIdx.x;
@@ -3270,7 +3261,7 @@ void bin_hist1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restr
 // digit's offset), as rs_scatter_kernel does for the later passes.
 __global__ __launch_bounds__(64)
 void bin_scatter1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restrict__ Mp, int64_t Mub,
-                         StepConst sc, int nbx, int nby, int ntiles, const uint32_t *__restrict__ offs,
+                         StepConst sc, BinShape bs, int nbx, int nby, int ntiles, const uint32_t *__restrict__ offs,
                          uint32_t *__restrict__ kout, uint32_t *__restrict__ vout)
 {
 	__shared__ uint32_t base[256];
@@ -3304,9 +3295,9 @@ void bin_scatter1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__re
 				uint64_t m = __ballot(valid);
 #pragma unroll
 				for (int bit = 0; bit < 8; bit++) {
-					const bool bs = (d >> bit) & 1u;
-					const uint64_t bb = __ballot(valid && bs);
-					m &= bs ? bb : ~bb;
+					const bool on = (d >> bit) & 1u;
+					const uint64_t bb = __ballot(valid && on);
+					m &= on ? bb : ~bb;
 				}
 				const uint32_t rk = (uint32_t)__popcll(m & lt);
 				const uint32_t bd = base[d];
@@ -3363,280 +3354,276 @@ void bin_bounds_kernel(const uint32_t *__restrict__ keys, const uint32_t *__rest
 	}
 }
 
-// CC channels; NBR (<= 32) rows per chunk; patches of 4 PQ samples, frame
-// slices of 4 SQ samples (PQ <= 16).
-//
-// LDS, in floats: a zero area Z, then NBR + 1 slots of CC P + 4 floats.
-// Slot j >= 0 holds chunk row j: its samples (channel-major) and, after
-// them, its record (byte offset wb4 of the window / sample index of the
-// block pixel (0, 0) at the bin's first frame, weight).  Slot -1 holds the
-// window (its first P floats) and the record (-4 |Z|, +0): a round's
-// missing rows have index -1 (the lowest set bit of an empty mask), so
-// their samples and window values are read from Z, and every round adds
-// RPR terms without a select (adding +0 leaves a sum that is not -0
-// unchanged, and these sums start at +0 and never become -0).
-template <int CC, int NBR, int PQ, int SQ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CC == 1 ? 4 : 3)))
-void agg_bin_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *__restrict__ blist,
-                         const uint4 *__restrict__ erec, const float *__restrict__ est,
-                         const float *__restrict__ win, StepConst sc, int nbx, int nby, int nbins,
-                         float *__restrict__ num, float *__restrict__ wsum)
+// bits [a, b) of a word, 0 <= a, a < 64; none when b <= a
+__device__ __forceinline__ uint64_t bits64(int a, int b)
 {
-	static_assert(NBR <= 32, "row masks are 32 bits");
-	constexpr int TB = AGG_TB;
-	constexpr int P = 4 * PQ, SL = 4 * SQ, QR = CC * PQ;   // QR: float4 of one row's samples
-	constexpr int QS = QR + 1;                             // float4 per slot (samples, record)
-	constexpr int SPL = (NBR * QR + 63) / 64;              // float4 staged per lane per chunk
-	constexpr int RPR = CC == 1 ? 4 : 2;                   // rows folded per round
-	static_assert(SPL * 64 == NBR * QR, "the staging fills the chunk's slots exactly");
-	constexpr int ZR = (TB - 1) * SL + 64;                 // span of the lane offsets f SL + pix_l
-	constexpr int ZQ = ((CC - 1) * P + ZR + 3) / 4;        // float4 of Z
-	__shared__ __align__(16) float4 lds4[ZQ + (NBR + 1) * QS];
-	float *const slotm1 = reinterpret_cast<float *>(lds4 + ZQ);   // slot -1
-	float *const slot0 = slotm1 + 4 * QS;                          // slot 0
-	constexpr int SB = 16 * QS;                                    // bytes per slot
-	constexpr int RECB = 4 * CC * P;                               // record offset in a slot
-	// per row of a chunk (two chunks in flight): (row index e, bit dt set
-	// for the slices at the bin's frames)
-	__shared__ uint2 rowm[2][NBR];
+	const uint64_t hi = b >= 64 ? ~0ull : (1ull << max(b, 0)) - 1ull;
+	return b > a ? hi & (~0ull << a) : 0ull;
+}
+
+// order[i] = the bins by falling pair count (in classes of an eighth of a
+// power of two), so that the longest lists start first: matches gather on
+// some pixels, and a long list started last is the launch's tail (step 2 of
+// 960x540x20: 8.4 -> 7.5 ms).  One block.
+__global__ __launch_bounds__(1024)
+void bin_order_kernel(const uint32_t *__restrict__ boff, int nbins, uint32_t *__restrict__ order)
+{
+	__shared__ uint32_t h[256];
+	const int tid = threadIdx.x;
+	if (tid < 256) h[tid] = 0;
+	__syncthreads();
+	auto cls = [&](int b) {
+		const uint32_t n = boff[b + 1] - boff[b];
+		const uint32_t c = n ? (__float_as_uint((float)n) >> 20) - (127u << 3) + 1u : 0u;
+		return 255u - min(c, 255u);
+	};
+	for (int b = tid; b < nbins; b += 1024) atomicAdd(&h[cls(b)], 1u);
+	__syncthreads();
+	if (tid < 64) {
+		const uint32_t c0 = h[4 * tid], c1 = h[4 * tid + 1], c2 = h[4 * tid + 2], c3 = h[4 * tid + 3];
+		const uint32_t t = c0 + c1 + c2 + c3;
+		const uint32_t ex = (uint32_t)wave_incl_scan((int)t) - t;
+		h[4 * tid] = ex;
+		h[4 * tid + 1] = ex + c0;
+		h[4 * tid + 2] = ex + c0 + c1;
+		h[4 * tid + 3] = ex + c0 + c1 + c2;
+	}
+	__syncthreads();
+	for (int b = tid; b < nbins; b += 1024) order[atomicAdd(&h[cls(b)], 1u)] = (uint32_t)b;
+}
+
+// running sums of one pixel
+template <int CC> struct __align__(CC == 1 ? 8 : 16) RegionAcc {
+	float w, n[CC];
+};
+
+// One wave per region of RX x RY pixels x RT frames; lane = sample of a
+// patch (sample lane + 64 u in slot u < PS).  The region's sums live in LDS,
+// (CC + 1) planes of RT frames at stride FS, rows at stride RS; a row of the
+// region's list is one LDS add of each covered sample per plane.  A wave's
+// LDS operations execute in order and an add rounds to nearest even like
+// v_add_f32, so every pixel's sum takes its rows in list order, one float
+// addition each: the sums computeAggregationStep{1,2} forms.
+//
+// Nothing in the row loop waits for a sum, only for the samples, which are
+// requested 16 rows ahead; per row it issues five lane reads of what the
+// chunk of 64 records holds (mask, LDS offset, row, weight), the load, and
+// CC + 1 adds.  Lanes outside the region or the row's tile are off: their
+// buffer offset is past the row's end, so they fetch nothing.
+// Strides: 4x4x4 patches meet every LDS bank once per half wave with RS = 20,
+// FS = 16 mod 64; rows of 8 samples with RS = 8 mod 16.
+// One wave per region of RX x RY pixels x RT frames; lane = sample of a
+// patch (sample lane + 64 u in slot u < PS).  The region's sums live in LDS,
+// a pixel's weight and channel sums side by side, rows at stride RS, frames
+// at FS; every row of the region's list reads, adds to and writes the sums of
+// the samples it covers.  A wave's LDS accesses execute in order, so each
+// pixel's sum takes its rows in list order, one float addition each: the
+// sums computeAggregationStep{1,2} forms (nldct.cpp:2284-2300, 2376-2393).
+//
+// Bound: instruction issue, about 25 per row and wave, at some 4.6 TB/s of
+// sample reads.  The samples are requested U rows ahead and nothing else in
+// the row loop waits but the sums' own LDS read; what a row needs (row, LDS
+// offset, weight, mask of the covered samples) is computed for 64 rows at a
+// time, lane = row, and read back by lane.  Lanes outside the region or the
+// interior of the row's tile are off: their buffer offset is past the row's
+// end, so they fetch nothing.  Strides put the 16 lanes an 8-byte access
+// serves at once on different banks.
+//
+// Lane = patch sample against lane = pixel walking masks of staged rows (the
+// form before): every lane of a row's access has a term to add, where the
+// walk filled 17 % of its slots.  960x540x20, step 2 (71 M rows): 14.9 ->
+// 8.4 ms, with the longest lists first (bin_order_kernel) 7.5 ms; step 1
+// 6.0 -> 3.3 ms.  Adding with LDS float atomics instead took 82 ms (about
+// 160 cycles per instruction), pairs of rows without a common pixel read
+// together 9.3 ms.
+template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS>
+__global__ __launch_bounds__(64)
+void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *__restrict__ order,
+                            const uint32_t *__restrict__ blist, const uint4 *__restrict__ erec,
+                            const float *__restrict__ est, const float *__restrict__ win, StepConst sc, int nbx,
+                            int nby, float *__restrict__ num, float *__restrict__ wsum)
+{
+	constexpr int RX = 1 << LX, RY = 1 << LY, RT = 1 << LT;
+	constexpr int U = PS == 1 && CC == 1 ? 16 : 8;   // rows requested ahead
+	using Acc = RegionAcc<CC>;
+	static_assert(RS >= RX && FS >= RY * RS, "the region fits its array");
+	// RT frames, or as many as the video has
+	extern __shared__ char region_lds[];
+	Acc *const acc = reinterpret_cast<Acc *>(region_lds);
 	const int lane = threadIdx.x;
-	// bins are dealt to the 8 XCDs in contiguous eighths (x fastest)
-	const uint32_t per_xcd = ((uint32_t)nbins + 7) / 8;
-	const uint32_t b = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-	if (b >= (uint32_t)nbins) return;
+	const uint32_t b = order[blockIdx.x];
 	const uint32_t k0 = boff[b], k1 = boff[b + 1];
 	if (k0 >= k1) return;
 	const int bx = (int)(b % (uint32_t)nbx);
 	const uint32_t rb = b / (uint32_t)nbx;
-	const int x0 = bx * 8, y0 = (int)(rb % (uint32_t)nby) * 8, t0 = (int)(rb / (uint32_t)nby) * TB;
-	const int sPx = sc.sPx, sPt = sc.sPt;
-	const int lx = lane & 7, ly = lane >> 3;
-	const int x = x0 + lx, y = y0 + ly;
-	const bool valid = x < sc.W && y < sc.H;
-	// the lanes owned by each tile present in the block
-	const int owner = valid ? owner_tile(x, y, sc) : -1;
-	int own_t[4] = {-1, -1, -1, -1};
-	uint64_t own_m[4] = {0, 0, 0, 0};
-	{
-		uint64_t rest = __ballot(valid);
+	const int x0 = bx << LX, y0 = (int)(rb % (uint32_t)nby) << LY, t0 = (int)(rb / (uint32_t)nby) << LT;
+	const int xe = min(x0 + RX, sc.W), ye = min(y0 + RY, sc.H), te = min(t0 + RT, sc.F);
+	const int px = PX ? PX : sc.sPx, pt = PT ? PT : sc.sPt, P = px * px * pt;
+	for (int i = lane; i < min(RT, sc.F) * RY * RX; i += 64) {
+		const int lx = i & (RX - 1), ly = (i >> LX) & (RY - 1), lt = i >> (LX + LY);
+		const int x = x0 + lx, y = y0 + ly, t = t0 + lt, o = lt * FS + ly * RS + lx;
+		const bool in = x < xe && y < ye && t < te;
+		Acc a;
+		a.w = in ? wsum[(size_t)t * sc.WH + (size_t)y * sc.W + x] : 0.f;
 #pragma unroll
-		for (int i = 0; i < 4; i++) {
-			if (rest) {
-				const int lead = __ffsll((unsigned long long)rest) - 1;
-				const int o = __shfl(owner, lead, 64);
-				const uint64_t m = __ballot(owner == o);
-				own_t[i] = o;
-				own_m[i] = m;
-				rest &= ~m;
+		for (int c = 0; c < CC; c++)
+			a.n[c] = in ? num[(size_t)t * sc.WHC + (size_t)c * sc.WH + (size_t)y * sc.W + x] : 0.f;
+		acc[o] = a;
+	}
+	// the lane's samples: place in the region, window value
+	int soff[PS];
+	float wv[PS];
+#pragma unroll
+	for (int u = 0; u < PS; u++) {
+		const int p = min(lane + 64 * u, P - 1);
+		const int dt = p / (px * px), r = p - dt * px * px, dy = r / px, dx = r - dy * px;
+		soff[u] = dt * FS + dy * RS + dx;
+		wv[u] = WIN ? win[p] : 1.f;
+	}
+	const uint32_t row_bytes = (uint32_t)(CC * P) * 4u;
+
+	// records of a chunk of 64 rows, lane = row: row, LDS offset, weight, the
+	// mask of the covered samples
+	struct Meta {
+		uint32_t e, lo[PS], hi[PS];
+		int o;
+		float w;
+	};
+	auto meta = [&](uint32_t kc, uint32_t e, const uint4 &rec) {
+		const int t = (int)(rec.w >> 16), y = (int)(rec.w & 0xffffu);
+		const int x = (int)(rec.x - (uint32_t)t * (uint32_t)sc.WH - (uint32_t)y * (uint32_t)sc.W);
+		// the region and the interior of the row's tile, in patch samples
+		const int ty = (int)rec.y / sc.nW, tx = (int)rec.y - ty * sc.nW;
+		const int ax = max(max(x0, tx * sc.wTmp) - x, 0), ex = min(min(xe, (tx + 1) * sc.wTmp) - x, px);
+		const int ay = max(max(y0, ty * sc.hTmp) - y, 0), ey = min(min(ye, (ty + 1) * sc.hTmp) - y, px);
+		const int at = max(t0 - t, 0), et = min(te - t, pt);
+		const bool live = kc + lane < k1 && ex > ax && ey > ay && et > at;
+		Meta r;
+		r.e = e;
+		r.o = (t - t0) * FS + (y - y0) * RS + (x - x0);
+		r.w = __uint_as_float(rec.z);
+		uint64_t m[PS];
+#pragma unroll
+		for (int u = 0; u < PS; u++) m[u] = 0;
+		if constexpr (PX == 4 && PT == 4) {
+			const uint32_t f = ((((1u << ex) - (1u << ax)) * 0x1111u) & ((1u << (4 * ey)) - (1u << (4 * ay)))) * 0x10001u;
+			m[0] = (((uint64_t)f << 32) | f) & bits64(16 * at, 16 * et);
+		} else if constexpr (PX == 8 && PT == 1) {
+			const uint32_t f = ((1u << ex) - (1u << ax)) * 0x01010101u;
+			m[0] = (((uint64_t)f << 32) | f) & bits64(8 * ay, 8 * ey);
+		} else if (live) {
+			for (int dt = at; dt < et; dt++)
+				for (int dy = ay; dy < ey; dy++) {
+					const int q = (dt * px + dy) * px;
+#pragma unroll
+					for (int u = 0; u < PS; u++) {
+						const int lo = max(q + ax - 64 * u, 0), hi = q + ex - 64 * u;
+						if (lo < 64) m[u] |= bits64(lo, hi);
+					}
+				}
+		}
+#pragma unroll
+		for (int u = 0; u < PS; u++) {
+			r.lo[u] = live ? (uint32_t)m[u] : 0u;
+			r.hi[u] = live ? (uint32_t)(m[u] >> 32) : 0u;
+		}
+		return r;
+	};
+	auto on_lane = [](const Meta &m, int s, int row) {
+		return __builtin_amdgcn_inverse_ballot_w64(((uint64_t)(uint32_t)__builtin_amdgcn_readlane(m.hi[s], row) << 32) |
+		                                           (uint32_t)__builtin_amdgcn_readlane(m.lo[s], row));
+	};
+	// the samples of rows r0 .. r0 + U - 1 of a chunk requested, and added
+	struct Rows { float v[U][PS][CC]; };
+	auto request = [&](const Meta &m, int r0, Rows &q) {
+#pragma unroll
+		for (int u = 0; u < U; u++) {
+			const char *row = reinterpret_cast<const char *>(est) +
+			                  (uint64_t)(uint32_t)__builtin_amdgcn_readlane(m.e, r0 + u) * row_bytes;
+			const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(row), 0, row_bytes, 0x00027000);
+#pragma unroll
+			for (int s = 0; s < PS; s++) {
+				const bool on = on_lane(m, s, r0 + u);
+#pragma unroll
+				for (int c = 0; c < CC; c++)   // -4: past the row's end, nothing fetched
+					q.v[u][s][c] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+					    rs, on ? 4 * (lane + 64 * s + c * P) : -4, 0, 0));
+			}
+		}
+	};
+	auto add = [&](const Meta &m, int r0, const Rows &q) {
+#pragma unroll
+		for (int u = 0; u < U; u++) {
+			const int o = __builtin_amdgcn_readlane(m.o, r0 + u);
+			const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m.w), r0 + u));
+#pragma unroll
+			for (int s = 0; s < PS; s++) {
+				const float wt = WIN ? w * wv[s] : w;   // a window of ones: the same bits
+				if (on_lane(m, s, r0 + u)) {
+					Acc a = acc[o + soff[s]];
+					a.w = a.w + wt;
+#pragma unroll
+					for (int c = 0; c < CC; c++) a.n[c] = a.n[c] + q.v[u][s][c];
+					acc[o + soff[s]] = a;
+				}
+			}
+		}
+	};
+	// entries two chunks ahead, records one (indices clamped to the list)
+	auto entry = [&](uint32_t kc) { return blist[min(kc + (uint32_t)lane, k1 - 1u)]; };
+	uint32_t eN = entry(k0);
+	uint4 rN = erec[eN];
+	Meta mc = meta(k0, eN, rN);
+	eN = entry(k0 + 64);
+	rN = erec[eN];
+	uint32_t eNN = entry(k0 + 128);
+	__syncthreads();   // the sums' first values are in LDS
+	Rows qa, qb;
+	request(mc, 0, qa);
+	for (uint32_t kc = k0; kc < k1; kc += 64) {
+		static_assert((64 / U) % 2 == 0, "packets in pairs");
+#pragma unroll
+		for (int r = 0; r < 64; r += 2 * U) {
+			request(mc, r + U, qb);
+			add(mc, r, qa);
+			if (r + 2 * U < 64) {
+				request(mc, r + 2 * U, qa);
+				add(mc, r + U, qb);
+			} else {
+				const Meta mn = meta(kc + 64, eN, rN);
+				request(mn, 0, qa);
+				eN = eNN;
+				rN = erec[eN];
+				eNN = entry(kc + 192);
+				add(mc, r + U, qb);
+				mc = mn;
 			}
 		}
 	}
-	float aw[TB], an[TB][CC];
-#pragma unroll
-	for (int f = 0; f < TB; f++) {
-		aw[f] = 0.f;
-#pragma unroll
-		for (int c = 0; c < CC; c++) an[f][c] = 0.f;
-		if (valid && t0 + f < sc.F) {
-			aw[f] = wsum[(size_t)(t0 + f) * sc.WH + (size_t)y * sc.W + x];
-#pragma unroll
-			for (int c = 0; c < CC; c++)
-				an[f][c] = num[(size_t)(t0 + f) * sc.WHC + (size_t)c * sc.WH + (size_t)y * sc.W + x];
-		}
-	}
-	for (int i = lane; i < ZQ; i += 64) lds4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-	for (int i = lane; i < P; i += 64) slotm1[i] = win[i];
-	if (lane == 0) *reinterpret_cast<int2 *>(slotm1 + CC * P) = make_int2(-16 * ZQ, 0);
-	const int pix_l = ly * sPx + lx;
-	const float4 *est4 = reinterpret_cast<const float4 *>(est);
-	const int nch = (int)((k1 - k0 + NBR - 1) / NBR);
-
-	// Software pipeline: while chunk c is folded, the slices of chunk c+1,
-	// the row records of chunk c+2 and the list entries of chunk c+3 are in
-	// flight (eA, rA: chunk c+1's entries and records, eB, rB: chunk c+2's,
-	// eC: chunk c+3's entries), so no record load waits for its entry load.
-	// The loads are unconditional (index clamped to the bin's last entry,
-	// and the lanes past the chunk's NBR rows all at its first entry, one
-	// line; meta_commit uses only the lanes of the chunk's rows), so their
-	// results land in the registers that carry them and nothing waits for
-	// them before they are used.
-	auto ent_load = [&](int c) -> uint32_t {
-		const uint32_t kc = k0 + (uint32_t)c * NBR;
-		return blist[min(kc + (uint32_t)(lane < NBR ? lane : 0), k1 - 1u)];
-	};
-	uint32_t eA = ent_load(0);
-	uint4 rA = erec[eA];
-	uint32_t eB = 0, eC = 0;
-	uint4 rB = make_uint4(0, 0, 0, 0);
-	uint32_t &eN = eA;
-	uint4 &recN = rA;
-	// the chunk's row masks into rowm[c & 1] and its records (lane = row)
-	// into rw, for the slot write with the chunk's samples; returns the
-	// lane's coverage mask (lanes = rows) and the rows present at each frame
-	int2 rw = make_int2(0, 0);
-	auto meta_commit = [&](int c, uint32_t (&vm)[TB]) -> uint64_t {
-		const uint32_t kc = k0 + (uint32_t)c * NBR;
-		const bool rv = lane < NBR && kc + lane < k1;
-		uint64_t msp = 0;
-		int qt = 0;
-		if (rv) {
-			const uint32_t q = recN.x;
-			qt = (int)(recN.w >> 16);
-			const int qy = (int)(recN.w & 0xffffu);
-			const int qx = (int)(q - (uint32_t)qt * (uint32_t)sc.WH - (uint32_t)qy * (uint32_t)sc.W);
-			const int dx0 = qx - x0, dy0 = qy - y0;
-			const uint32_t cols = span8(dx0, dx0 + sPx), rows = span8(dy0, dy0 + sPx);
-			uint64_t rsel = 0;
-#pragma unroll
-			for (int r = 0; r < 8; r++) if ((rows >> r) & 1u) rsel |= 1ull << (8 * r);
-			msp = (uint64_t)cols * rsel;
-			uint64_t om = 0;
-#pragma unroll
-			for (int i = 0; i < 4; i++) if (own_t[i] == (int)recN.y) om = own_m[i];
-			msp &= om;
-			// slices dt of the bin's frames t0 .. t0 + TB - 1
-			const int dlo = max(0, t0 - qt), dhi = min(sPt - 1, t0 + TB - 1 - qt);
-			const uint32_t dm = (msp != 0 && dhi >= dlo) ? ((2u << dhi) - (1u << dlo)) : 0u;
-			const int wb = (t0 - qt) * SL - (dy0 * sPx + dx0);
-			rw = make_int2(4 * wb, (int)recN.z);
-			rowm[c & 1][lane] = make_uint2(eN, dm);
-		} else if (lane < NBR) {
-			rowm[c & 1][lane] = make_uint2(0u, 0u);   // past the list's end: nothing staged
-		}
-#pragma unroll
-		for (int f = 0; f < TB; f++) {
-			const int dt = t0 + f - qt;
-			vm[f] = (uint32_t)__ballot(rv && msp != 0 && dt >= 0 && dt < sPt);
-		}
-		return msp;
-	};
-	// staged slices of a chunk: float4 i = lane + 64 m of the chunk's rows
-	// (row i / QR); only the slices at the bin's frames are loaded and
-	// stored, the rest of a row's slot is never read
-	float4 sv[SPL];
-#pragma unroll
-	for (int m = 0; m < SPL; m++) sv[m] = make_float4(0.f, 0.f, 0.f, 0.f);
-	uint32_t sneed = 0;
-#define AGG_BIN_STAGE_ISSUE(c)                                                                      \
-	{                                                                                               \
-		sneed = 0;                                                                                  \
-		const int nbc_ = (int)min<uint32_t>(NBR, k1 - (k0 + (uint32_t)(c) * NBR));                 \
-		_Pragma("unroll") for (int m = 0; m < SPL; m++) {                                         \
-			const int i = lane + 64 * m;                                                            \
-			const int j = i / QR, rq = i - j * QR;                                                  \
-			if (j < nbc_) {                                                                         \
-				const uint2 rm = rowm[(c) & 1][j];                                                  \
-				if ((rm.y >> ((rq % PQ) / SQ)) & 1u) {                                              \
-					sv[m] = est4[(size_t)rm.x * QR + rq];                                           \
-					sneed |= 1u << m;                                                               \
-				}                                                                                   \
-			}                                                                                       \
-		}                                                                                           \
-	}
-#define AGG_BIN_STAGE_WRITE()                                                                       \
-	{                                                                                               \
-		_Pragma("unroll") for (int m = 0; m < SPL; m++)                                           \
-			if ((sneed >> m) & 1u) {                                                                \
-				const int i = lane + 64 * m;                                                        \
-				const int j = i / QR;                                                               \
-				lds4[ZQ + QS + j * QS + (i - j * QR)] = sv[m];                                      \
-			}                                                                                       \
-		if (lane < NBR) *reinterpret_cast<int2 *>(slot0 + 4 * QS * lane + CC * P) = rw;            \
-	}
-	uint32_t vmC[TB], vmN[TB];
-	uint64_t mC = meta_commit(0, vmC);
-	eA = ent_load(1);
-	rA = erec[eA];
-	eB = ent_load(2);
 	__syncthreads();
-	AGG_BIN_STAGE_ISSUE(0);
-	AGG_BIN_STAGE_WRITE();
-	// byte offset of the lane's slice at each frame of the bin
-	int plf4[TB];
+	for (int i = lane; i < min(RT, sc.F) * RY * RX; i += 64) {
+		const int lx = i & (RX - 1), ly = (i >> LX) & (RY - 1), lt = i >> (LX + LY);
+		const int x = x0 + lx, y = y0 + ly, t = t0 + lt, o = lt * FS + ly * RS + lx;
+		if (!(x < xe && y < ye && t < te)) continue;
+		const Acc a = acc[o];
+		wsum[(size_t)t * sc.WH + (size_t)y * sc.W + x] = a.w;
 #pragma unroll
-	for (int f = 0; f < TB; f++) plf4[f] = 4 * (f * SL + pix_l);
-	// the sums' first values are complete here (an empty asm that reads and
-	// writes them), so the fold below waits for no global load of its own:
-	// the slices of the next chunk stay in flight while a chunk is folded
-#pragma unroll
-	for (int f = 0; f < TB; f++) {
-		asm volatile("" : "+v"(aw[f]));
-#pragma unroll
-		for (int cc = 0; cc < CC; cc++) asm volatile("" : "+v"(an[f][cc]));
+		for (int c = 0; c < CC; c++) num[(size_t)t * sc.WHC + (size_t)c * sc.WH + (size_t)y * sc.W + x] = a.n[c];
 	}
-	for (int c = 0; c < nch; c++) {
-		uint64_t mN = 0;
-		if (c + 1 < nch) mN = meta_commit(c + 1, vmN);
-		rB = erec[eB];
-		eC = ent_load(c + 3);
-		__syncthreads();
-		if (c + 1 < nch) AGG_BIN_STAGE_ISSUE(c + 1);
-		// each lane folds the rows that cover its pixel, frame by frame, in
-		// row order, RPR rows per round (their LDS reads overlap)
-		const uint32_t mine_sp = (uint32_t)transpose_bits64(mC);
-#pragma unroll
-		for (int f = 0; f < TB; f++) {
-			uint32_t mine = mine_sp & vmC[f];
-			while (mine) {
-				int so[RPR];   // byte offset of the row's slot from slot 0 (-SB: no row)
-#pragma unroll
-				for (int u = 0; u < RPR; u++) {
-					// the lowest set bit's index, -1 for an empty mask
-					int jj;
-					asm("v_ffbl_b32 %0, %1" : "=v"(jj) : "v"(mine));
-					mine &= mine - 1;
-					so[u] = __mul24(jj, SB);
-				}
-				const char *s0 = reinterpret_cast<const char *>(slot0);
-				const char *wn = reinterpret_cast<const char *>(slotm1) + plf4[f];
-				int2 rr[RPR];
-				float vv[RPR], xx[RPR][CC];
-#pragma unroll
-				for (int u = 0; u < RPR; u++) rr[u] = *reinterpret_cast<const int2 *>(s0 + so[u] + RECB);
-#pragma unroll
-				for (int u = 0; u < RPR; u++) {
-					vv[u] = *reinterpret_cast<const float *>(wn + rr[u].x);
-					const char *sp = s0 + (so[u] + rr[u].x + plf4[f]);
-#pragma unroll
-					for (int cc = 0; cc < CC; cc++) xx[u][cc] = *reinterpret_cast<const float *>(sp + 4 * cc * P);
-				}
-#pragma unroll
-				for (int u = 0; u < RPR; u++) {
-					aw[f] = aw[f] + __int_as_float(rr[u].y) * vv[u];
-#pragma unroll
-					for (int cc = 0; cc < CC; cc++) an[f][cc] = an[f][cc] + xx[u][cc];
-				}
-			}
-		}
-		__syncthreads();
-		if (c + 1 < nch) AGG_BIN_STAGE_WRITE();
-		eA = eB;
-		rA = rB;
-		eB = eC;
-		mC = mN;
-#pragma unroll
-		for (int f = 0; f < TB; f++) vmC[f] = vmN[f];
-	}
-#pragma unroll
-	for (int f = 0; f < TB; f++)
-		if (valid && t0 + f < sc.F) {
-			wsum[(size_t)(t0 + f) * sc.WH + (size_t)y * sc.W + x] = aw[f];
-#pragma unroll
-			for (int c = 0; c < CC; c++)
-				num[(size_t)(t0 + f) * sc.WHC + (size_t)c * sc.WH + (size_t)y * sc.W + x] = an[f][c];
-		}
 }
-#undef AGG_BIN_STAGE_ISSUE
-#undef AGG_BIN_STAGE_WRITE
 
-#define AGGB_ARGS const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, StepConst, \
-	int, int, int, float *, float *
-template __global__ void agg_bin_fold_kernel<1, 32, 16, 4>(AGGB_ARGS);
-template __global__ void agg_bin_fold_kernel<1, 32, 16, 16>(AGGB_ARGS);
-template __global__ void agg_bin_fold_kernel<3, 16, 16, 4>(AGGB_ARGS);
-template __global__ void agg_bin_fold_kernel<3, 16, 16, 16>(AGGB_ARGS);
-template __global__ void agg_bin_fold_kernel<4, 16, 16, 4>(AGGB_ARGS);
-template __global__ void agg_bin_fold_kernel<4, 16, 16, 16>(AGGB_ARGS);
+#define AGGB_ARGS const uint32_t *, const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, \
+	StepConst, int, int, float *, float *
+#define AGGB_INST(CC)                                                                                       \
+	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68>(AGGB_ARGS);          \
+	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68>(AGGB_ARGS); \
+	template __global__ void agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64>(AGGB_ARGS);           \
+	template __global__ void agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);         \
+	template __global__ void agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);         \
+	template __global__ void agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);
+AGGB_INST(1)
+AGGB_INST(3)
+AGGB_INST(4)
 
 __global__ void normalize_kernel(const float *__restrict__ num, const float *__restrict__ wsum,
                                  const float *__restrict__ noisy, StepConst sc,

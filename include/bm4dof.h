@@ -120,12 +120,13 @@ const char *bm4dof_global_error(void);
  *   "agg_cap"      rows sorted per step of the chunked aggregation, for one
  *                  channel: 512, 768, 1024 (default) or 1536.
  *   "agg_binned"   1 (default): where the chunked aggregation applies and
- *                  patches have at most 64 samples (at most 8x8 pixels and
- *                  4 frames, 1, 3 or 4 channels), each bin of 8 x 8 pixels
- *                  x 4 frames gets its rows as one list in row order, built
- *                  beside the filter, and one wave folds the list into the
- *                  bin's four frames; 0: the chunked aggregation sorts the
- *                  rows of every 8 x 8 x 1 block itself.
+ *                  patches are 4x4x4 or of one frame (1, 3 or 4 channels),
+ *                  each region (8 x 8 pixels x 4 to 32 frames, 16 x 16 x 1
+ *                  for one-frame patches other than 8x8) gets its rows as
+ *                  one list in row order, built beside the filter, and one
+ *                  wave folds the list into the region's sums; 0: the
+ *                  chunked aggregation sorts the rows of every 8 x 8 x 1
+ *                  block itself.
  *   "coef_beside_bm" 1 (default): a gray step's coefficient tables are
  *                  computed on the second stream beside its block matching;
  *                  0: after it, on the main stream.
