@@ -49,7 +49,7 @@ __global__ void filter2_kernel(const float *, const float *, const uint32_t *, c
 	const float *, const float *
 template <int PX> __global__ void filter1_fast_kernel(FILTER1_ARGS);
 template <int PX> __global__ void coef_kernel(const float *, int, int, int, const float *, float *);
-template <int PX> __global__ void filter2_fast_kernel(FILTER2_ARGS);
+template <int PX, int NMAX, bool TAB> __global__ void filter2_fast_kernel(FILTER2_ARGS);
 #define LEARNED_ARGS const float *, const uint32_t *, const uint32_t *, const uint32_t *, const uint32_t *, \
 	StepConst, int, int, const uint16_t *, const float *, MlpInfer, float, float, float *, \
 	float *, uint32_t *, uint8_t *, float *, uint8_t *, uint32_t *, int, int
@@ -1125,6 +1125,20 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 	}
 }
 
+using Filter2 = void (*)(FILTER2_ARGS);
+template <int PX, bool TAB> Filter2 filter2_rows(int np)
+{
+	return np < 16 ? filter2_fast_kernel<PX, 8, TAB> : np < 32 ? filter2_fast_kernel<PX, 16, TAB>
+	                                                            : filter2_fast_kernel<PX, 32, TAB>;
+}
+// The step-2 filter for a patch shape and the rows its groups can have (the
+// largest power of two up to npmax).
+Filter2 filter2_of(const StepConst &sc, bool tab)
+{
+	if (sc.sPx == 4) return tab ? filter2_rows<4, true>(sc.npmax) : filter2_rows<4, false>(sc.npmax);
+	return tab ? filter2_rows<8, true>(sc.npmax) : filter2_rows<8, false>(sc.npmax);
+}
+
 // Launches one step on ctx->stream.  With `tm` it records stage events; a
 // captured enqueue passes none.  Needs reserve_step(plan) first.
 // parts: 1 set-up and block matching, 2 the rest (filter, aggregation,
@@ -1253,12 +1267,17 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 				                   dim3(64), 0, ctx->stream, d_nplanes, d_idx, d_nsim, d_base, dv.gtile, sc, g0,
 				                   Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile, d_early, d_gw, d_cnt, C, c,
 				                   (int64_t)WHF, d_gacc, d_coef_n);
-		else if (pl.fast)
+		else if (pl.fast) {
+			const auto kern = filter2_of(sc, d_coef_n != nullptr);
+			// about 100 blocks per CU, looping: fewer (3 per CU, all that fit)
+			// leave the row sort beside it no room, which then ends 1.4 ms
+			// after it; 8 and 32 per CU end unevenly (17.1, 15.6 against 14.9 ms)
+			const unsigned blocks = (unsigned)std::min(nblk(Gc, d_coef_n ? 4 : 2), 25600);
 			for (int c = 0; c < C; c++)
-				hipLaunchKernelGGL(sc.sPx == 4 ? filter2_fast_kernel<4> : filter2_fast_kernel<8>, dim3(Gc),
-				                   dim3(64), 0, ctx->stream, d_nplanes, d_bplanes, d_idx, d_nsim, d_base,
-				                   dv.gtile, sc, g0, Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile, d_early,
-				                   d_gw, d_cnt, C, c, (int64_t)WHF, d_gacc, d_coef_n, d_coef_b);
+				hipLaunchKernelGGL(kern, dim3(blocks), dim3(d_coef_n ? 256 : 128), 0, ctx->stream, d_nplanes, d_bplanes, d_idx, d_nsim,
+				                   d_base, dv.gtile, sc, g0, Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile,
+				                   d_early, d_gw, d_cnt, C, c, (int64_t)WHF, d_gacc, d_coef_n, d_coef_b);
+		}
 		else if (step1)
 			hipLaunchKernelGGL(filter1_kernel, dim3(Gc), dim3(256), pl.filt_lds, ctx->stream, noisy_w,
 			                   d_idx, d_nsim, d_base, dv.gtile, sc, g0, Gc, dv.basis, dv.binv, dv.win, d_est,

@@ -18,6 +18,8 @@
 //     (nldct.cpp:2284-2300, 2376-2393), separately rounded.
 // The GPU output is therefore bitwise equal to the sequential oracle.
 #include "common.hpp"
+
+#include <type_traits>
 #include "mlp_dev.hpp"
 
 namespace bm4dof {
@@ -1539,16 +1541,16 @@ void filter2_kernel(const float *__restrict__ noisy, const float *__restrict__ b
 // Rows n >= N must be +0 on entry and stay so: the butterflies that start
 // at such a row pair two of them (n + h > n >= N) and give +0 again, so
 // they run unguarded, without a select per row.
-__device__ __forceinline__ void haar_lane(float (&z)[FAST_NMAX], int N, bool forward)
+template <int NMAX> __device__ __forceinline__ void haar_lane(float (&z)[NMAX], int N, bool forward)
 {
 	const float isqrt2 = 0.70710678118654752440f;
 #pragma unroll
-	for (int l = 0; l < 5; l++) {
-		const int s = forward ? (2 << l) : (32 >> l);   // 2..32 / 32..2
+	for (int u = 2; u <= NMAX; u *= 2) {
+		const int s = forward ? u : 2 * NMAX / u;   // 2..NMAX / NMAX..2
 		const int h = s >> 1;
 		if (s <= N) {
 #pragma unroll
-			for (int n = 0; n < FAST_NMAX; n += s) {
+			for (int n = 0; n < NMAX; n += s) {
 				const float z0 = z[n] * isqrt2;
 				const float z1 = z[n + h] * isqrt2;
 				z[n] = z0 + z1;
@@ -1556,6 +1558,147 @@ __device__ __forceinline__ void haar_lane(float (&z)[FAST_NMAX], int N, bool for
 			}
 		}
 	}
+}
+
+// ---------------------------------------------------------------------------
+// Dense patch transforms on the fp32 matrix instructions.  v_mfma_f32_32x32x2
+// and _16x16x4 add their products to the accumulator one term after another,
+// each as one fused multiply-add: bit for bit the sequential sums of
+// fast_forward, at twice the vector unit's rate and beside its work.
+// Operands of the instruction that takes terms 2 s, 2 s + 1 (ROWS = 32; lane
+// l: h = l / 32, j = l % 32) or 4 s .. 4 s + 3 (ROWS = 16; h = l / 16, j =
+// l % 16): A[row j][term TS s + h], B[term TS s + h][column j].
+// ---------------------------------------------------------------------------
+typedef float mm_f32x16 __attribute__((ext_vector_type(16)));
+typedef float mm_f32x4 __attribute__((ext_vector_type(4)));
+
+template <int ROWS> struct MmTile;
+template <> struct MmTile<32> {
+	static constexpr int TS = 2;              // terms an instruction takes
+	static constexpr int NR = 16;             // results a lane holds
+	using Acc = mm_f32x16;
+	static __device__ __forceinline__ Acc mac(float a, float b, Acc c)
+	{
+		return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+	}
+	static __device__ __forceinline__ int row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
+};
+template <> struct MmTile<16> {
+	static constexpr int TS = 4;
+	static constexpr int NR = 4;
+	using Acc = mm_f32x4;
+	static __device__ __forceinline__ Acc mac(float a, float b, Acc c)
+	{
+		return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+	}
+	static __device__ __forceinline__ int row(int r, int h) { return 4 * h + r; }
+};
+constexpr int MM_ZS = 68;   // LDS row stride of an A operand
+
+// The P x P matrix m[term * ts + column * cs] as B operands in LDS: float4 q
+// of lane l and column tile t holds the operands of instructions 4 q .. 4 q + 3.
+template <int ROWS>
+__device__ __forceinline__ void mm_load_b(const float *__restrict__ m, int ts, int cs, int P, float4 *__restrict__ bf)
+{
+	constexpr int TS = MmTile<ROWS>::TS, Q = FAST_P / (4 * TS);
+	for (int i = threadIdx.x; i < FAST_P * FAST_P / 4; i += blockDim.x) {
+		const int l = i & 63, q = (i >> 6) % Q, t = (i >> 6) / Q, h = l / ROWS, col = ROWS * t + l % ROWS;
+		float v[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			const int k = TS * (4 * q + u) + h;
+			v[u] = k < P && col < P ? m[k * ts + col * cs] : 0.f;
+		}
+		bf[i] = make_float4(v[0], v[1], v[2], v[3]);
+	}
+}
+
+// Place of term k in an A operand's LDS row: the terms a lane takes lie
+// together.
+template <int ROWS> __device__ __forceinline__ int mm_pos(int k)
+{
+	constexpr int TS = MmTile<ROWS>::TS;
+	return (k % TS) * (FAST_P / TS) + k / TS;
+}
+
+// The lane's A operands, four instructions to a float4.
+template <int ROWS>
+__device__ __forceinline__ void mm_load_a(const float *__restrict__ zs, float4 (&a)[FAST_P / 4 / MmTile<ROWS>::TS])
+{
+	constexpr int TS = MmTile<ROWS>::TS;
+	const int l = threadIdx.x & 63;
+	const float *p = zs + (l % ROWS) * MM_ZS + l / ROWS * (FAST_P / TS);
+#pragma unroll
+	for (int q = 0; q < FAST_P / 4 / TS; q++) a[q] = *reinterpret_cast<const float4 *>(p + 4 * q);
+}
+
+// Column tile t of the product A B, terms in order.
+template <int ROWS>
+__device__ __forceinline__ typename MmTile<ROWS>::Acc mm_product(const float4 (&a)[FAST_P / 4 / MmTile<ROWS>::TS],
+                                                                 const float4 *__restrict__ bf, int t)
+{
+	using T = MmTile<ROWS>;
+	constexpr int Q = FAST_P / 4 / T::TS;
+	const int l = threadIdx.x & 63;
+	typename T::Acc c = {};
+#pragma unroll
+	for (int q = 0; q < Q; q++) {
+		const float4 b = bf[(t * Q + q) * 64 + l];
+		c = T::mac(a[q].x, b.x, c);
+		c = T::mac(a[q].y, b.y, c);
+		c = T::mac(a[q].z, b.z, c);
+		c = T::mac(a[q].w, b.w, c);
+	}
+	return c;
+}
+
+// v0 + (the terms of lane 0 in order) + (those of lane 1) + ...: the
+// sequential float sum of 64 M terms, bit for bit, in every lane.
+// Every lane folds its M terms from a predicted start at once; the start of
+// lane k is right when the starts before it are and lane k - 1 ends on it.
+// Lanes from the first wrong start on take that lane's right value plus the
+// sums of the changes before them, and fold again: the first wrong start is
+// then right, so it ends, and as a fold's change depends on its start only
+// through the rounding of ties and at powers of two, three to five rounds
+// (55 instructions each at M = 32) do for the 2112 of the chain.
+template <int M> __device__ __forceinline__ float ordered_wave_sum(const float (&y)[M], float v0)
+{
+	const int lane = threadIdx.x & 63;
+	auto shr1 = [](float v, float first) {   // lane k: v of lane k - 1
+		return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138, 0xf, 0xf, false));
+	};
+	auto dpp = [](float v, auto ctrl, auto rows) {
+		return __int_as_float(
+		    __builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, false));
+	};
+	auto before = [&](float v) {   // sum of the lanes before (any order)
+		using std::integral_constant;
+		v = v + dpp(v, integral_constant<int, 0x111>(), integral_constant<int, 0xf>());
+		v = v + dpp(v, integral_constant<int, 0x112>(), integral_constant<int, 0xf>());
+		v = v + dpp(v, integral_constant<int, 0x114>(), integral_constant<int, 0xf>());
+		v = v + dpp(v, integral_constant<int, 0x118>(), integral_constant<int, 0xf>());
+		v = v + dpp(v, integral_constant<int, 0x142>(), integral_constant<int, 0xa>());
+		v = v + dpp(v, integral_constant<int, 0x143>(), integral_constant<int, 0xc>());
+		return shr1(v, 0.f);
+	};
+	float t = 0.f;
+#pragma unroll
+	for (int n = 0; n < M; n++) t = t + y[n];
+	float s = v0 + before(t), e = s;
+	if (lane == 0) s = v0;
+	for (int it = 0; it < 64; it++) {   // bounded for NaN, which equals nothing
+		e = s;
+#pragma unroll
+		for (int n = 0; n < M; n++) e = e + y[n];
+		const float prev = shr1(e, v0);
+		const uint64_t wrong = __ballot(__float_as_uint(prev) != __float_as_uint(s));
+		if (!wrong) break;
+		const int f = __ffsll((unsigned long long)wrong) - 1;
+		const float base = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(prev), f));
+		const float x = before(lane >= f ? e - s : 0.f);
+		if (lane >= f) s = lane == f ? base : base + x;
+	}
+	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), 63));
 }
 
 __device__ __forceinline__ int wave_sum_int(int v)
@@ -1797,22 +1940,24 @@ template __global__ void coef_kernel<8>(const float *, int, int, int, const floa
 // (anchor 0) and are set to 0.  (The step-2 filter keeps the scalar loads:
 // there the 32 indices held in scalar registers spill and the filter is
 // slower.)
-template <bool VIDX = false>
+template <int P, bool VIDX = false, int NMAX>
 __device__ __forceinline__ void fast_rows(const float *__restrict__ coef, const uint32_t *__restrict__ gidx, int N,
-                                          float (&z)[FAST_NMAX])
+                                          float (&z)[NMAX])
 {
-	static_assert(FAST_NMAX <= 64, "one index per lane");
+	static_assert(NMAX <= 64, "one index per lane");
+	const int lane = threadIdx.x & 63;
+	const bool in = P == FAST_P || lane < P;
 	if (VIDX) {
-		const uint32_t my_idx = (int)threadIdx.x < N ? gidx[threadIdx.x] : 0u;
+		const uint32_t my_idx = lane < N ? gidx[lane] : 0u;
 #pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) {
+		for (int n = 0; n < NMAX; n++) {
 			const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)my_idx, n);
-			const float v = coef[(size_t)r * FAST_P + threadIdx.x];
+			const float v = in ? coef[(size_t)r * FAST_P + lane] : 0.f;
 			z[n] = n < N ? v : 0.f;
 		}
 	} else {
 #pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) z[n] = n < N ? coef[(size_t)gidx[n] * FAST_P + threadIdx.x] : 0.f;
+		for (int n = 0; n < NMAX; n++) z[n] = n < N && in ? coef[(size_t)gidx[n] * FAST_P + lane] : 0.f;
 	}
 }
 
@@ -1821,12 +1966,12 @@ __device__ __forceinline__ void fast_rows(const float *__restrict__ coef, const 
 // a +-0 term cannot change a sum that starts at +0 (it never becomes -0).
 // So rows that differ rule out the equality early-out without reading the
 // patches.
-__device__ __forceinline__ bool fast_rows_equal(const float (&z)[FAST_NMAX], int N)
+template <int NMAX> __device__ __forceinline__ bool fast_rows_equal(const float (&z)[NMAX], int N)
 {
 	const uint32_t z0 = __float_as_uint(z[0]);
 	bool d = false;
 #pragma unroll
-	for (int n = 1; n < FAST_NMAX; n++) d |= n < N && __float_as_uint(z[n]) != z0;
+	for (int n = 1; n < NMAX; n++) d |= n < N && __float_as_uint(z[n]) != z0;
 	return !__any(d);
 }
 
@@ -1841,7 +1986,8 @@ __device__ __forceinline__ bool fast_early_out(const float *__restrict__ img, co
                                                float *__restrict__ gweight, uint32_t *__restrict__ n_early)
 {
 	if (N <= 1) return false;
-	const int l = threadIdx.x;
+	constexpr int P = PX * PX * (PX == 4 ? 4 : 1);
+	const int lane = threadIdx.x & 63, l = min(lane, P - 1);
 	const int off = (l / (PX * PX)) * WH + ((l / PX) % PX) * W + (l % PX);
 	int differs = 0;
 	for (int c = 0; c < C; c++) {
@@ -1852,8 +1998,8 @@ __device__ __forceinline__ bool fast_early_out(const float *__restrict__ img, co
 	if (__any(differs)) return false;
 	for (int c = 0; c < C; c++)
 		for (int n = 0; n < N; n++)
-			est[((size_t)(row0 + n) * C + c) * FAST_P + l] = img[c * cstride + gidx[n] + off];
-	if (l == 0) { early[g] = 1; gweight[g] = 0.f; atomicAdd(n_early, 1u); }
+			if (lane < P) est[((size_t)(row0 + n) * C + c) * P + l] = img[c * cstride + gidx[n] + off];
+	if (lane == 0) { early[g] = 1; gweight[g] = 0.f; atomicAdd(n_early, 1u); }
 	return true;
 }
 
@@ -1863,11 +2009,12 @@ __device__ __forceinline__ bool fast_early_out(const float *__restrict__ img, co
 // sum from launch to launch; launches before the last store the inverse
 // transform unweighted and the last one scales them by its weight: the same
 // products (w * window) * value as one pass over all channels.
+template <int P>
 __device__ __forceinline__ void fast_scale_channels(int N, int C, float ww, uint32_t row0, float *__restrict__ est)
 {
 	for (int n = 0; n < N; n++)
 		for (int c = 0; c < C - 1; c++) {
-			float *e = est + ((size_t)(row0 + n) * C + c) * FAST_P + threadIdx.x;
+			float *e = est + ((size_t)(row0 + n) * C + c) * P + (threadIdx.x & 63);
 			*e = ww * *e;
 		}
 }
@@ -1893,7 +2040,7 @@ void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restri
 	const uint32_t row0 = base[gl];
 	const uint32_t *gidx = idx + (size_t)g * sc.npmax;
 	float z[FAST_NMAX];
-	if (coef) fast_rows<true>(coef + c * cstride * FAST_P, gidx, N, z);
+	if (coef) fast_rows<FAST_P, true>(coef + c * cstride * FAST_P, gidx, N, z);
 	if (c == 0) {
 		if (lane < N) etile[row0 + lane] = gtile[g];
 		if ((!coef || fast_rows_equal(z, N)) &&
@@ -1941,11 +2088,90 @@ void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restri
 	// launches before the last store unweighted rows
 	const float ww = last ? w * win[lane] : 1.f;
 	fast_inverse_sparse(z, zs, binv, N, ww, row0, est, kmask, C * FAST_P, c * FAST_P);
-	if (last && C > 1) fast_scale_channels(N, C, w * win[lane], row0, est);
+	if (last && C > 1) fast_scale_channels<FAST_P>(N, C, w * win[lane], row0, est);
 }
 
-template <int PX>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+// Orders a wave's LDS writes before its lanes' later reads (LDS accesses of a
+// wave execute in order: this only holds the compiler).
+__device__ __forceinline__ void wave_sync()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
+// Forward transform of the N patches at anchors gidx[0..N) of `img` (one
+// channel, anchor address = position): zs[n * MM_ZS + k].  One wave.
+template <int PX, int ROWS>
+__device__ __forceinline__ void mm_forward(const float *__restrict__ img, const uint32_t *__restrict__ gidx, int N,
+                                           int W, int WH, const float4 *__restrict__ bf, float *__restrict__ zs)
+{
+	using T = MmTile<ROWS>;
+	constexpr int PT = PX == 4 ? 4 : 1, P = PX * PX * PT, Q = FAST_P / 4 / T::TS;
+	const int l = threadIdx.x & 63, h = l / ROWS, j = l % ROWS;
+	const float *src = img + gidx[min(j, N - 1)];
+	float4 a[Q];
+#pragma unroll
+	for (int q = 0; q < Q; q++) {
+		float v[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			const int p = T::TS * (4 * q + u) + h;
+			v[u] = j < N && p < P ? src[p / (PX * PX) * WH + p / PX % PX * W + p % PX] : 0.f;
+		}
+		a[q] = make_float4(v[0], v[1], v[2], v[3]);
+	}
+#pragma unroll
+	for (int t = 0; t < FAST_P / ROWS; t++) {
+		const auto c = mm_product<ROWS>(a, bf, t);
+#pragma unroll
+		for (int r = 0; r < T::NR; r++) zs[T::row(r, h) * MM_ZS + ROWS * t + j] = c[r];
+	}
+}
+
+// Inverse transform of the coefficients z[n] (lane = coefficient) and the
+// weighted est rows: est[(row0 + n) rs + ro + p] = (w win[p]) * sample p of
+// patch n.  One wave; zs: ROWS rows of MM_ZS floats.
+template <int P, int NMAX, int ROWS>
+__device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__restrict__ zs,
+                                           const float4 *__restrict__ bf, int N, float w,
+                                           const float *__restrict__ win, uint32_t row0, float *__restrict__ est,
+                                           int rs, int ro)
+{
+	using T = MmTile<ROWS>;
+	const int l = threadIdx.x & 63, h = l / ROWS, j = l % ROWS;
+	const int at = mm_pos<ROWS>(l);
+#pragma unroll
+	for (int n = 0; n < NMAX; n++) zs[n * MM_ZS + at] = z[n];
+	wave_sync();
+	float4 a[FAST_P / 4 / T::TS];
+	mm_load_a<ROWS>(zs, a);
+	float *e0 = est + (size_t)row0 * rs + ro;
+#pragma unroll
+	for (int t = 0; t < FAST_P / ROWS; t++) {
+		const auto c = mm_product<ROWS>(a, bf, t);
+		const int col = ROWS * t + j;
+		if (P < FAST_P && col >= P) continue;
+		const float ww = win ? w * win[col] : 1.f;
+#pragma unroll
+		for (int r = 0; r < T::NR; r++) {
+			const int n = T::row(r, h);
+			if (n < NMAX && n < N) e0[(size_t)n * rs + col] = ww * c[r];
+		}
+	}
+	wave_sync();
+}
+
+// Step-2 filter, one wave per group (grid-stride), lane = coefficient of
+// every row.  NMAX: rows held (8, 16, 32).
+// Bound: HBM, 34 GB of table rows and 19 GB of est per launch at 960x540x20
+// (13.3 ms alone: 4.0 TB/s), beside 1700 vector instructions and 4096 cycles
+// of matrix instructions a group.  The inverse on the matrix instructions and
+// the sum of w^2 folded by all lanes at once took it from 19.1 ms alone
+// (with the sort beside it 21.7 -> 14.9 ms).  Blocks of four waves share the
+// inverse basis in LDS.  Groups dealt to the XCDs in contiguous eighths
+// fetched 4 % less and ran the same.
+template <int PX, int NMAX, bool TAB>
+__global__ __launch_bounds__(TAB ? 256 : 128) __attribute__((amdgpu_waves_per_eu(TAB ? 3 : 2)))
 void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restrict__ basic,
                          const uint32_t *__restrict__ idx, const uint32_t *__restrict__ nsim,
                          const uint32_t *__restrict__ base, const uint32_t *__restrict__ gtile,
@@ -1958,82 +2184,72 @@ void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restric
                          float *__restrict__ gacc, const float *__restrict__ coef_n,
                          const float *__restrict__ coef_b)
 {
-	__shared__ __align__(16) float zs[FAST_NMAX * FAST_P];
-	const int gl = blockIdx.x;
-	if (gl >= Gc) return;
-	const int g = g0 + gl;
-	const int lane = threadIdx.x;
-	const int N = (int)nsim[g];
-	const uint32_t row0 = base[gl];
-	const uint32_t *gidx = idx + (size_t)g * sc.npmax;
-	float z[FAST_NMAX], y[FAST_NMAX];
-	if (coef_n) fast_rows(coef_n + c * cstride * FAST_P, gidx, N, z);
-	if (c == 0) {
-		if (lane < N) etile[row0 + lane] = gtile[g];
-		if ((!coef_n || fast_rows_equal(z, N)) &&
-		    fast_early_out<PX>(noisy, gidx, N, sc.W, sc.WH, C, cstride, g, row0, est, early, gweight, n_early))
-			return;
-	} else if (early[g])
-		return;
-
-	if (coef_n)
-		fast_rows(coef_b + c * cstride * FAST_P, gidx, N, y);
-	else {
-		{
-			float brow[FAST_P];
-#pragma unroll
-			for (int p = 0; p < FAST_P; p++) brow[p] = basis[lane * FAST_P + p];
-			fast_forward<PX>(basic + c * cstride, gidx, N, sc.W, sc.WH, brow, zs);
-			__syncthreads();
-#pragma unroll
-			for (int n = 0; n < FAST_NMAX; n++) y[n] = n < N ? zs[n * FAST_P + lane] : 0.f;
-			__syncthreads();
-			fast_forward<PX>(noisy + c * cstride, gidx, N, sc.W, sc.WH, brow, zs);
-		}
-		__syncthreads();
-#pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) z[n] = n < N ? zs[n * FAST_P + lane] : 0.f;
-	}
-	haar_lane(z, N, true);
-	haar_lane(y, N, true);
-	// Wiener shrinkage; y[n] becomes the energy term w^2
-#pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) {
-		if (n < N) {
-			const float w = y[n] * y[n] / (y[n] * y[n] + sc.beta_sigma2);
-			z[n] = z[n] * w;
-			y[n] = w * w;
-		}
-	}
-	// sum of w^2 in the reference's order, channel, coefficient, then patch:
-	// lane k folds its N terms into the running sum handed on by lane k-1.
-	// Rows n >= N hold +0 and the sum is >= +0 (or NaN), so adding them
-	// leaves it unchanged bit for bit: no select per term.
-	float v = c ? gacc[g] : 0.f;
-	for (int k = 0; k < FAST_P; k++) {
-		float t = v;
-#pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) t = t + y[n];
-		v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), k));
-	}
-	haar_lane(z, N, false);
+	constexpr int P = PX * PX * (PX == 4 ? 4 : 1), ROWS = NMAX > 16 ? 32 : 16, NW = TAB ? 4 : 2;
+	__shared__ __align__(16) float4 bf[FAST_P * FAST_P / 4];                // inverse basis
+	__shared__ __align__(16) float4 bfwd[TAB ? 1 : FAST_P * FAST_P / 4];    // basis
+	__shared__ __align__(16) float zsm[NW * ROWS * MM_ZS];
+	mm_load_b<ROWS>(binv, P, 1, P, bf);
+	if (!TAB) mm_load_b<ROWS>(basis, 1, P, P, bfwd);
 	__syncthreads();
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	float *zs = zsm + wave * ROWS * MM_ZS;
+	for (int gl = blockIdx.x * NW + wave; gl < Gc; gl += gridDim.x * NW) {
+		const int g = g0 + gl;
+		const int N = (int)nsim[g];
+		const uint32_t row0 = base[gl];
+		const uint32_t *gidx = idx + (size_t)g * sc.npmax;
+		float z[NMAX], y[NMAX];
+		if (TAB) fast_rows<P>(coef_n + c * cstride * FAST_P, gidx, N, z);
+		if (c == 0) {
+			if (lane < N) etile[row0 + lane] = gtile[g];
+			if ((!TAB || fast_rows_equal(z, N)) &&
+			    fast_early_out<PX>(noisy, gidx, N, sc.W, sc.WH, C, cstride, g, row0, est, early, gweight, n_early))
+				continue;
+		} else if (early[g])
+			continue;
+		if (TAB)
+			fast_rows<P>(coef_b + c * cstride * FAST_P, gidx, N, y);
+		else if (N > 0) {
+			mm_forward<PX, ROWS>(basic + c * cstride, gidx, N, sc.W, sc.WH, bfwd, zs);
+			wave_sync();
 #pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) if (n < N) zs[n * FAST_P + lane] = z[n];
-	if (c < C - 1) {
-		if (lane == 0) { gacc[g] = v; early[g] = 0; }
-		__syncthreads();
-		fast_inverse(zs, binv, N, 1.f, row0, est, C * FAST_P, c * FAST_P);
-		return;
+			for (int n = 0; n < NMAX; n++) y[n] = zs[n * MM_ZS + lane];
+			wave_sync();
+			mm_forward<PX, ROWS>(noisy + c * cstride, gidx, N, sc.W, sc.WH, bfwd, zs);
+			wave_sync();
+#pragma unroll
+			for (int n = 0; n < NMAX; n++) z[n] = zs[n * MM_ZS + lane];
+			wave_sync();
+		}
+		haar_lane(z, N, true);
+		haar_lane(y, N, true);
+		// Wiener shrinkage; y[n] becomes the energy term w^2
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) {
+			if (n < N) {
+				const float w = y[n] * y[n] / (y[n] * y[n] + sc.beta_sigma2);
+				z[n] = z[n] * w;
+				y[n] = P == FAST_P || lane < P ? w * w : 0.f;
+			}
+		}
+		// sum of w^2 in the reference's order, channel, coefficient, then
+		// patch.  Rows n >= N hold +0 and the sum is >= +0 (or NaN), so adding
+		// them leaves it unchanged bit for bit.
+		const float v = ordered_wave_sum(y, c ? gacc[g] : 0.f);
+		haar_lane(z, N, false);
+		const bool last = c == C - 1;
+		const float w = (float)(1. / (double)sc.sigma2 / (double)v);
+		if (lane == 0) {
+			if (last) gweight[g] = w;
+			else gacc[g] = v;
+			early[g] = 0;
+		}
+		if (last && lane < N) entry_w[row0 + lane] = w;
+		// launches before the last store unweighted rows
+		mm_inverse<P, NMAX, ROWS>(z, zs, bf, N, w, last ? win : nullptr, row0, est, C * P, c * P);
+		if (last && C > 1 && lane < P) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
 	}
-	const float w = (float)(1. / (double)sc.sigma2 / (double)v);
-	if (lane == 0) { gweight[g] = w; early[g] = 0; }
-	if (lane < N) entry_w[row0 + lane] = w;
-	__syncthreads();
-	fast_inverse(zs, binv, N, w * win[lane], row0, est, C * FAST_P, c * FAST_P);
-	if (C > 1) fast_scale_channels(N, C, w * win[lane], row0, est);
 }
-
 
 // ---------------------------------------------------------------------------
 // Learned single pass (no counterpart in the reference).  Groups and
@@ -2408,8 +2624,15 @@ template __global__ void learned_pairs_kernel<8>(PAIRS_ARGS);
 	const float *, const float *
 template __global__ void filter1_fast_kernel<4>(FILTER1_ARGS);
 template __global__ void filter1_fast_kernel<8>(FILTER1_ARGS);
-template __global__ void filter2_fast_kernel<4>(FILTER2_ARGS);
-template __global__ void filter2_fast_kernel<8>(FILTER2_ARGS);
+#define FILTER2_INST(PX, N)                                                                                \
+	template __global__ void filter2_fast_kernel<PX, N, true>(FILTER2_ARGS);                                \
+	template __global__ void filter2_fast_kernel<PX, N, false>(FILTER2_ARGS);
+FILTER2_INST(4, 8)
+FILTER2_INST(4, 16)
+FILTER2_INST(4, 32)
+FILTER2_INST(8, 8)
+FILTER2_INST(8, 16)
+FILTER2_INST(8, 32)
 
 // ---------------------------------------------------------------------------
 // Aggregation in the reference's order.
