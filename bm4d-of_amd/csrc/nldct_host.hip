@@ -27,11 +27,24 @@ __global__ void bm_window_kernel(const float *, const float *, const uint32_t *,
                                  const TileBox *, StepConst, int, int4 *, int2 *);
 #define BMF_ARGS const float *, const int4 *, const int2 *, const uint32_t *, const uint32_t *, \
 	const TileBox *, StepConst, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int
-template <int PX, int PT, bool MC> __global__ void bm_reg_kernel(const float *, const int4 *, const int2 *,
+template <int PX, int PT, bool MC, bool LIST> __global__ void bm_reg_kernel(const float *, const int4 *, const int2 *,
                                                         const uint32_t *, const uint32_t *, const TileBox *,
                                                         StepConst, int, int, uint32_t *, uint32_t *, int,
-                                                        uint32_t *, uint32_t *, int);
+                                                        uint32_t *, uint32_t *, int, const uint32_t *);
 template <int PX, int PT, int NF> __global__ void bm_fast_kernel(BMF_ARGS);
+__global__ void bmq_range_kernel(const float *, int, int, int, float2 *);
+__global__ void bmq_scale_kernel(const float2 *, int, float, float2 *);
+template <int PT>
+__global__ void bmq_pack_kernel(const float *, int, int, int, int64_t, int64_t, const float2 *, int16_t *);
+template <int PX, int PT>
+__global__ void bmq_norm_kernel(const int16_t *, int, int, int, int64_t, int, uint32_t *);
+#define BMB_ARGS const float *, const int16_t *, const uint32_t *, const float2 *, const int4 *, const int2 *, \
+	const uint32_t *, const uint32_t *, const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int,    \
+	uint32_t *, uint32_t *, uint32_t *, uint32_t *
+template <int PX, int PT, bool MC, bool CH> __global__ void bm_bound_kernel(BMB_ARGS);
+__global__ void bm_list_kernel(const float *, const float *, const float *, const uint32_t *, const uint32_t *,
+                               const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, const uint32_t *,
+                               const uint32_t *, uint32_t *, uint32_t *);
 __global__ void filter1_kernel(const float *, const uint32_t *, const uint32_t *, const uint32_t *,
                                const uint32_t *, StepConst, int, int, const float *, const float *,
                                const float *, float *, float *, uint32_t *, uint8_t *, float *,
@@ -531,6 +544,103 @@ static void bm_ties(bm4dof_ctx *ctx, const StepConst &sc, int step, const float 
 	HIPCHK(hipGetLastError());
 }
 
+// Matching by bounded distances: whether a step takes it, and its launches.
+// It has five launches more (some 15 us) and about a thousand instructions a
+// group that do not grow with the window, so it takes over where the window
+// repays them.  Measured against bm_reg_kernel (milliseconds, bounded first):
+//   4x4x4, 960x540x20 (2.4e9 candidates): 10.3 / 20.5; 1.4e7: .29 / .32;
+//     2e6: .073 / .061
+//   8x8x1, 39x39 window, 2.8e7: .32 / .44; 9x9x9 (729 a group), 1.5e8:
+//     2.28 / 2.34; 7x7x9 (441), 4e7: .72 / .65
+// and against bm_kernel, the only other one for their sizes: 7x7x1, 3e7:
+// .35 / 1.39; 11x11x1, 39x39, 1.2e7: .48 / .82.
+constexpr int BMQ_RANGE_BLOCKS = 512;
+static bool bm_bound_ok(const StepConst &sc, int step, int G)
+{
+	const int nch = step == 1 ? 1 : sc.C;
+	const int64_t cand = (int64_t)sc.sWx * sc.sWx * std::max(1, std::min(sc.wtf + sc.wtb + 1, sc.F - sc.sPt + 1));
+	const int64_t all = cand * G;
+	// what the kernels hold: scan indices in 16 bits, places' byte offsets in
+	// 32, a lane per frame; past 512 samples the float sums' own rounding
+	// would leave the bound's slack
+	if (sc.npmax <= 1 || sc.P * nch > 512 || sc.wtf + sc.wtb + 1 > 64 ||
+	    (int64_t)sc.sWx * sc.sWx * (sc.wtf + sc.wtb + 1) >= 65536 || (int64_t)sc.WH * sc.F >= ((int64_t)1 << 28))
+		return false;
+	if (sc.sPx == 4 && sc.sPt == 4) return all >= 4000000;
+	if (sc.sPt != 1) return false;
+	if (sc.sPx == 8) return all >= 4000000 && cand >= 640;
+	return (sc.sPx == 7 || sc.sPx == 11) && all >= 1000000;
+}
+using BoundKernel = void (*)(BMB_ARGS);
+template <int PX, int PT> BoundKernel bound_of(bool mc, bool ch)
+{
+	return mc ? (ch ? bm_bound_kernel<PX, PT, true, true> : bm_bound_kernel<PX, PT, true, false>)
+	          : (ch ? bm_bound_kernel<PX, PT, false, true> : bm_bound_kernel<PX, PT, false, false>);
+}
+// Buffers: ranges and (mid, scale), integer samples (32 past the end: a row's
+// words reach over it), norms, the list.
+static void bm_bound_reserve(bm4dof_ctx *ctx, const StepConst &sc, int step, int G)
+{
+	const size_t WHF = (size_t)sc.WH * sc.F;
+	(void)ctx->bmq_part.as<float2>(BMQ_RANGE_BLOCKS + 1);
+	(void)ctx->bmq_img.as<int16_t>((step == 1 ? 1 : sc.C) * WHF * sc.sPt + 32);
+	(void)ctx->bmq_norm.as<uint32_t>(WHF);
+	(void)ctx->bmq_list.as<uint32_t>((size_t)G + 1);
+}
+static void bm_bound(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, const float *ff,
+                     const float *bf, const uint32_t *d_gpos, const uint32_t *d_gtile, const TileBox *d_tiles, int G,
+                     uint32_t *d_idx, uint32_t *d_nsim, uint32_t *d_ties, int maxCand, size_t lds)
+{
+	const int sWt = sc.wtf + sc.wtb + 1, nch = step == 1 ? 1 : sc.C;
+	const int64_t WHF = (int64_t)sc.WH * sc.F;
+	hipStream_t st = ctx->stream;
+	bm_bound_reserve(ctx, sc, step, G);
+	float2 *part = ctx->bmq_part.as<float2>(BMQ_RANGE_BLOCKS + 1), *qp = part + BMQ_RANGE_BLOCKS;
+	int16_t *qimg = ctx->bmq_img.as<int16_t>((size_t)nch * WHF * sc.sPt + 32);
+	uint32_t *norm = ctx->bmq_norm.as<uint32_t>((size_t)WHF);
+	uint32_t *list = ctx->bmq_list.as<uint32_t>((size_t)G + 1);
+	int4 *d_wins = ctx->bm_wins.as<int4>((size_t)G * sWt);
+	int2 *d_wmeta = ctx->bm_wmeta.as<int2>((size_t)G);
+	fill_u32(ctx, list, 0u, 1);
+	// the channels the distances run on: the first nch planes of a frame
+	const int nf = sc.WH * nch, rx = std::min(32, nblk(nf, 1024)), ry = std::min(sc.F, BMQ_RANGE_BLOCKS / rx);
+	hipLaunchKernelGGL(bmq_range_kernel, dim3(rx, ry), dim3(256), 0, st, img, sc.WHC, nf, sc.F, part);
+	const int nblocks = rx * ry;
+	const float Q = floorf(sqrtf(2147483648.f / (float)(sc.P * nch))) - 2.f;
+	hipLaunchKernelGGL(bmq_scale_kernel, dim3(1), dim3(64), 0, st, part, nblocks, Q, qp);
+	hipLaunchKernelGGL(sc.sPt == 4 ? bmq_pack_kernel<4> : bmq_pack_kernel<1>, dim3(nblk(nch * WHF, 256)), dim3(256), 0, st, img, sc.WH, sc.WHC, sc.F, WHF,
+	                   nch * WHF, qp, qimg);
+	const auto nk = sc.sPx == 4 ? bmq_norm_kernel<4, 4> : sc.sPx == 8 ? bmq_norm_kernel<8, 1>
+	                : sc.sPx == 7 ? bmq_norm_kernel<7, 1> : bmq_norm_kernel<11, 1>;
+	hipLaunchKernelGGL(nk, dim3(nblk(WHF, 256)), dim3(256), 0, st, qimg, sc.W, sc.WH / sc.W, sc.F, WHF, nch, norm);
+	hipLaunchKernelGGL(bm_window_kernel, dim3(nblk(G, 256)), dim3(256), 0, st, ff, bf, d_gpos, d_gtile, d_tiles, sc, G,
+	                   d_wins, d_wmeta);
+	HIPCHK(hipGetLastError());
+	// row chunks per candidate column: the fewest steps (rows, and half a
+	// step for each row a chunk loads first) over rounds of 64 items of 2
+	// columns (11x11: 1)
+	int rchunks = 1, best = 1 << 30;
+	const int cols = nblk(sc.sWx, sc.sPx <= 8 ? 2 : 1) * std::min(sWt, sc.F - sc.sPt + 1);
+	for (int r = 1; r <= std::min(sc.sWx, 8); r++) {
+		const int cost = nblk((int64_t)cols * r, 64) * (2 * nblk(sc.sWx, r) + sc.sPx - 1);
+		if (cost < best) best = cost, rchunks = r;
+	}
+	const auto kern = sc.sPx == 4 ? bound_of<4, 4>(nch > 1, rchunks > 1) : sc.sPx == 8 ? bound_of<8, 1>(nch > 1, rchunks > 1)
+	                  : sc.sPx == 7 ? bound_of<7, 1>(nch > 1, rchunks > 1) : bound_of<11, 1>(nch > 1, rchunks > 1);
+	hipLaunchKernelGGL(kern, dim3(G), dim3(64), std::max((size_t)maxCand * 4, (size_t)256 * 8), st, img, qimg, norm, qp, d_wins, d_wmeta, d_gpos,
+	                   d_gtile, d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, list, list + 1);
+	if ((sc.sPx == 4 || sc.sPx == 8) && maxCand * 8 <= 56 * 1024) {
+		const auto reg = nch == 1 ? (sc.sPx == 4 ? bm_reg_kernel<4, 4, false, true> : bm_reg_kernel<8, 1, false, true>)
+		                          : (sc.sPx == 4 ? bm_reg_kernel<4, 4, true, true> : bm_reg_kernel<8, 1, true, true>);
+		const int rc = std::max(1, std::min(sc.sWx, 64 / std::max(1, sWt * sc.sWx)));
+		hipLaunchKernelGGL(reg, dim3((unsigned)std::min(G, 8192)), dim3(64), (size_t)maxCand * 8, st, img, d_wins, d_wmeta,
+		                   d_gpos, d_gtile, d_tiles, sc, rc, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G, list);
+	} else
+		hipLaunchKernelGGL(bm_list_kernel, dim3((unsigned)std::min(G, 2048)), dim3(256), lds, st, img, ff, bf, d_gpos,
+		                   d_gtile, d_tiles, sc, step, maxCand, d_idx, d_nsim, G, list, list + 1, d_ties, d_ties + 1);
+	HIPCHK(hipGetLastError());
+}
+
 // Block matching of all groups of a step.
 void run_bm(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, const float *ff,
             const float *bf, const uint32_t *d_gpos, const uint32_t *d_gtile, const TileBox *d_tiles,
@@ -568,6 +678,11 @@ void run_bm(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, co
 	                                             (size_t)maxCand);
 	const size_t lds_fast = ((size_t)maxCand + stage_floats) * 4;
 	const size_t lds_reg = (size_t)maxCand * 8;
+	if (ctx->fast_bm == 2 && bm_bound_ok(sc, step, G)) {
+		bm_bound(ctx, sc, step, img, ff, bf, d_gpos, d_gtile, d_tiles, G, d_idx, d_nsim, d_ties, maxCand, lds);
+		bm_ties(ctx, sc, step, img, ff, bf, d_gpos, d_gtile, d_tiles, G, d_idx, d_nsim, d_ties, maxCand, lds);
+		return;
+	}
 	if (ctx->fast_bm == 2 && shape_ok && lds_reg <= 56 * 1024) {
 		int4 *d_wins = ctx->bm_wins.as<int4>((size_t)G * sWt);
 		int2 *d_wmeta = ctx->bm_wmeta.as<int2>((size_t)G);
@@ -577,10 +692,10 @@ void run_bm(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, co
 		// row chunks per candidate column: enough work items for a wave
 		const int rchunks = std::max(1, std::min(sc.sWx, 64 / std::max(1, sWt * sc.sWx)));
 		const int nch = step == 1 ? 1 : sc.C;
-		auto kern = nch == 1 ? (PX == 4 ? bm_reg_kernel<4, 4, false> : bm_reg_kernel<8, 1, false>)
-		                     : (PX == 4 ? bm_reg_kernel<4, 4, true> : bm_reg_kernel<8, 1, true>);
+		auto kern = nch == 1 ? (PX == 4 ? bm_reg_kernel<4, 4, false, false> : bm_reg_kernel<8, 1, false, false>)
+		                     : (PX == 4 ? bm_reg_kernel<4, 4, true, false> : bm_reg_kernel<8, 1, true, false>);
 		hipLaunchKernelGGL(kern, dim3(G), dim3(64), lds_reg, ctx->stream, img, d_wins, d_wmeta, d_gpos, d_gtile,
-		                   d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G);
+		                   d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G, (const uint32_t *)nullptr);
 		HIPCHK(hipGetLastError());
 		bm_ties(ctx, sc, step, img, ff, bf, d_gpos, d_gtile, d_tiles, G, d_idx, d_nsim, d_ties, maxCand, lds);
 		return;
@@ -1056,6 +1171,7 @@ void reserve_step(bm4dof_ctx *ctx, const StepPlan &pl)
 	(void)ctx->bm_wins.as<int4>(G * sWt);
 	(void)ctx->ties.as<uint32_t>(G + 1);
 	(void)ctx->bm_wmeta.as<int2>(G);
+	if (bm_bound_ok(pl.sc, pl.step1 ? 1 : 2, (int)G)) bm_bound_reserve(ctx, pl.sc, pl.step1 ? 1 : 2, (int)G);
 	if (pl.learned) {
 		(void)ctx->gflag.as<uint8_t>(G);
 		(void)ctx->fmask.as<uint8_t>(pl.WHF);

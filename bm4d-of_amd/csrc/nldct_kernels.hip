@@ -1002,14 +1002,15 @@ __device__ __forceinline__ void bmr_load_row(float (&dst)[PT][PX], const float *
 		}
 }
 
-template <int PX, int PT, bool MC>
+// LIST: the groups to match are list[1 ..], list[0] of them (grid-stride).
+template <int PX, int PT, bool MC, bool LIST>
 __global__ __launch_bounds__(64)
 void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
                    const int2 *__restrict__ wmeta, const uint32_t *__restrict__ gpos,
                    const uint32_t *__restrict__ gtile, const TileBox *__restrict__ tiles,
                    StepConst sc, int rchunks, int nch, uint32_t *__restrict__ out_idx,
                    uint32_t *__restrict__ out_nsim, int G, uint32_t *__restrict__ tie_count,
-                   uint32_t *__restrict__ tie_list, int tie_cap)
+                   uint32_t *__restrict__ tie_list, int tie_cap, const uint32_t *__restrict__ list)
 {
 	constexpr int PP = PX * PX * PT;
 	extern __shared__ unsigned char smem[];
@@ -1021,14 +1022,16 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 	__shared__ uint32_t out_key[64];
 	__shared__ int out_rank[64];
 
-	const int g = blockIdx.x;
-	if (g >= G) return;
 	const int lane = threadIdx.x;
+	const int count = LIST ? (int)min(list[0], (uint32_t)G) : G;
+	for (int gi = blockIdx.x; gi < count; gi += gridDim.x) {
+	const int g = LIST ? (int)list[gi + 1] : gi;
 	const uint32_t pos = gpos[g];
 	uint32_t *oidx = out_idx + (size_t)g * sc.npmax;
 	if (sc.npmax <= 1) {
 		if (lane == 0) { oidx[0] = pos; out_nsim[g] = 1; }
-		return;
+		if (!LIST) return;
+		continue;
 	}
 	int gx, gy, gt;
 	pos_decode(pos, sc.W, sc.WH, gx, gy, gt);
@@ -1196,14 +1199,509 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 	                          : false;
 	if (tie && lane == 0) bm_tie_append(g, tie_count, tie_list, tie_cap);
 	bm_emit(out_key, out_rank, nSimP, sc, gw, nframes, pos, tb, oidx, out_nsim + g);
+	if (!LIST) return;   // one group per block
+	__syncthreads();     // the next group rewrites the shared arrays
+	}
 }
 
 #define BMR_ARGS const float *, const int4 *, const int2 *, const uint32_t *, const uint32_t *, \
-	const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int
-template __global__ void bm_reg_kernel<4, 4, false>(BMR_ARGS);
-template __global__ void bm_reg_kernel<8, 1, false>(BMR_ARGS);
-template __global__ void bm_reg_kernel<4, 4, true>(BMR_ARGS);
-template __global__ void bm_reg_kernel<8, 1, true>(BMR_ARGS);
+	const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int, const uint32_t *
+template __global__ void bm_reg_kernel<4, 4, false, false>(BMR_ARGS);
+template __global__ void bm_reg_kernel<4, 4, false, true>(BMR_ARGS);
+template __global__ void bm_reg_kernel<8, 1, false, false>(BMR_ARGS);
+template __global__ void bm_reg_kernel<8, 1, false, true>(BMR_ARGS);
+template __global__ void bm_reg_kernel<4, 4, true, false>(BMR_ARGS);
+template __global__ void bm_reg_kernel<4, 4, true, true>(BMR_ARGS);
+template __global__ void bm_reg_kernel<8, 1, true, false>(BMR_ARGS);
+template __global__ void bm_reg_kernel<8, 1, true, true>(BMR_ARGS);
+
+// ---------------------------------------------------------------------------
+// Block matching by bounded distances (patches 4x4x4, 8x8x1, 7x7x1, 11x11x1).
+//
+// A group keeps its 8 to 32 nearest of some hundred to thousand candidates,
+// and the reference's float distance of one candidate is three separately
+// rounded operations a sample.  So every candidate gets a distance on integer
+// samples first, two samples an instruction, and only those that can still be
+// among the nearest get the reference's sum:
+//   q = round((v - mid) scale), |q| <= Q
+//   h = |a|^2 / 2 + |b|^2 / 2 - a.b <= 2 PC Q^2 < 2^32 for PC samples
+// (the patches' half norms from a table).
+// 2 h is the integer distance D but for the halves added (D <= 2 h <= D + 2).
+// A sample difference is off by at most 1.001 units, so sqrt(D) by at
+// most 1.001 sqrt(PC).  With T at or above the kk-th smallest D, the kk-th
+// smallest true distance is at most (sqrt(T) + 1.001 sqrt(PC))^2 units, and a
+// candidate with D > (sqrt(T) + 2.002 sqrt(PC))^2 lies above it.  The float
+// sums' own rounding (below 2e-5 of a distance) is in the slack of
+// bmq_limit.  What stays, some 40 to 100 candidates, is summed and ranked
+// exactly as bm_reg_kernel does it.  Groups with more than BMQ_CAP left, with
+// too few candidates to bound, or an image without a finite range are listed
+// and matched again (bm_reg_kernel or bm_list_kernel).
+// ---------------------------------------------------------------------------
+#define BMQ_CAP 256
+
+// Range of the first n samples of every frame (stride whc): one (min, max)
+// per block, blocks strided over the frames; a NaN or infinity makes the pair
+// (-inf, inf).
+__global__ __launch_bounds__(256)
+void bmq_range_kernel(const float *__restrict__ v, int whc, int n, int F, float2 *__restrict__ part)
+{
+	__shared__ float2 sh[4];
+	float lo = INFINITY, hi = -INFINITY;
+	bool bad = false;
+	for (int t = blockIdx.y; t < F; t += gridDim.y) {
+		const float *f = v + (size_t)t * whc;
+		for (int i0 = blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += 4 * gridDim.x * 256) {
+			float x[4];
+#pragma unroll
+			for (int u = 0; u < 4; u++) x[u] = f[min(i0 + u * (int)gridDim.x * 256, n - 1)];
+#pragma unroll
+			for (int u = 0; u < 4; u++) {
+				bad |= !(fabsf(x[u]) <= 3.0e38f);
+				lo = fminf(lo, x[u]);
+				hi = fmaxf(hi, x[u]);
+			}
+		}
+	}
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) {
+		lo = fminf(lo, __shfl_xor(lo, o, 64));
+		hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+	}
+	if (__any(bad)) lo = -INFINITY, hi = INFINITY;
+	if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = make_float2(lo, hi);
+	__syncthreads();
+	if (threadIdx.x == 0)
+		part[blockIdx.y * gridDim.x + blockIdx.x] = make_float2(fminf(fminf(sh[0].x, sh[1].x), fminf(sh[2].x, sh[3].x)),
+		                               fmaxf(fmaxf(sh[0].y, sh[1].y), fmaxf(sh[2].y, sh[3].y)));
+}
+
+// (mid, scale) for samples in +-Q, scale 0 when the range is not finite or
+// empty.  One wave.
+__global__ __launch_bounds__(64)
+void bmq_scale_kernel(const float2 *__restrict__ part, int nb, float Q, float2 *__restrict__ out)
+{
+	float lo = INFINITY, hi = -INFINITY;
+	for (int i = threadIdx.x; i < nb; i += 64) {
+		lo = fminf(lo, part[i].x);
+		hi = fmaxf(hi, part[i].y);
+	}
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) {
+		lo = fminf(lo, __shfl_xor(lo, o, 64));
+		hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+	}
+	if (threadIdx.x == 0) {
+		const float mid = 0.5f * lo + 0.5f * hi, half = 0.5f * hi - 0.5f * lo;
+		// the largest |v - mid| times scale stays below Q + 1/2; no scale for
+		// ranges whose squares leave the normal floats (then the reference's
+		// distances meet at 0 or infinity) or whose v - mid is coarse
+		const float s = half > 1e-15f && half < 1e15f && half > 1e-4f * fabsf(mid) ? Q / half * 0.9999f : 0.f;
+		*out = make_float2(mid, s);
+	}
+}
+
+// Integer samples of nch channels (out: channel planes of WHF places).  PT 1:
+// 16 bits a place; PT 4: a place holds its four frames' samples (those past
+// the last frame 0), so that a patch row is one run of memory.
+template <int PT>
+__global__ void bmq_pack_kernel(const float *__restrict__ img, int WH, int WHC, int F, int64_t WHF, int64_t n,
+                                const float2 *__restrict__ qp, int16_t *__restrict__ out)
+{
+	const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+	if (i >= n) return;
+	const int c = (int)(i / WHF);
+	const int64_t pos = i - c * WHF;
+	const int t = (int)(pos / WH), r = (int)(pos - (int64_t)t * WH);
+	const float *p = img + (int64_t)t * WHC + (int64_t)c * WH + r;
+	const float2 q = *qp;
+	int16_t v[PT];
+#pragma unroll
+	for (int k = 0; k < PT; k++) v[k] = t + k < F ? (int16_t)(int)rintf((p[(int64_t)k * WHC] - q.x) * q.y) : (int16_t)0;
+	__builtin_memcpy(out + PT * i, v, sizeof v);
+}
+template __global__ void bmq_pack_kernel<1>(const float *, int, int, int, int64_t, int64_t, const float2 *, int16_t *);
+template __global__ void bmq_pack_kernel<4>(const float *, int, int, int, int64_t, int64_t, const float2 *, int16_t *);
+
+typedef short bmq_s2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ int bmq_dot2(uint32_t a, uint32_t b, int c)
+{
+	return __builtin_amdgcn_sdot2(__builtin_bit_cast(bmq_s2, a), __builtin_bit_cast(bmq_s2, b), c, false);
+}
+
+// One row of a patch (all its frames) in words of two samples: PT 4, a
+// column's frames; PT 1, neighbours along the row (PX odd: the last word's
+// upper half is not the patch's).  A lane takes NC columns side by side, and
+// what they share is loaded once.
+template <int PX, int PT> struct BmqRow {
+	static constexpr int NW = PT == 1 ? (PX + 1) / 2 : PX * PT / 2;   // words of a patch row
+	static constexpr int NC = PX <= 8 ? 2 : 1;                        // columns a lane takes
+	static constexpr int NL = PT == 1 ? (PX + NC) / 2 : (PX + NC - 1) * PT / 2;   // words they cover
+	static constexpr int NV = PT == 1 ? NC * NW : NL;                 // words kept
+	uint32_t v[NV];
+	// p: the place of the first column
+	__device__ __forceinline__ void load(const int16_t *__restrict__ p)
+	{
+		uint32_t d[NL];
+		__builtin_memcpy(d, p, sizeof d);   // any alignment
+		if (PT > 1) {
+#pragma unroll
+			for (int k = 0; k < NV; k++) v[k] = d[k < NL ? k : 0];
+			return;
+		}
+#pragma unroll
+		for (int k = 0; k < NW; k++) {
+			v[k] = d[k < NL ? k : 0];
+			// the second column's words lie across the first's
+			if (NC == 2) v[(NC - 1) * NW + k] = k + 1 < NL ? __builtin_amdgcn_alignbit(d[k + 1 < NL ? k + 1 : 0], d[k < NL ? k : 0], 16) : d[k < NL ? k : 0] >> 16;
+		}
+	}
+	__device__ __forceinline__ uint32_t word(int o, int k) const { return v[PT == 1 ? o * NW + k : o * PT / 2 + k]; }
+	// word k of the row at p alone, samples past the patch 0
+	static __device__ __forceinline__ uint32_t ref_word(const int16_t *__restrict__ p, int k)
+	{
+		uint32_t w;
+		__builtin_memcpy(&w, p + 2 * k, sizeof w);
+		return PT == 1 && (PX & 1) && k == NW - 1 ? w & 0xffffu : w;
+	}
+};
+
+// Half the squared norm of every anchor's patch over nch channels, rounded up.
+template <int PX, int PT>
+__global__ void bmq_norm_kernel(const int16_t *__restrict__ q, int W, int H, int F, int64_t WHF, int nch,
+                                uint32_t *__restrict__ norm)
+{
+	constexpr int NW = BmqRow<PX, PT>::NW;
+	const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+	if (i >= WHF) return;
+	const int WH = W * H;
+	const int t = (int)(i / WH), r = (int)(i - (int64_t)t * WH), y = r / W, x = r - y * W;
+	if (x > W - PX || y > H - PX || t > F - PT) return;
+	int s = 0;
+	for (int c = 0; c < nch; c++)
+#pragma unroll
+		for (int hy = 0; hy < PX; hy++)
+#pragma unroll
+			for (int k = 0; k < NW; k++) {
+				const uint32_t d = BmqRow<PX, PT>::ref_word(q + PT * ((size_t)c * WHF + i + (size_t)hy * W), k);
+				s = bmq_dot2(d, d, s);
+			}
+	norm[i] = ((uint32_t)s + 1u) >> 1;
+}
+
+// Largest h that can belong to one of the kk nearest when h = T is at or
+// above the kk-th smallest.
+__device__ __forceinline__ uint32_t bmq_limit(uint32_t T, int pc)
+{
+	const float r = sqrtf(2.f * (float)T) + 2.01f * sqrtf((float)pc) + 1.f;
+	const float l = 0.5f * (r * r * 1.0001f) + 2.f;
+	return l < 4.0e9f ? (uint32_t)l : 0xfffffffeu;
+}
+
+// One wave per group; item = two candidate columns (11x11: one) of one frame
+// (CH: rchunks row chunks of them) walking down their rows with the patch rows
+// they cover in registers, so a step loads one row.  A tile's windows all have
+// nx x ny candidates.  T comes from the two smallest h of each lane's columns,
+// then again, exactly, from what stays under the first bound.
+// Bound: vector instructions, 1900 a group of 9 windows of 11 x 11 at 4x4x4 (830
+// of them products and row steps; the rest selection, the reference's sums of
+// what stays, ranks) against 4500 in bm_reg_kernel, 74 % of the time issuing.
+// The vector cache was the limit before a row's frames lay side by side and a
+// lane took two columns (3140 lines a group, now 1790; 5.8 to 5.0 ms for
+// 991 thousand groups of 960x540x20's first step); candidates over the keys
+// they came from and 7 waves a SIMD made it 4.25.  Both steps' matching:
+// 10.5 to 6.8 and 20.5 to 12.3 ms.
+template <int PX, int PT, bool MC, bool CH>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PX == 4 ? 7 : 1)))
+void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ qimg, const uint32_t *__restrict__ norm,
+                     const float2 *__restrict__ qp, const int4 *__restrict__ wins, const int2 *__restrict__ wmeta,
+                     const uint32_t *__restrict__ gpos, const uint32_t *__restrict__ gtile,
+                     const TileBox *__restrict__ tiles, StepConst sc, int rchunks, int nch,
+                     uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_nsim, int G,
+                     uint32_t *__restrict__ tie_count, uint32_t *__restrict__ tie_list,
+                     uint32_t *__restrict__ redo_count, uint32_t *__restrict__ redo_list)
+{
+	using R = BmqRow<PX, PT>;
+	constexpr int NW = R::NW, NC = R::NC;
+	extern __shared__ unsigned char smem[];
+	uint32_t *skey = (uint32_t *)smem;   // h (partial sums between channels)
+	uint64_t *cand = (uint64_t *)smem;   // then (distance << 32) | (scan index + 1; 0: the reference patch)
+	__shared__ uint16_t left[BMQ_CAP];   // scan indices that stay
+	__shared__ uint32_t out_key[64];
+	__shared__ int out_rank[64];
+	__shared__ uint32_t f_at[64];        // per frame: place of its first candidate
+	__shared__ int f_qt[64];             // and the frame
+
+	const int g = blockIdx.x;
+	if (g >= G) return;
+	const int lane = threadIdx.x;
+	const int sWt = sc.wtf + sc.wtb + 1;
+	const uint32_t pos = gpos[g];
+	uint32_t *oidx = out_idx + (size_t)g * sc.npmax;
+	const TileBox tb = tiles[gtile[g]];
+	const int2 meta = wmeta[g];
+	const int nframes = meta.x, nsrch = meta.y;
+	const int4 *gw = wins + (size_t)g * sWt;
+	const int W = sc.W, WH = sc.WH;
+	const uint32_t WHF = (uint32_t)WH * (uint32_t)sc.F;
+	const int nSimP = min(sc.npmax, nsrch);
+	int kk = 1;
+	while (kk * 2 <= nSimP) kk *= 2;
+	const int full = 2 * ((sc.sWx - 1) / 2) + 1;
+	const int nx = min(full, tb.ex - tb.ox - PX + 1), ny = min(full, tb.ey - tb.oy - PX + 1);
+	if (lane < nframes) {
+		const int4 f = gw[lane];
+		f_at[lane] = (uint32_t)f.x * (uint32_t)WH + (uint32_t)(tb.oy + (f.y >> 16)) * (uint32_t)W +
+		             (uint32_t)(tb.ox + (f.y & 0xffff));
+		f_qt[lane] = f.x;
+	}
+	__syncthreads();
+	const int nl = (nx + NC - 1) / NC;   // items of a frame's row
+	const int total = nframes * nl * (CH ? rchunks : 1);
+	const int rows = CH ? (ny + rchunks - 1) / rchunks : ny;
+	const float inx = 1.f / (float)nx, inl = 1.f / (float)nl;
+	const uint32_t na = norm[pos];
+	uint32_t lmin[NC], lmin2[NC];   // the two smallest h of each of the lane's columns
+#pragma unroll
+	for (int o = 0; o < NC; o++) lmin[o] = lmin2[o] = 0xffffffffu;
+	const int nc = MC ? nch : 1;
+	for (int c = 0; c < nc; c++) {
+		const bool last = c == nc - 1;
+		const int16_t *qc = qimg + (size_t)PT * c * WHF;
+		// -a, wave-uniform: word i of the patch from lane i
+		constexpr int NR = PX * NW;
+		uint32_t ref[NR];
+#pragma unroll
+		for (int i0 = 0; i0 < NR; i0 += 64) {
+			const int i = min(i0 + lane, NR - 1), k = i / NW;
+			uint32_t v = R::ref_word(qc + (size_t)PT * (pos + (uint32_t)k * (uint32_t)W), i - k * NW);
+			v = ((0u - v) & 0xffffu) | ((0u - (v >> 16)) << 16);
+#pragma unroll
+			for (int u = i0; u < min(i0 + 64, NR); u++) ref[u] = (uint32_t)__builtin_amdgcn_readlane((int)v, u - i0);
+		}
+		for (int it = lane; it < total; it += 64) {
+			// item = (frame, chunk, columns): small integers, so the products
+			// with the reciprocal truncate to the quotients
+			int q = (int)(((float)it + 0.5f) * inl);
+			const int cx = NC * (it - q * nl);
+			int r = 0;
+			if (CH) {
+				const int jf = (int)(((float)q + 0.5f) / (float)rchunks);
+				r = q - jf * rchunks;
+				q = jf;
+			}
+			const int y0 = CH ? min(r * rows, ny - rows) : 0;
+			const int ynew = CH ? r * rows : 0;   // rows above belong to the chunk before
+			const bool two = NC == 2 && cx + 1 < nx;
+			uint32_t at = f_at[q] + (uint32_t)(y0 * W + cx);
+			uint32_t *kout = skey + q * (nx * ny) + y0 * nx + cx;
+			R w[PX];
+			const int16_t *pl = qc + (size_t)PT * at;   // row being loaded
+#pragma unroll
+			for (int k = 0; k < PX - 1; k++) {
+				w[k].load(pl);
+				pl += PT * W;
+			}
+			for (int y = 0; y < rows; y += PX) {
+#pragma unroll
+				for (int u = 0; u < PX; u++) {
+					if (y + u < rows) {
+						w[(u + PX - 1) % PX].load(pl);
+						pl += PT * W;
+						int d[NC] = {};
+						if (!MC || last) {
+							uint32_t nb[NC];
+							__builtin_memcpy(nb, norm + at, sizeof nb);
+#pragma unroll
+							for (int o = 0; o < NC; o++) d[o] = (int)(na + nb[o]);
+						}
+						if (MC && c) {
+							d[0] += (int)kout[0];
+							if (two) d[NC - 1] += (int)kout[1];
+						}
+						at += W;
+#pragma unroll
+						for (int hy = 0; hy < PX; hy++)
+#pragma unroll
+							for (int k = 0; k < NW; k++)
+#pragma unroll
+								for (int o = 0; o < NC; o++)
+									d[o] = bmq_dot2(ref[hy * NW + k], w[(u + hy) % PX].word(o, k), d[o]);
+						// rows of the chunk before: its own store (between channels
+						// the sum must go in once)
+						const bool own = !CH || y0 + y + u >= ynew;
+						if (!MC || own) {
+							kout[0] = (uint32_t)d[0];
+							if (two) kout[1] = (uint32_t)d[NC - 1];
+						}
+						kout += nx;
+						if (!MC || last) {
+#pragma unroll
+							for (int o = 0; o < NC; o++) {
+								const uint32_t kn = own && (o == 0 || two) ? (uint32_t)d[o] : 0xffffffffu;
+								lmin2[o] = min(max(lmin[o], kn), max(min(lmin[o], kn), lmin2[o]));   // the middle one
+								lmin[o] = min(lmin[o], kn);
+							}
+						}
+					}
+				}
+			}
+		}
+	}
+	// T: at or above the kk-th smallest of these, its leading 12 bits below
+	// the largest found one by one
+	auto kth = [&](uint32_t mx, auto upto) {
+#pragma unroll
+		for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+		int b = 31 - __clz(__builtin_amdgcn_readfirstlane((int)(mx | 1u)));
+		const int bl = max(b - 11, 0);
+		uint32_t T = 0;
+		for (; b >= bl; b--)
+			if (upto(T + ((1u << b) - 1u)) < kk) T += 1u << b;
+		return T + ((1u << bl) - 1u);
+	};
+	auto of_columns = [&](uint32_t v) {
+		int n = 0;
+#pragma unroll
+		for (int o = 0; o < NC; o++) n += __popcll(__ballot(lmin[o] <= v)) + __popcll(__ballot(lmin2[o] <= v));
+		return n;
+	};
+	bool fits = qp->y > 0.f && of_columns(0xfffffffeu) >= kk;
+	int cnt = 0;
+	if (fits) {
+		uint32_t mx = 0;
+#pragma unroll
+		for (int o = 0; o < NC; o++) {
+			mx = max(mx, lmin[o] == 0xffffffffu ? 0u : lmin[o]);
+			mx = max(mx, lmin2[o] == 0xffffffffu ? 0u : lmin2[o]);
+		}
+		const uint32_t lim = bmq_limit(kth(mx, of_columns), PX * PX * PT * nch);
+		for (int b0 = 0; b0 < nsrch; b0 += 64) {
+			const int s = b0 + lane;
+			const bool take = s < nsrch && skey[s] <= lim;
+			const uint64_t m = __ballot(take);
+			const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+			                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+			if (take && at < BMQ_CAP) left[at] = (uint16_t)s;
+			cnt += __popcll(m);
+		}
+		fits = cnt <= BMQ_CAP;
+	}
+	if (!fits) {
+		if (lane == 0) redo_list[atomicAdd(redo_count, 1u)] = (uint32_t)g;
+		return;
+	}
+	__syncthreads();
+	// the kk-th smallest of all is among these: a tighter bound
+	{
+		uint32_t h[BMQ_CAP / 64], mx = 0;
+		int s[BMQ_CAP / 64];
+#pragma unroll
+		for (int k = 0; k < BMQ_CAP / 64; k++) {
+			const int e = lane + 64 * k;
+			s[k] = e < cnt ? (int)left[e] : 0;
+			h[k] = e < cnt ? skey[s[k]] : 0xffffffffu;
+			mx = max(mx, e < cnt ? h[k] : 0u);
+		}
+		const uint32_t lim = bmq_limit(kth(mx, [&](uint32_t v) {
+			int n = __popcll(__ballot(h[0] <= v));
+#pragma unroll
+			for (int k = 1; k < BMQ_CAP / 64; k++)
+				if (64 * k < cnt) n += __popcll(__ballot(h[k] <= v));
+			return n;
+		}), PX * PX * PT * nch);
+		__syncthreads();
+		int n = 0;
+#pragma unroll
+		for (int k = 0; k < BMQ_CAP / 64; k++) {
+			const bool take = h[k] <= lim;
+			const uint64_t m = __ballot(take);
+			const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+			                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+			if (take) left[at] = (uint16_t)s[k];
+			n += __popcll(m);
+		}
+		cnt = n;
+		__syncthreads();
+	}
+	const int nxy = nx * ny;
+	const float inxy = 1.f / (float)nxy;
+	int gx, gy, gt;
+	pos_decode(pos, W, WH, gx, gy, gt);
+	const int4 f0 = gw[0];
+	const int s_self = (gy - tb.oy - (f0.y >> 16)) * nx + (gx - tb.ox - (f0.y & 0xffff));
+	// the reference's distances of what stays: channels, frames, rows, columns
+	const float *a0 = img + (size_t)gt * sc.WHC + (size_t)gy * W + gx;
+	for (int e = lane; e < cnt; e += 64) {
+		const int s = (int)left[e];
+		const int j = (int)(((float)s + 0.5f) * inxy), o = s - j * nxy, qy = (int)(((float)o + 0.5f) * inx);
+		const uint32_t at = f_at[j] + (uint32_t)(qy * W + (o - qy * nx));
+		const float *b0 = img + (size_t)at + (size_t)f_qt[j] * (size_t)(sc.WHC - WH);
+		float d = 0.f;
+		for (int c = 0; c < nc; c++) {
+			const float *a = a0 + (size_t)c * WH, *b = b0 + (size_t)c * WH;
+#pragma unroll
+			for (int ht = 0; ht < PT; ht++) {
+				float v[PX][PX];
+#pragma unroll
+				for (int hy = 0; hy < PX; hy++)
+					__builtin_memcpy(v[hy], b + (size_t)ht * sc.WHC + hy * W, sizeof v[hy]);
+#pragma unroll
+				for (int hy = 0; hy < PX; hy++)
+#pragma unroll
+					for (int hx = 0; hx < PX; hx++) {
+						const float dif = a[(size_t)ht * sc.WHC + hy * W + hx] - v[hy][hx];
+						d = d + dif * dif;
+					}
+			}
+		}
+		cand[e] = ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)(s == s_self ? 0 : s + 1);
+	}
+	__syncthreads();
+	for (int e = lane; e < cnt; e += 64) {
+		const uint64_t c = cand[e];
+		int p = 0;
+		for (int j = 0; j < cnt; j++) p += cand[j] < c;
+		if (p < kk) {
+			out_key[p] = (uint32_t)(c >> 32);
+			out_rank[p] = (int)(uint32_t)c - 1;
+		}
+	}
+	__syncthreads();
+	// every distance up to the kk-th is among the ranked ones
+	if (bm_has_tie(cand, cnt, out_key, nSimP, sc.tau2) && lane == 0) bm_tie_append(g, tie_count, tie_list, G);
+	bm_emit(out_key, out_rank, nSimP, sc, gw, nframes, pos, tb, oidx, out_nsim + g);
+}
+
+// The listed groups by the general matcher.
+__global__ __launch_bounds__(BM_THREADS)
+void bm_list_kernel(const float *__restrict__ img, const float *__restrict__ fflow, const float *__restrict__ bflow,
+                    const uint32_t *__restrict__ gpos, const uint32_t *__restrict__ gtile,
+                    const TileBox *__restrict__ tiles, StepConst sc, int step, int maxCand,
+                    uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_nsim, int G,
+                    const uint32_t *__restrict__ list_count, const uint32_t *__restrict__ list,
+                    uint32_t *__restrict__ tie_count, uint32_t *__restrict__ tie_list)
+{
+	const uint32_t n = min(*list_count, (uint32_t)G);
+	for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+		bm_group<false>((int)list[i], img, fflow, bflow, gpos, gtile, tiles, sc, step, maxCand, out_idx, out_nsim, G,
+		                tie_count, tie_list, G);
+		__syncthreads();
+	}
+}
+
+#define BMB_ARGS const float *, const int16_t *, const uint32_t *, const float2 *, const int4 *, const int2 *, \
+	const uint32_t *, const uint32_t *, const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int,    \
+	uint32_t *, uint32_t *, uint32_t *, uint32_t *
+#define BMB_INST(PX, PT)                                                   \
+	template __global__ void bm_bound_kernel<PX, PT, false, false>(BMB_ARGS); \
+	template __global__ void bm_bound_kernel<PX, PT, false, true>(BMB_ARGS);  \
+	template __global__ void bm_bound_kernel<PX, PT, true, false>(BMB_ARGS);  \
+	template __global__ void bm_bound_kernel<PX, PT, true, true>(BMB_ARGS);   \
+	template __global__ void bmq_norm_kernel<PX, PT>(const int16_t *, int, int, int, int64_t, int, uint32_t *);
+BMB_INST(4, 4)
+BMB_INST(8, 1)
+BMB_INST(7, 1)
+BMB_INST(11, 1)
 
 #define BMF_ARGS const float *, const int4 *, const int2 *, const uint32_t *, const uint32_t *, \
 	const TileBox *, StepConst, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int
