@@ -248,36 +248,54 @@ __global__ void tv_warp_kernel(const float *__restrict__ I0, const float *__rest
 
 // ------------------------------------------------- primal-dual iterations
 // K iterations of the TV-L1 primal-dual scheme (tvl1flow_lib.c:165-246) per
-// launch, on LDS tiles: a block loads its TX x TY tile with a K-pixel halo
-// (clipped to the image) and iterates there; after iteration j the pixels at
-// least j pixels inside a cut halo edge are exact (an iteration reaches one
-// pixel in each direction: the divergence backwards, the gradient forwards),
-// so after K iterations the tile itself is, and only it is written back.
-// Per iteration: the TH step, divergence of p and u update for every pixel
-// (phase A), then the forward gradient of the new u and the p update
+// launch, on tiles held in registers: a lane is a column and a thread has R
+// rows of it, W waves below one another make the block, so a block covers
+// 64 x R W pixels, the tile and K pixels of halo on each side.  After
+// iteration j the pixels at least j pixels inside a cut halo edge are exact
+// (an iteration reaches one pixel in each direction: the divergence backwards,
+// the gradient forwards), so after K iterations the tile itself is, and only
+// it is written back.  Per iteration: the TH step, divergence of p and u
+// update (phase A), then the forward gradient of the new u and the p update
 // (phase B); each pixel's arithmetic is the reference's, operation for
-// operation, as in the one-iteration form.  The squared update of every
-// tile pixel and iteration is summed in double (pixels in thread order,
-// lanes by xor tree, waves in order) into part[pair][j][tile].
+// operation, as in the one-iteration form.  Left and right neighbours come
+// from the next lane, those above and below from the thread's own registers;
+// only the rows where two waves meet go through LDS.  Pixels outside the
+// image hold zeros throughout: what the reference leaves out of the
+// divergence at a border is then a zero, and p's components across the last
+// row and column stay zero because their gradients are (mask.c:43-144).  The
+// squared update of every tile pixel and iteration is summed in double in a
+// fixed order into part[pair][j][tile].
 //
 // The state (u1, u2, p11, p12, p21, p22) is double-buffered: a pair reads
 // buffer cur[pair] and writes the other.  ctl[pair] is the number of
-// iterations to run this round (0: idle).  tv_round_kernel then sums the
-// tiles' partials and applies the stopping test to each iteration of the
-// round in order (tv_round_decide); if it fires before the round's last
+// iterations to run this round (0: idle).  The pair's last block of the round
+// sums the tiles' partials and applies the stopping test to each iteration of
+// the round in order (tv_round_decide); if it fires before the round's last
 // iteration, the pair runs that many iterations again from the same source
 // buffer (an exact re-run), so the state and the iteration count are those
 // of the iteration the test fired on.
+//
+// Bound, many pairs: vector instructions, some 76 a pixel in phase B (two
+// roots in double, four quotients) and 36 in phase A, times 1.29 for the halo
+// (1.14 in x, 27 rows of 24 in y), issuing 80 % of the time at four waves a
+// SIMD; 38 pairs of 960x540, all active: 550 us a round of four iterations,
+// 2.9 TB/s.  With the state in LDS (64 x 32 tiles, 26 LDS accesses a pixel,
+// both pipes 75 % busy) both flows of 960x540x20 took 73 ms, with two columns
+// a lane or 1024 threads, which leave the loads of a block nothing to run
+// beside, 93; five or more rows a thread spill.
+// A single pair is latency: 56 x 8 tiles of two rows a thread, 9.3 us a round
+// with its test, against 14.2 and 3.7 us for 32 x 16 tiles of three waves and a
+// launch for the test.  Flow of one 333x251 pair: 11.2 to 6.7 ms; both flows
+// of 960x540x20: 82.5 to 68 ms.
 // ---------------------------------------------------------------------------
 struct TVPlanes {
 	float *u1, *u2, *p11, *p12, *p21, *p22;
 };
 
-#define TV_TX 64
-#define TV_TY 32
 #define TV_K 4
-#define TV_NT 512
-enum { TV_RUN = 0, TV_REDO = 1 };
+// mode[pair]: TV_REDO in the re-run, and TV_BLOCK for each block of the round
+// that is done.
+enum { TV_RUN = 0, TV_REDO = 1, TV_BLOCK = 2 };
 
 // The stopping test of every iteration of a round, in order
 // (tvl1flow_lib.c:165, 225), given errs[j] = the mean squared update of
@@ -285,57 +303,53 @@ enum { TV_RUN = 0, TV_REDO = 1 };
 // MAX_ITERATIONS.  state[pair] receives the final count.  A round that
 // stops before its last iteration is run again from the same source buffer
 // with that many iterations (mode TV_REDO), so the state and the count are
-// those of the iteration the test fired on.
-__device__ void tv_round_decide(int pr, int kk, const float *errs, float eps2, int K, int *__restrict__ ctl,
+// those of the iteration the test fired on.  The next round gets the
+// iterations the test needs if the updates go on falling at the last rate,
+// at most K: most solves then end with a round and are not run again.
+template <int K>
+__device__ void tv_round_decide(int pr, int kk, const float (&errs)[K], float eps2, bool redo, int *__restrict__ ctl,
                                 int *__restrict__ cur, int *__restrict__ iters, int *__restrict__ mode,
                                 int *__restrict__ state, int *__restrict__ n_active)
 {
 	const int done = iters[pr];
-	if (mode[pr] == TV_REDO) {   // the exact re-run of the iterations up to the test
-		iters[pr] = done + kk;
-		cur[pr] ^= 1;
+	int stop = -1;
+	float last = 0.f, before = 0.f;
+#pragma unroll
+	for (int j = 0; j < K; j++) {
+		if (j >= kk) continue;
+		if (stop < 0 && (!(errs[j] > eps2) || done + j + 1 >= TV_MAX_ITERATIONS)) stop = j;
+		before = last;
+		last = errs[j];
+	}
+	mode[pr] = TV_RUN;
+	if (!redo && stop >= 0 && stop < kk - 1) {
+		mode[pr] = TV_REDO;
+		ctl[pr] = stop + 1;
+		return;
+	}
+	iters[pr] = done + kk;
+	cur[pr] ^= 1;
+	if (redo || stop >= 0) {
 		state[pr] = done + kk;
 		ctl[pr] = 0;
 		atomicSub(n_active, 1);
 		return;
 	}
-	int stop = -1;
-	for (int j = 0; j < kk && stop < 0; j++)
-		if (!(errs[j] > eps2) || done + j + 1 >= TV_MAX_ITERATIONS) stop = j;
-	if (stop < 0) {
-		iters[pr] = done + kk;
-		cur[pr] ^= 1;
-		ctl[pr] = min(K, TV_MAX_ITERATIONS - (done + kk));
-	} else if (stop == kk - 1) {
-		iters[pr] = done + kk;
-		cur[pr] ^= 1;
-		state[pr] = done + kk;
-		ctl[pr] = 0;
-		atomicSub(n_active, 1);
-	} else {
-		mode[pr] = TV_REDO;
-		ctl[pr] = stop + 1;
+	int n = K;
+	if (kk > 1 && last < before) {
+		const float rate = last / before;
+		float e = last * rate;
+		for (n = 1; n < K && e > eps2; n++) e *= rate;
 	}
+	ctl[pr] = min(n, TV_MAX_ITERATIONS - (done + kk));
 }
-
-
-// Per-slot flags of a tile pixel (the LDS index is in the low 16 bits).
-enum : unsigned {
-	TVF_VALID = 1u << 16,  // the slot holds a pixel
-	TVF_TILE = 1u << 17,   // inside the tile itself (written back, counted in the error)
-	TVF_TOP = 1u << 18,    // image row 0
-	TVF_BOT = 1u << 19,    // image row ny - 1
-	TVF_LEFT = 1u << 20,   // image column 0
-	TVF_RIGHT = 1u << 21,  // image column nx - 1
-	TVF_BORDER = TVF_TOP | TVF_BOT | TVF_LEFT | TVF_RIGHT,
-};
 
 // sqrt of a double that is +0 or at least 2^-767, as the compiler's
 // correctly rounded sqrt computes it (rsq, then the Newton steps below) with
 // its range scaling left out: that scaling applies only below 2^-767, and
 // x^2 + y^2 of floats is +0 or at least 2^-298.  Same bits, five
-// instructions fewer.
-__device__ __forceinline__ double sqrt_sum_sq(double s)
+// instructions fewer.  POS: s is positive and finite.
+template <bool POS> __device__ __forceinline__ double sqrt_sum_sq(double s)
 {
 	const double y = __builtin_amdgcn_rsq(s);
 	double g = s * y, h = y * 0.5;
@@ -346,178 +360,229 @@ __device__ __forceinline__ double sqrt_sum_sq(double s)
 	g = __builtin_fma(d, h, g);
 	d = __builtin_fma(-g, g, s);
 	g = __builtin_fma(d, h, g);
+	if (POS) return g;
 	return __builtin_amdgcn_class(s, 0x260) ? s : g;   // +-0 and +inf give themselves
 }
 
-// divergence of (v1, v2) with backward differences at an image-border pixel
-// (mask.c:43-92); v1m / v2u are the left / upper neighbours.
-__device__ __forceinline__ float div_border(float v1, float v1m, float v2, float v2u, unsigned f)
+// a / d for several a and one finite d: a times the reciprocal in double
+// (two Newton steps from the float one, within 2^-51), rounded to float.  The
+// quotient of two floats is 2^-49 or more away, relatively, from where two
+// floats meet, so this is the correctly rounded quotient (of results below
+// 2^-126 the last bit can differ).
+__device__ __forceinline__ double tv_recip(float d)
 {
-	const bool top = f & TVF_TOP, bot = f & TVF_BOT, left = f & TVF_LEFT, right = f & TVF_RIGHT;
-	if (top && !left && !right) return v1 - v1m + v2;
-	if (bot && !left && !right) return v1 - v1m - v2u;
-	if (left && !top && !bot) return v1 + v2 - v2u;
-	if (right && !top && !bot) return -v1m + v2 - v2u;
-	if (top && left) return v1 + v2;
-	if (top && right) return -v1m + v2;
-	if (bot && left) return v1 - v2u;
-	return -v1m - v2u;
+	const double e = (double)d;
+	double y = (double)__builtin_amdgcn_rcpf(d);
+	y = __builtin_fma(__builtin_fma(-e, y, 1.0), y, y);
+	return __builtin_fma(__builtin_fma(-e, y, 1.0), y, y);
+}
+__device__ __forceinline__ float tv_quot(float a, double y) { return (float)((double)a * y); }
+
+// Phase A of a pixel: TH, divergence (dp1, dp2), u (tvl1flow_lib.c:170-225).
+// yg: tv_recip(g), 0 where g < TV_GRAD_IS_ZERO (the quotient then comes out
+// 0, as the reference sets it).  Returns the squared update.
+__device__ __forceinline__ float tv_pixel_u(float &u1, float &u2, float dp1, float dp2, float wx, float wy, float g,
+                                            double yg, float rc, float l_t, float theta)
+{
+	const float rho = rc + (wx * u1 + wy * u2);
+	const float lg = l_t * g;
+	float fi = tv_quot(-rho, yg);
+	fi = rho > lg ? -l_t : fi;
+	fi = rho < -lg ? l_t : fi;
+	const float v1 = u1 + fi * wx, v2 = u2 + fi * wy;
+	const float n1 = v1 + theta * dp1;
+	const float n2 = v2 + theta * dp2;
+	const float q = (n1 - u1) * (n1 - u1) + (n2 - u2) * (n2 - u2);
+	u1 = n1;
+	u2 = n2;
+	return q;
 }
 
-// kk iterations on the LDS tile (planes at L + c * PS, rows of RW floats);
-// BORDER: the tile touches the image border, so the boundary cases of the
-// divergence and gradient apply to some of its pixels.
-template <int RW, int PS, int NPT, int K, bool BORDER>
-__device__ __forceinline__ void tv_iterate(float *L, unsigned (&sl)[NPT], const float (&cwx)[NPT],
-                                           const float (&cwy)[NPT], const float (&cg)[NPT],
-                                           const float (&crc)[NPT], int kk, float l_t, float theta,
-                                           float taut, double (&err)[K])
+// Phase B: p from the forward gradient of the new u (tvl1flow_lib.c:228-245).
+__device__ __forceinline__ void tv_pixel_p(float &p11, float &p12, float &p21, float &p22, float u1x, float u1y,
+                                           float u2x, float u2y, float taut)
 {
-	constexpr int U1 = 0, U2 = PS, P11 = 2 * PS, P12 = 3 * PS, P21 = 4 * PS, P22 = 5 * PS;
+	// x^2 + y^2 in double: the squares are exact, so the fma rounds as the
+	// sum does; 2^-400 is lost in a sum that is not zero and gives a zero one
+	// a root that rounds to 0
+	const double s1 = __builtin_fma((double)u1x, (double)u1x, __builtin_fma((double)u1y, (double)u1y, 0x1p-400));
+	const double s2 = __builtin_fma((double)u2x, (double)u2x, __builtin_fma((double)u2y, (double)u2y, 0x1p-400));
+	// the reference adds 1.0 in double and stores to float; for a
+	// float t >= 0 that is the float sum 1 + t: the double sum is
+	// exact for 2^-29 <= t < 2^53, rounds to a value that rounds to 1
+	// below, and to t above, as the float sum does
+	float ng1 = 1.0f + taut * (float)sqrt_sum_sq<true>(s1);
+	float ng2 = 1.0f + taut * (float)sqrt_sum_sq<true>(s2);
+	const float b11 = p11 + taut * u1x, b12 = p12 + taut * u1y;
+	const float b21 = p21 + taut * u2x, b22 = p22 + taut * u2y;
+	const double y1 = tv_recip(ng1), y2 = tv_recip(ng2);
+	p11 = tv_quot(b11, y1);
+	p12 = tv_quot(b12, y1);
+	p21 = tv_quot(b21, y2);
+	p22 = tv_quot(b22, y2);
+	if (__builtin_expect(!(ng1 + ng2 < INFINITY), 0)) {
+		asm volatile("");   // (a branch, not both sides)
+		ng1 = 1.0f + taut * (float)sqrt_sum_sq<false>((double)u1x * u1x + (double)u1y * u1y);
+		ng2 = 1.0f + taut * (float)sqrt_sum_sq<false>((double)u2x * u2x + (double)u2y * u2y);
+		p11 = b11 / ng1;
+		p12 = b12 / ng1;
+		p21 = b21 / ng2;
+		p22 = b22 / ng2;
+	}
+}
+
+// The value of the lane before / after (first / last lane: 0).
+__device__ __forceinline__ float tv_lane_before(float v)
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));   // wave_shr:1
+}
+__device__ __forceinline__ float tv_lane_after(float v)
+{
+	return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));   // wave_shl:1
+}
+
+template <int R> struct TVRows {
+	float u1[R], u2[R], p11[R], p12[R], p21[R], p22[R];
+	float wx[R], wy[R], rc[R], g[R];
+	double yg[R];
+};
+// Rows the waves hand to each other: the first row's u, the last row's p12
+// and p22.
+template <int W> struct TVEdge {
+	float u[W][2][64], p[W][2][64];
+};
+
+// kk iterations.  x, y0: the thread's column and first row; yt: that row in
+// the tile.  XB: the block reaches the first or last column of the image.
+template <int R, int W, int K, bool XB>
+__device__ __forceinline__ void tv_iterate(TVRows<R> &t, TVEdge<W> &L, int wv, int lane, int x, int y0, int yt, int nx,
+                                           int ny, int kk, float l_t, float theta, float taut, double (&err)[K])
+{
+	constexpr int TX = 64 - 2 * K, TY = R * W - 2 * K;
+	const bool own = lane >= K && lane < TX + K && (!XB || x < nx);   // column of the tile
+	const bool side = XB && (x == 0 || x == nx - 1), out = XB && (x < 0 || x >= nx), last = XB && x == nx - 1;
 	for (int j = 0; j < kk; j++) {
-		// the flags are re-read every iteration (not held as masks across it)
-#pragma unroll
-		for (int k = 0; k < NPT; k++) asm volatile("" : "+v"(sl[k]));
-		// phase A: TH, divergence, u (tvl1flow_lib.c:170-225)
+		// with m iterations still to come: u is needed on the tile's rows
+		// -m .. TY + m, p on -m .. TY + m - 1
+		const int m = kk - 1 - j;
+		const int lo = max(-m, yt - y0), hi = min(TY + m, yt - y0 + ny - 1);   // rows of the image among them
 		double ej = 0.0;
 #pragma unroll
-		for (int k = 0; k < NPT; k++) {
-			const unsigned f = sl[k];
-			if (!(f & TVF_VALID)) continue;
-			const int e = f & 0xffff;
-			const float u1k = L[U1 + e], u2k = L[U2 + e];
-			const float wx = cwx[k], wy = cwy[k], g = cg[k];
-			const float rho = crc[k] + (wx * u1k + wy * u2k);
-			float d1, d2;
-			if (rho < -l_t * g) { d1 = l_t * wx; d2 = l_t * wy; }
-			else if (rho > l_t * g) { d1 = -l_t * wx; d2 = -l_t * wy; }
-			else if (g < TV_GRAD_IS_ZERO) d1 = d2 = 0;
-			else { const float fi = -rho / g; d1 = fi * wx; d2 = fi * wy; }
-			const float v1 = u1k + d1, v2 = u2k + d2;
-			const float a11 = L[P11 + e], a11m = L[P11 + e - 1], a12 = L[P12 + e], a12u = L[P12 + e - RW];
-			const float a21 = L[P21 + e], a21m = L[P21 + e - 1], a22 = L[P22 + e], a22u = L[P22 + e - RW];
-			float dp1, dp2;
-			if (!BORDER || !(f & TVF_BORDER)) {
-				dp1 = (a11 - a11m) + (a12 - a12u);
-				dp2 = (a21 - a21m) + (a22 - a22u);
-			} else {
-				dp1 = div_border(a11, a11m, a12, a12u, f);
-				dp2 = div_border(a21, a21m, a22, a22u, f);
+		for (int r = 0; r < R; r++) {
+			const int y = yt + r;
+			if (y < lo || y > hi) continue;
+			const float a11m = tv_lane_before(t.p11[r]), a21m = tv_lane_before(t.p21[r]);
+			const float a12u = r ? t.p12[r ? r - 1 : 0] : L.p[wv ? wv - 1 : 0][0][lane];
+			const float a22u = r ? t.p22[r ? r - 1 : 0] : L.p[wv ? wv - 1 : 0][1][lane];
+			const float h1 = t.p11[r] - a11m, h2 = t.p21[r] - a21m;
+			float dp1 = h1 + (t.p12[r] - a12u), dp2 = h2 + (t.p22[r] - a22u);
+			if (XB && y0 + r > 0 && y0 + r < ny - 1) {   // in the first and last column the reference sums from the left
+				dp1 = side ? (h1 + t.p12[r]) - a12u : dp1;
+				dp2 = side ? (h2 + t.p22[r]) - a22u : dp2;
 			}
-			const float n1 = v1 + theta * dp1;
-			const float n2 = v2 + theta * dp2;
-			L[U1 + e] = n1;
-			L[U2 + e] = n2;
-			// squared update of the tile's own pixels (an and-mask, not a branch)
-			const double q = (double)((n1 - u1k) * (n1 - u1k) + (n2 - u2k) * (n2 - u2k));
-			const long long tm = (f & TVF_TILE) ? -1ll : 0ll;
-			ej += __longlong_as_double(__double_as_longlong(q) & tm);
+			const float q = tv_pixel_u(t.u1[r], t.u2[r], dp1, dp2, t.wx[r], t.wy[r], t.g[r], t.yg[r], t.rc[r], l_t, theta);
+			if (y >= 0 && y < TY) ej += (double)(own ? q : 0.f);
 		}
 #pragma unroll
 		for (int q = 0; q < K; q++) if (q == j) err[q] = ej;
+		L.u[wv][0][lane] = t.u1[0];
+		L.u[wv][1][lane] = t.u2[0];
 		__syncthreads();
-		// phase B: forward gradient of the new u, p (tvl1flow_lib.c:228-245,
-		// mask.c:101-144)
 #pragma unroll
-		for (int k = 0; k < NPT; k++) {
-			const unsigned f = sl[k];
-			if (!(f & TVF_VALID)) continue;
-			const int e = f & 0xffff;
-			const float a1 = L[U1 + e], a2 = L[U2 + e];
-			const float r1 = L[U1 + e + 1], d1 = L[U1 + e + RW], r2 = L[U2 + e + 1], d2 = L[U2 + e + RW];
-			float u1x = r1 - a1, u1y = d1 - a1, u2x = r2 - a2, u2y = d2 - a2;
-			if (BORDER) {
-				if (f & TVF_RIGHT) u1x = u2x = 0.f;
-				if (f & TVF_BOT) u1y = u2y = 0.f;
+		for (int r = 0; r < R; r++) {
+			const int y = yt + r;
+			if (y < lo || y > min(hi, TY + m - 1)) continue;
+			const float d1 = r + 1 < R ? t.u1[r + 1 < R ? r + 1 : 0] : L.u[wv + 1 < W ? wv + 1 : wv][0][lane];
+			const float d2 = r + 1 < R ? t.u2[r + 1 < R ? r + 1 : 0] : L.u[wv + 1 < W ? wv + 1 : wv][1][lane];
+			float u1x = tv_lane_after(t.u1[r]) - t.u1[r], u1y = d1 - t.u1[r];
+			float u2x = tv_lane_after(t.u2[r]) - t.u2[r], u2y = d2 - t.u2[r];
+			if (XB) {
+				u1x = out || last ? 0.f : u1x;
+				u2x = out || last ? 0.f : u2x;
+				u1y = out ? 0.f : u1y;
+				u2y = out ? 0.f : u2y;
 			}
-			const float g1 = (float)sqrt_sum_sq((double)u1x * u1x + (double)u1y * u1y);
-			const float g2 = (float)sqrt_sum_sq((double)u2x * u2x + (double)u2y * u2y);
-			// the reference adds 1.0 in double and stores to float; for a
-			// float t >= 0 that is the float sum 1 + t: the double sum is
-			// exact for 2^-29 <= t < 2^53, rounds to a value that rounds to 1
-			// below, and to t above, as the float sum does
-			const float ng1 = 1.0f + taut * g1;
-			const float ng2 = 1.0f + taut * g2;
-			L[P11 + e] = (L[P11 + e] + taut * u1x) / ng1;
-			L[P12 + e] = (L[P12 + e] + taut * u1y) / ng1;
-			L[P21 + e] = (L[P21 + e] + taut * u2x) / ng2;
-			L[P22 + e] = (L[P22 + e] + taut * u2y) / ng2;
+			if (y0 + r == ny - 1) u1y = u2y = 0.f;
+			tv_pixel_p(t.p11[r], t.p12[r], t.p21[r], t.p22[r], u1x, u1y, u2x, u2y, taut);
 		}
+		L.p[wv][0][lane] = t.p12[R - 1];
+		L.p[wv][1][lane] = t.p22[R - 1];
 		__syncthreads();
 	}
 }
 
-template <int TX, int TY, int K, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+template <int R, int W, int K>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
 void tv_iter_kernel(const float *__restrict__ I1wx, const float *__restrict__ I1wy,
                     const float *__restrict__ grad, const float *__restrict__ rho_c, TVPlanes A, TVPlanes B,
                     int nx, int ny, int stride, int tiles_x, float l_t, float theta, float taut,
-                    const int *__restrict__ ctl, const int *__restrict__ cur, double *__restrict__ part)
+                    double *__restrict__ part, float eps2, int *__restrict__ ctl, int *__restrict__ cur,
+                    int *__restrict__ iters, int *__restrict__ mode, int *__restrict__ state,
+                    int *__restrict__ n_active)
 {
-	// LDS: six planes u1, u2, p11, p12, p21, p22 of the tile with its halo,
-	// rows of RW floats, one spare row before and after so that the
-	// neighbours of every slot are inside the plane
-	constexpr int RW = TX + 2 * K, RH = TY + 2 * K, EN = RW * RH, PS = EN + 2 * RW;
-	constexpr int NPT = (EN + NT - 1) / NT, NW = NT / 64;
-	constexpr int U1 = 0, U2 = PS, P11 = 2 * PS, P12 = 3 * PS, P21 = 4 * PS, P22 = 5 * PS;
-	__shared__ float L[6 * PS];
-	__shared__ double red[NW][K];
+	constexpr int TX = 64 - 2 * K, TY = R * W - 2 * K;
+	__shared__ TVEdge<W> L;
+	__shared__ double red[W][K];
 	const int pr = blockIdx.y;
 	const int kk = ctl[pr];
 	if (kk <= 0) return;
-	const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int tile = blockIdx.x, ntiles = gridDim.x;
 	const int tx0 = (tile % tiles_x) * TX, ty0 = (tile / tiles_x) * TY;
-	const int xs = max(0, tx0 - K), ys = max(0, ty0 - K);
-	const int EW = min(nx, tx0 + TX + K) - xs, EH = min(ny, ty0 + TY + K) - ys, en = EW * EH;
 	const bool flip = cur[pr] != 0;
-	const TVPlanes S = flip ? B : A;
 	const size_t off = (size_t)pr * stride;
-	float cwx[NPT], cwy[NPT], cg[NPT], crc[NPT];
-	unsigned sl[NPT];
+	auto planes = [&](bool b) {
+		return b ? TVPlanes{B.u1 + off, B.u2 + off, B.p11 + off, B.p12 + off, B.p21 + off, B.p22 + off}
+		         : TVPlanes{A.u1 + off, A.u2 + off, A.p11 + off, A.p12 + off, A.p21 + off, A.p22 + off};
+	};
+	const TVPlanes S = planes(flip), D = planes(!flip);
+	const int x = tx0 - K + lane, yt = wv * R - K, y0 = ty0 + yt;
+	const bool in = x >= 0 && x < nx;
+	TVRows<R> t = {};
+	// one byte offset a row for all planes (an image is below 4 GB)
+	auto at = [](const float *p, unsigned o) { return *(const float *)((const char *)p + o); };
 #pragma unroll
-	for (int k = 0; k < NPT; k++) {
-		const int q = tid + k * NT;
-		sl[k] = 0;
-		cwx[k] = cwy[k] = cg[k] = crc[k] = 0.f;
-		if (q < en) {
-			const int ey = q / EW, ex = q - ey * EW;
-			const int gx = xs + ex, gy = ys + ey;
-			const int e = RW + ey * RW + ex;
-			const size_t gi = off + (size_t)gy * nx + gx;
-			cwx[k] = I1wx[gi]; cwy[k] = I1wy[gi]; cg[k] = grad[gi]; crc[k] = rho_c[gi];
-			L[U1 + e] = S.u1[gi]; L[U2 + e] = S.u2[gi];
-			L[P11 + e] = S.p11[gi]; L[P12 + e] = S.p12[gi]; L[P21 + e] = S.p21[gi]; L[P22 + e] = S.p22[gi];
-			unsigned f = (unsigned)e | TVF_VALID;
-			if (gx >= tx0 && gx < tx0 + TX && gy >= ty0 && gy < ty0 + TY) f |= TVF_TILE;
-			if (gy == 0) f |= TVF_TOP;
-			if (gy == ny - 1) f |= TVF_BOT;
-			if (gx == 0) f |= TVF_LEFT;
-			if (gx == nx - 1) f |= TVF_RIGHT;
-			sl[k] = f;
-		}
+	for (int r = 0; r < R; r++) {
+		if (y0 + r < 0 || y0 + r >= ny) continue;
+		const unsigned o = 4u * (unsigned)((y0 + r) * nx + x);
+		if (!in) continue;
+		t.u1[r] = at(S.u1, o);
+		t.u2[r] = at(S.u2, o);
+		t.p11[r] = at(S.p11, o);
+		t.p12[r] = at(S.p12, o);
+		t.p21[r] = at(S.p21, o);
+		t.p22[r] = at(S.p22, o);
+		t.wx[r] = at(I1wx + off, o);
+		t.wy[r] = at(I1wy + off, o);
+		t.g[r] = at(grad + off, o);
+		t.rc[r] = at(rho_c + off, o);
 	}
+#pragma unroll
+	for (int r = 0; r < R; r++)
+		t.yg[r] = t.g[r] < TV_GRAD_IS_ZERO || t.g[r] == INFINITY ? 0.0 : tv_recip(t.g[r]);
+	L.p[wv][0][lane] = t.p12[R - 1];
+	L.p[wv][1][lane] = t.p22[R - 1];
 	double err[K];
 #pragma unroll
 	for (int j = 0; j < K; j++) err[j] = 0.0;
 	__syncthreads();
-	// block-uniform: does the tile with its halo reach the image border
-	if (xs == 0 || ys == 0 || xs + EW == nx || ys + EH == ny)
-		tv_iterate<RW, PS, NPT, K, true>(L, sl, cwx, cwy, cg, crc, kk, l_t, theta, taut, err);
+	if (tx0 - K <= 0 || tx0 + TX + K >= nx)   // block-uniform
+		tv_iterate<R, W, K, true>(t, L, wv, lane, x, y0, yt, nx, ny, kk, l_t, theta, taut, err);
 	else
-		tv_iterate<RW, PS, NPT, K, false>(L, sl, cwx, cwy, cg, crc, kk, l_t, theta, taut, err);
-	// the tile itself back to the other buffer
-	const TVPlanes D = flip ? A : B;
+		tv_iterate<R, W, K, false>(t, L, wv, lane, x, y0, yt, nx, ny, kk, l_t, theta, taut, err);
+	// the tile itself to the other buffer
+	auto put = [](float *p, unsigned o, float v) { *(float *)((char *)p + o) = v; };
 #pragma unroll
-	for (int k = 0; k < NPT; k++) {
-		const unsigned f = sl[k];
-		if (!(f & TVF_TILE)) continue;
-		const int q = tid + k * NT;
-		const int ey = q / EW, ex = q - ey * EW;
-		const int e = f & 0xffff;
-		const size_t gi = off + (size_t)(ys + ey) * nx + (xs + ex);
-		D.u1[gi] = L[U1 + e]; D.u2[gi] = L[U2 + e];
-		D.p11[gi] = L[P11 + e]; D.p12[gi] = L[P12 + e]; D.p21[gi] = L[P21 + e]; D.p22[gi] = L[P22 + e];
+	for (int r = 0; r < R; r++) {
+		if (yt + r < 0 || yt + r >= TY || y0 + r >= ny) continue;
+		if (!in || lane < K || lane >= TX + K) continue;
+		const unsigned o = 4u * (unsigned)((y0 + r) * nx + x);
+		put(D.u1, o, t.u1[r]);
+		put(D.u2, o, t.u2[r]);
+		put(D.p11, o, t.p11[r]);
+		put(D.p12, o, t.p12[r]);
+		put(D.p21, o, t.p21[r]);
+		put(D.p22, o, t.p22[r]);
 	}
 	// squared updates of the tile, per iteration
 #pragma unroll
@@ -528,35 +593,36 @@ void tv_iter_kernel(const float *__restrict__ I1wx, const float *__restrict__ I1
 		if (lane == 0) red[wv][j] = v;
 	}
 	__syncthreads();
-	if (tid < kk) {
+	if (wv > 0) return;
+	// The pair's last block to get here sums the tiles' partials and decides.
+	// The partials go past the caches of this XCD and are out before the block
+	// is counted (mode: the count above the bit); every block has read ctl and
+	// cur by then.
+	double *pp = part + (size_t)pr * K * ntiles;
+	if (lane < kk) {
 		double v = 0.0;
-		for (int w = 0; w < NW; w++) v += red[w][tid];
-		part[((size_t)pr * K + tid) * ntiles + tile] = v;
+		for (int w = 0; w < W; w++) v += red[w][lane];
+		__hip_atomic_store(pp + (size_t)lane * ntiles + tile, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	}
-}
-
-// The stopping test of a round: error of iteration j = (sum over the
-// tiles' partials) / size, then tv_round_decide.  One wave per pair: 256
-// strided sums (sum v: tiles v, v + 256, ...) held four to a lane, then a
-// tree over them (sum v += sum v + s for s = 128, 64, ..., 1).
-__global__ __launch_bounds__(64)
-void tv_round_kernel(const double *__restrict__ part, int K, int ntiles, int size, float eps2,
-                     int *__restrict__ ctl, int *__restrict__ cur, int *__restrict__ iters,
-                     int *__restrict__ mode, int *__restrict__ state, int *__restrict__ n_active)
-{
-	const int pr = blockIdx.x, lane = threadIdx.x;
-	const int kk = ctl[pr];
-	if (kk <= 0) return;
-	__shared__ float errs[TV_K];
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	int md = 0;
+	if (lane == 0) md = __hip_atomic_fetch_add(mode + pr, TV_BLOCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	md = __builtin_amdgcn_readfirstlane(md);
+	if (md / TV_BLOCK != ntiles - 1) return;
+	// error of iteration j = (sum over the tiles' partials) / pixels: 256
+	// strided sums (sum v: tiles v, v + 256, ...) held four to a lane, then a
+	// tree over them (sum v += sum v + s for s = 128, 64, ..., 1)
+	float errs[K];
 #pragma unroll
-	for (int j = 0; j < TV_K; j++) {
+	for (int j = 0; j < K; j++) {
+		errs[j] = 0.f;
 		if (j >= kk) continue;
-		const double *pj = part + ((size_t)pr * K + j) * ntiles;
 		double v[4];
 #pragma unroll
 		for (int i = 0; i < 4; i++) {
 			double e = 0.0;
-			for (int t = lane + 64 * i; t < ntiles; t += 256) e += pj[t];
+			for (int t = lane + 64 * i; t < ntiles; t += 256)
+				e += __hip_atomic_load(pp + (size_t)j * ntiles + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 			v[i] = e;
 		}
 		v[0] = v[0] + v[2];   // s = 128
@@ -567,9 +633,9 @@ void tv_round_kernel(const double *__restrict__ part, int K, int ntiles, int siz
 			const double o = __shfl_down(x, st, 64);
 			if (lane < st) x = x + o;
 		}
-		if (lane == 0) errs[j] = (float)x / (float)size;
+		errs[j] = (float)x / (float)stride;
 	}
-	if (lane == 0) tv_round_decide(pr, kk, errs, eps2, K, ctl, cur, iters, mode, state, n_active);
+	if (lane == 0) tv_round_decide<K>(pr, kk, errs, eps2, md & TV_REDO, ctl, cur, iters, mode, state, n_active);
 }
 
 // Per pair: run state of the solve of one warp.
@@ -749,22 +815,20 @@ struct TVScratch {
 constexpr int TV_MMB = 64;      // blocks of the min/max reduction per pair
 constexpr int TV_WORK = 16;     // working planes at the finest size
 
-inline int tv_tiles(int nx, int ny) { return ((nx + TV_TX - 1) / TV_TX) * ((ny + TV_TY - 1) / TV_TY); }
-
-// Scales whose 64 x 32 tiles give fewer than TV_SMALL_BLOCKS blocks over all
-// pairs run 32 x 16 tiles in blocks of three waves: more blocks to spread over
-// the CUs where the launch is too small to fill them.  A pixel's arithmetic
-// does not depend on the tile it is in.
-#define TV_STX 32
-#define TV_STY 16
-#define TV_SNT 192
-#define TV_SMALL_BLOCKS 1024
-inline bool tv_small(int nx, int ny, int P) { return (int64_t)tv_tiles(nx, ny) * P < TV_SMALL_BLOCKS; }
-inline int tv_tiles_x(int nx, int ny, int P) { return (nx + (tv_small(nx, ny, P) ? TV_STX : TV_TX) - 1) / (tv_small(nx, ny, P) ? TV_STX : TV_TX); }
-inline int tv_tiles_at(int nx, int ny, int P)
+// Shapes of the iteration blocks (rows a thread, waves): 56 x 24 pixels, or
+// 56 x 8 where those would be fewer than TV_SMALL_BLOCKS blocks over all pairs
+// and not fill the CUs.  A pixel's arithmetic does not depend on the tile it
+// is in.
+struct TVShape { int r, w; int tx() const { return 64 - 2 * TV_K; } int ty() const { return r * w - 2 * TV_K; } };
+constexpr TVShape TV_LARGE_TILE = {4, 8}, TV_SMALL_TILE = {2, 8};
+#define TV_SMALL_BLOCKS 512
+inline int tv_tiles(const TVShape &t, int nx, int ny) { return ((nx + t.tx() - 1) / t.tx()) * ((ny + t.ty() - 1) / t.ty()); }
+inline const TVShape &tv_shape(int nx, int ny, int P)
 {
-	return tv_small(nx, ny, P) ? ((nx + TV_STX - 1) / TV_STX) * ((ny + TV_STY - 1) / TV_STY) : tv_tiles(nx, ny);
+	return (int64_t)tv_tiles(TV_LARGE_TILE, nx, ny) * P < TV_SMALL_BLOCKS ? TV_SMALL_TILE : TV_LARGE_TILE;
 }
+inline int tv_tiles_x(int nx, int ny, int P) { return (nx + tv_shape(nx, ny, P).tx() - 1) / tv_shape(nx, ny, P).tx(); }
+inline int tv_tiles_at(int nx, int ny, int P) { return tv_tiles(tv_shape(nx, ny, P), nx, ny); }
 // most tiles of any scale: the per-iteration partial sums per pair
 inline int tv_part_tiles(const TVPlan &pl)
 {
@@ -905,7 +969,7 @@ void tv_flow_pairs(bm4dof_ctx *ctx, const bm4dof_tvl1_params &prm, const float *
 	// With the pinned words, a poll copies the count and the GPU runs one
 	// more round while the host waits for the copy, and a warp's iteration
 	// counts are copied at its end and read at the next poll.
-	const int max_rounds = (TV_MAX_ITERATIONS + TV_K - 1) / TV_K + 1;
+	const int max_rounds = TV_MAX_ITERATIONS + 1;
 	int guess = 0;   // most iterations of a pair in the last warp read back
 	const bool piped = ctx->tv_pin && P <= ctx->tv_pin_pairs;
 	int pend_s = -1, pend_w = -1, pend_slot = 0, nwarp = 0;
@@ -937,19 +1001,13 @@ void tv_flow_pairs(bm4dof_ctx *ctx, const bm4dof_tvl1_params &prm, const float *
 		const int g = tv_grid(n);
 		const TVPlanes SA = {u1, u2, p11, p12, p21, p22};
 		const TVPlanes SB = {tmp, tmp2, work + 12 * W, work + 13 * W, work + 14 * W, work + 15 * W};
-		const bool small = tv_small(nx, ny, P);
+		const TVShape &shape = tv_shape(nx, ny, P);
+		const auto kern = shape.r == TV_LARGE_TILE.r ? tv_iter_kernel<TV_LARGE_TILE.r, TV_LARGE_TILE.w, TV_K>
+		                                             : tv_iter_kernel<TV_SMALL_TILE.r, TV_SMALL_TILE.w, TV_K>;
 		const int tiles_x = tv_tiles_x(nx, ny, P), ntiles = tv_tiles_at(nx, ny, P);
 		auto launch_round = [&]() {
-			if (small)
-				hipLaunchKernelGGL((tv_iter_kernel<TV_STX, TV_STY, TV_K, TV_SNT>), dim3(ntiles, P), dim3(TV_SNT), 0, st,
-				                   I1wx, I1wy, grad, rho_c, SA, SB, nx, ny, n, tiles_x, l_t, prm.theta, taut, d_ctl,
-				                   d_cur, d_part);
-			else
-				hipLaunchKernelGGL((tv_iter_kernel<TV_TX, TV_TY, TV_K, TV_NT>), dim3(ntiles, P), dim3(TV_NT), 0, st,
-				                   I1wx, I1wy, grad, rho_c, SA, SB, nx, ny, n, tiles_x, l_t, prm.theta, taut, d_ctl,
-				                   d_cur, d_part);
-			hipLaunchKernelGGL(tv_round_kernel, dim3(P), dim3(64), 0, st, d_part, TV_K, ntiles, n, eps2,
-			                   d_ctl, d_cur, d_iters, d_mode, d_state, d_nact);
+			hipLaunchKernelGGL(kern, dim3(ntiles, P), dim3(64 * shape.w), 0, st, I1wx, I1wy, grad, rho_c, SA, SB, nx, ny, n,
+			                   tiles_x, l_t, prm.theta, taut, d_part, eps2, d_ctl, d_cur, d_iters, d_mode, d_state, d_nact);
 		};
 		hipLaunchKernelGGL(tv_cgrad_kernel, dim3(g, P), dim3(TV_THREADS), 0, st, I1, nx, ny, n, I1x, I1y);
 		const size_t nP = (size_t)P * n;
