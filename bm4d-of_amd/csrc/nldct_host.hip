@@ -63,6 +63,10 @@ __global__ void filter2_kernel(const float *, const float *, const uint32_t *, c
 template <int PX> __global__ void filter1_fast_kernel(FILTER1_ARGS);
 template <int PX> __global__ void coef_kernel(const float *, int, int, int, const float *, float *);
 template <int PX, int NMAX, bool TAB> __global__ void filter2_fast_kernel(FILTER2_ARGS);
+#define FILTER2W_ARGS const float *, const float *, const uint32_t *, const uint32_t *, \
+	const uint32_t *, const uint32_t *, StepConst, int, int, const float *, const float *, \
+	const float *, float *, float *, uint32_t *, uint8_t *, float *, uint32_t *, int, int, int64_t, float *
+template <int NMAX> __global__ void filter2_wide_kernel(FILTER2W_ARGS);
 #define LEARNED_ARGS const float *, const uint32_t *, const uint32_t *, const uint32_t *, const uint32_t *, \
 	StepConst, int, int, const uint16_t *, const float *, MlpInfer, float, float, float *, \
 	float *, uint32_t *, uint8_t *, float *, uint8_t *, uint32_t *, int, int
@@ -1034,7 +1038,7 @@ void check_predictive(const bm4dof_ctx *ctx, const bm4dof_params &p, int W, int 
 struct StepPlan {
 	bm4dof_params p;
 	int W = 0, H = 0, F = 0, C = 0, nparts = 0;
-	bool step1 = true, use_flow = false, learned = false, fast = false, fast_shape = false;
+	bool step1 = true, use_flow = false, learned = false, fast = false, fast_shape = false, wide = false;
 	std::vector<float> hb, hbi, hw;
 	StepGeom geo;
 	StepConst sc;
@@ -1071,7 +1075,10 @@ StepPlan plan_step(bm4dof_ctx *ctx, const bm4dof_params &p, int W, int H, int F,
 	// (np < 64: the power-of-two cut keeps at most 32), one launch per channel
 	pl.fast_shape = pl.sc.P == 64 && pl.np < 64 &&
 	                ((pl.sc.sPx == 4 && pl.sc.sPt == 4) || (pl.sc.sPx == 8 && pl.sc.sPt == 1));
-	pl.fast = ctx->fast_filter && pl.fast_shape && !pl.sc.order_inv;
+	// step 2 also for 7x7x1 and for patches of 65 to 128 samples (wide)
+	pl.wide = !pl.step1 && pl.np < 64 && pl.sc.P > 64 && pl.sc.P <= 128;
+	const bool px7 = !pl.step1 && pl.np < 64 && pl.sc.sPx == 7 && pl.sc.sPt == 1;
+	pl.fast = ctx->fast_filter && (pl.fast_shape || pl.wide || px7) && !pl.sc.order_inv;
 	if (learned && !pl.fast_shape)
 		throw ArgError("learned pass: 4x4x4 or 8x8x1 patches and fewer than 64 similar patches", BM4DOF_EUNSUPP);
 	return pl;
@@ -1081,6 +1088,7 @@ StepPlan plan_step(bm4dof_ctx *ctx, const bm4dof_params &p, int W, int H, int F,
 // group per tile) in buffers that outlive the step's launches.
 struct StepDev {
 	float *basis = nullptr, *binv = nullptr, *win = nullptr;
+	float *basis_t = nullptr;  // the basis transposed (step-2 filter of patches over 64 samples)
 	uint16_t *bsp = nullptr;   // fp16 split tables of 64-sample bases (matrix-core transforms)
 	TileBox *tiles = nullptr;
 	uint32_t *gpos = nullptr, *gtile = nullptr, *tile_first = nullptr;
@@ -1095,7 +1103,7 @@ StepDev upload_plan(bm4dof_ctx *ctx, const StepPlan &pl, DevBuf &geo_buf)
 	const size_t o_basis = 0, o_binv = o_basis + al(nb * 4), o_win = o_binv + al(nbi * 4),
 	             o_tiles = o_win + al(nw * 4), o_gpos = o_tiles + al(nt * sizeof(TileBox)),
 	             o_gtile = o_gpos + al(G * 4), o_tf = o_gtile + al(G * 4), o_bsp = o_tf + al(std::max<size_t>(ntf, 1) * 4),
-	             total = o_bsp + al(nb == 4096 ? 4 * nb * 2 : 0);
+	             o_bt = o_bsp + al(nb == 4096 ? 4 * nb * 2 : 0), total = o_bt + al(pl.wide ? nb * 4 : 0);
 	char *b = (char *)geo_buf.get(total);
 	StepDev d;
 	d.basis = (float *)(b + o_basis);
@@ -1107,6 +1115,14 @@ StepDev upload_plan(bm4dof_ctx *ctx, const StepPlan &pl, DevBuf &geo_buf)
 	d.tile_first = (uint32_t *)(b + o_tf);
 	d.bsp = nb == 4096 ? (uint16_t *)(b + o_bsp) : nullptr;
 	HIPCHK(hipMemcpy(d.basis, pl.hb.data(), nb * 4, hipMemcpyHostToDevice));
+	if (pl.wide) {
+		const size_t P = (size_t)pl.sc.P;
+		std::vector<float> t(nb);
+		for (size_t k = 0; k < P; k++)
+			for (size_t q = 0; q < P; q++) t[q * P + k] = pl.hb[k * P + q];
+		d.basis_t = (float *)(b + o_bt);
+		HIPCHK(hipMemcpy(d.basis_t, t.data(), nb * 4, hipMemcpyHostToDevice));
+	}
 	HIPCHK(hipMemcpy(d.binv, pl.hbi.data(), nbi * 4, hipMemcpyHostToDevice));
 	HIPCHK(hipMemcpy(d.win, pl.hw.data(), nw * 4, hipMemcpyHostToDevice));
 	HIPCHK(hipMemcpy(d.tiles, pl.geo.til.crop.data(), nt * sizeof(TileBox), hipMemcpyHostToDevice));
@@ -1138,7 +1154,7 @@ int64_t coef_waves(const StepConst &sc)
 size_t coef_floats(const StepPlan &pl, size_t budget)
 {
 	const int64_t waves = coef_waves(pl.sc);
-	if (!pl.fast || pl.learned || waves <= 0 || waves * 64 >= ((int64_t)1 << 32)) return 0;
+	if (!pl.fast || !pl.fast_shape || pl.learned || waves <= 0 || waves * 64 >= ((int64_t)1 << 32)) return 0;
 	const size_t per = (size_t)pl.C * pl.WHF * pl.sc.P;
 	return per * sizeof(float) * (pl.step1 ? 1 : 2) <= budget ? per : 0;
 }
@@ -1242,8 +1258,14 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 }
 
 using Filter2 = void (*)(FILTER2_ARGS);
+template <int PX> Filter2 filter2_rows_no_table(int np)
+{
+	return np < 16 ? filter2_fast_kernel<PX, 8, false> : np < 32 ? filter2_fast_kernel<PX, 16, false>
+	                                                             : filter2_fast_kernel<PX, 32, false>;
+}
 template <int PX, bool TAB> Filter2 filter2_rows(int np)
 {
+	if (!TAB) return filter2_rows_no_table<PX>(np);
 	return np < 16 ? filter2_fast_kernel<PX, 8, TAB> : np < 32 ? filter2_fast_kernel<PX, 16, TAB>
 	                                                            : filter2_fast_kernel<PX, 32, TAB>;
 }
@@ -1251,6 +1273,7 @@ template <int PX, bool TAB> Filter2 filter2_rows(int np)
 // largest power of two up to npmax).
 Filter2 filter2_of(const StepConst &sc, bool tab)
 {
+	if (sc.sPx == 7) return filter2_rows_no_table<7>(sc.npmax);
 	if (sc.sPx == 4) return tab ? filter2_rows<4, true>(sc.npmax) : filter2_rows<4, false>(sc.npmax);
 	return tab ? filter2_rows<8, true>(sc.npmax) : filter2_rows<8, false>(sc.npmax);
 }
@@ -1383,14 +1406,24 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 				                   dim3(64), 0, ctx->stream, d_nplanes, d_idx, d_nsim, d_base, dv.gtile, sc, g0,
 				                   Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile, d_early, d_gw, d_cnt, C, c,
 				                   (int64_t)WHF, d_gacc, d_coef_n);
-		else if (pl.fast) {
+		else if (pl.wide && pl.fast) {
+			const auto kern = np < 32 ? filter2_wide_kernel<16> : filter2_wide_kernel<32>;
+			for (int c = 0; c < C; c++)
+				hipLaunchKernelGGL(kern, dim3((unsigned)std::min(Gc, 25600)), dim3(128), 0, ctx->stream, d_nplanes, d_bplanes,
+				                   d_idx, d_nsim, d_base, dv.gtile, sc, g0, Gc, dv.basis_t, dv.binv, dv.win, d_est, d_ew,
+				                   d_etile, d_early, d_gw, d_cnt, C, c, (int64_t)WHF, d_gacc);
+		} else if (pl.fast) {
 			const auto kern = filter2_of(sc, d_coef_n != nullptr);
 			// about 100 blocks per CU, looping: fewer (3 per CU, all that fit)
 			// leave the row sort beside it no room, which then ends 1.4 ms
 			// after it; 8 and 32 per CU end unevenly (17.1, 15.6 against 14.9 ms)
-			const unsigned blocks = (unsigned)std::min(nblk(Gc, d_coef_n ? 4 : 2), 25600);
+			// Without tables a block first lays out both matrices (32 KB): few
+			// blocks of up to eight waves (7x7x1, 640x361x11: .72 ms, .89 with
+			// 25600, 1.22 in blocks of two waves)
+			const int waves = d_coef_n || np >= 32 ? 4 : 8;
+			const unsigned blocks = (unsigned)std::min(nblk(Gc, waves), d_coef_n ? 25600 : 1024);
 			for (int c = 0; c < C; c++)
-				hipLaunchKernelGGL(kern, dim3(blocks), dim3(d_coef_n ? 256 : 128), 0, ctx->stream, d_nplanes, d_bplanes, d_idx, d_nsim,
+				hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * waves), 0, ctx->stream, d_nplanes, d_bplanes, d_idx, d_nsim,
 				                   d_base, dv.gtile, sc, g0, Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile,
 				                   d_early, d_gw, d_cnt, C, c, (int64_t)WHF, d_gacc, d_coef_n, d_coef_b);
 		}

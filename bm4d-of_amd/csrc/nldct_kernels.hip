@@ -2130,8 +2130,9 @@ __device__ __forceinline__ void mm_load_a(const float *__restrict__ zs, float4 (
 	for (int q = 0; q < FAST_P / 4 / TS; q++) a[q] = *reinterpret_cast<const float4 *>(p + 4 * q);
 }
 
-// Column tile t of the product A B, terms in order.
-template <int ROWS>
+// Column tile t of the product A B, terms in order (those from P on are zeros
+// and left out).
+template <int ROWS, int P>
 __device__ __forceinline__ typename MmTile<ROWS>::Acc mm_product(const float4 (&a)[FAST_P / 4 / MmTile<ROWS>::TS],
                                                                  const float4 *__restrict__ bf, int t)
 {
@@ -2142,10 +2143,10 @@ __device__ __forceinline__ typename MmTile<ROWS>::Acc mm_product(const float4 (&
 #pragma unroll
 	for (int q = 0; q < Q; q++) {
 		const float4 b = bf[(t * Q + q) * 64 + l];
-		c = T::mac(a[q].x, b.x, c);
-		c = T::mac(a[q].y, b.y, c);
-		c = T::mac(a[q].z, b.z, c);
-		c = T::mac(a[q].w, b.w, c);
+		if (T::TS * (4 * q) < P) c = T::mac(a[q].x, b.x, c);
+		if (T::TS * (4 * q + 1) < P) c = T::mac(a[q].y, b.y, c);
+		if (T::TS * (4 * q + 2) < P) c = T::mac(a[q].z, b.z, c);
+		if (T::TS * (4 * q + 3) < P) c = T::mac(a[q].w, b.w, c);
 	}
 	return c;
 }
@@ -2620,7 +2621,7 @@ __device__ __forceinline__ void mm_forward(const float *__restrict__ img, const 
 	}
 #pragma unroll
 	for (int t = 0; t < FAST_P / ROWS; t++) {
-		const auto c = mm_product<ROWS>(a, bf, t);
+		const auto c = mm_product<ROWS, P>(a, bf, t);
 #pragma unroll
 		for (int r = 0; r < T::NR; r++) zs[T::row(r, h) * MM_ZS + ROWS * t + j] = c[r];
 	}
@@ -2646,7 +2647,7 @@ __device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__rest
 	float *e0 = est + (size_t)row0 * rs + ro;
 #pragma unroll
 	for (int t = 0; t < FAST_P / ROWS; t++) {
-		const auto c = mm_product<ROWS>(a, bf, t);
+		const auto c = mm_product<ROWS, P>(a, bf, t);
 		const int col = ROWS * t + j;
 		if (P < FAST_P && col >= P) continue;
 		const float ww = win ? w * win[col] : 1.f;
@@ -2669,7 +2670,7 @@ __device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__rest
 // inverse basis in LDS.  Groups dealt to the XCDs in contiguous eighths
 // fetched 4 % less and ran the same.
 template <int PX, int NMAX, bool TAB>
-__global__ __launch_bounds__(TAB ? 256 : 128) __attribute__((amdgpu_waves_per_eu(TAB ? 3 : 2)))
+__global__ __launch_bounds__(TAB || NMAX > 16 ? 256 : 512) __attribute__((amdgpu_waves_per_eu(TAB ? 3 : 2)))
 void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restrict__ basic,
                          const uint32_t *__restrict__ idx, const uint32_t *__restrict__ nsim,
                          const uint32_t *__restrict__ base, const uint32_t *__restrict__ gtile,
@@ -2682,7 +2683,7 @@ void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restric
                          float *__restrict__ gacc, const float *__restrict__ coef_n,
                          const float *__restrict__ coef_b)
 {
-	constexpr int P = PX * PX * (PX == 4 ? 4 : 1), ROWS = NMAX > 16 ? 32 : 16, NW = TAB ? 4 : 2;
+	constexpr int P = PX * PX * (PX == 4 ? 4 : 1), ROWS = NMAX > 16 ? 32 : 16, NW = TAB || NMAX > 16 ? 4 : 8;
 	__shared__ __align__(16) float4 bf[FAST_P * FAST_P / 4];                // inverse basis
 	__shared__ __align__(16) float4 bfwd[TAB ? 1 : FAST_P * FAST_P / 4];    // basis
 	__shared__ __align__(16) float zsm[NW * ROWS * MM_ZS];
@@ -2746,6 +2747,179 @@ void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restric
 		// launches before the last store unweighted rows
 		mm_inverse<P, NMAX, ROWS>(z, zs, bf, N, w, last ? win : nullptr, row0, est, C * P, c * P);
 		if (last && C > 1 && lane < P) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
+	}
+}
+
+// Step-2 filter for patches of 65 to 128 samples: two waves per group
+// (grid-stride), lane = coefficient of every row, the same transforms and
+// sums as filter2_fast_kernel.  basis_t: the basis with a term's row of
+// coefficients together, so that both matrices' operands come in whole lines
+// (they do not fit LDS beside enough groups).
+// Bound: matrix instructions, three products of 32 rows by 121 x 128 a group
+// at 11x11 (23000 cycles a wave), and at two waves a SIMD the latency of their
+// operands' loads.  512x512, 11x11x1, 7735 groups of 32 patches: 4.8 ms in
+// filter2_kernel, .67 with the loads left to the compiler, .61 with eight
+// instructions' operands ahead (one wave a SIMD), .46 with four.
+template <int NMAX>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+void filter2_wide_kernel(const float *__restrict__ noisy, const float *__restrict__ basic,
+                         const uint32_t *__restrict__ idx, const uint32_t *__restrict__ nsim,
+                         const uint32_t *__restrict__ base, const uint32_t *__restrict__ gtile,
+                         StepConst sc, int g0, int Gc,
+                         const float *__restrict__ basis_t, const float *__restrict__ binv,
+                         const float *__restrict__ win, float *__restrict__ est,
+                         float *__restrict__ entry_w, uint32_t *__restrict__ etile,
+                         uint8_t *__restrict__ early, float *__restrict__ gweight,
+                         uint32_t *__restrict__ n_early, int C, int c, int64_t cstride,
+                         float *__restrict__ gacc)
+{
+	using T = MmTile<32>;
+	constexpr int ZS = 132;   // LDS row stride: 128 terms, rows on different banks
+	__shared__ __align__(16) float zs[32 * ZS];
+	__shared__ int off[128];   // sample p's distance from the anchor
+	__shared__ float s_v[2];
+	const int P = sc.P, sPx = sc.sPx, tid = threadIdx.x;
+	const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, j = lane & 31;
+	{
+		const int q = min(tid, P - 1), r = q % (sPx * sPx);
+		off[tid] = q / (sPx * sPx) * sc.WH + r / sPx * sc.W + r % sPx;
+	}
+	__syncthreads();
+	const int steps = (P + 1) / 2, col0 = 64 * wave + j;
+	// rows a lane of instruction s and column tile t takes of a P x P matrix
+	auto operand = [&](const float *__restrict__ m, int s, int t) {
+		const int k = 2 * s + h, col = col0 + 32 * t;
+		return k < P && col < P ? m[k * P + col] : 0.f;
+	};
+	// both column tiles of rows(terms) times m, the next four instructions'
+	// operands loaded before these four run
+	auto product = [&](auto rows, const float *__restrict__ m, T::Acc &a0, T::Acc &a1) {
+		constexpr int U = 4;
+		float x[2][U], b0[2][U], b1[2][U];
+		auto load = [&](int s0, int q) {
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				x[q][u] = rows(s0 + u);
+				b0[q][u] = operand(m, s0 + u, 0);
+				b1[q][u] = operand(m, s0 + u, 1);
+			}
+		};
+		auto mac = [&](int q) {
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				a0 = T::mac(x[q][u], b0[q][u], a0);
+				a1 = T::mac(x[q][u], b1[q][u], a1);
+			}
+		};
+		load(0, 0);
+		for (int s = 0; s < steps; s += 2 * U) {   // terms from P on are zeros
+			load(s + U, 1);
+			mac(0);
+			if (s + 2 * U < steps) load(s + 2 * U, 0);
+			mac(1);
+		}
+	};
+	auto forward = [&](const float *__restrict__ img, const uint32_t *__restrict__ gidx, int N, float (&z)[NMAX]) {
+		const float *src = img + gidx[min(j, N - 1)];
+		T::Acc a0 = {}, a1 = {};
+		product([&](int s) { return j < N && 2 * s + h < P ? src[off[2 * s + h]] : 0.f; }, basis_t, a0, a1);
+#pragma unroll
+		for (int r = 0; r < T::NR; r++) {
+			zs[T::row(r, h) * ZS + col0] = a0[r];
+			zs[T::row(r, h) * ZS + col0 + 32] = a1[r];
+		}
+		wave_sync();   // a wave reads its own columns
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) z[n] = zs[n * ZS + tid];
+		wave_sync();
+	};
+	for (int gl = blockIdx.x; gl < Gc; gl += gridDim.x) {
+		const int g = g0 + gl;
+		const int N = (int)nsim[g];
+		const uint32_t row0 = base[gl];
+		const uint32_t *gidx = idx + (size_t)g * sc.npmax;
+		if (c == 0) {
+			if (tid < N) etile[row0 + tid] = gtile[g];
+			// all patches equal in every channel: written raw (see fast_early_out)
+			int differs = N <= 1;
+			for (int cc = 0; cc < C && !differs; cc++) {
+				const float *im = noisy + cc * cstride + off[tid];
+				const float v0 = im[gidx[0]];
+				for (int n = 1; n < N && !__any(differs); n++) differs |= im[gidx[n]] != v0;
+			}
+			if (!__syncthreads_or(differs)) {
+				for (int cc = 0; cc < C; cc++)
+					for (int n = 0; n < N; n++)
+						if (tid < P) est[((size_t)(row0 + n) * C + cc) * P + tid] = noisy[cc * cstride + gidx[n] + off[tid]];
+				if (tid == 0) { early[g] = 1; gweight[g] = 0.f; atomicAdd(n_early, 1u); }
+				continue;
+			}
+		} else if (early[g])
+			continue;
+		float z[NMAX], y[NMAX];
+		if (N > 0) {
+			forward(basic + c * cstride, gidx, N, y);
+			forward(noisy + c * cstride, gidx, N, z);
+		} else {
+#pragma unroll
+			for (int n = 0; n < NMAX; n++) z[n] = y[n] = 0.f;
+		}
+		haar_lane(z, N, true);
+		haar_lane(y, N, true);
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) {
+			if (n < N) {
+				const float w = y[n] * y[n] / (y[n] * y[n] + sc.beta_sigma2);
+				z[n] = z[n] * w;
+				y[n] = tid < P ? w * w : 0.f;
+			}
+		}
+		// the sum of w^2 goes on from the first wave's coefficients to the second's
+		float v = 0.f;
+		if (wave == 0) {
+			v = ordered_wave_sum(y, c ? gacc[g] : 0.f);
+			if (lane == 0) s_v[0] = v;
+		}
+		__syncthreads();
+		if (wave == 1) {
+			v = ordered_wave_sum(y, s_v[0]);
+			if (lane == 0) s_v[1] = v;
+		}
+		haar_lane(z, N, false);
+		const int at = (tid & 1) * 64 + (tid >> 1);   // a lane's terms lie together
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) zs[n * ZS + at] = z[n];
+		__syncthreads();
+		v = s_v[1];
+		const bool last = c == C - 1;
+		const float w = (float)(1. / (double)sc.sigma2 / (double)v);
+		if (tid == 0) {
+			if (last) gweight[g] = w;
+			else gacc[g] = v;
+			early[g] = 0;
+		}
+		if (last && tid < N) entry_w[row0 + tid] = w;
+		T::Acc a0 = {}, a1 = {};
+		const float *zr = zs + min(j, NMAX - 1) * ZS + 64 * h;
+		product([&](int s) { return zr[s]; }, binv, a0, a1);
+		float *e0 = est + (size_t)row0 * (C * P) + c * P;
+#pragma unroll
+		for (int t = 0; t < 2; t++) {
+			const int col = col0 + 32 * t;
+			if (col >= P) continue;
+			const float ww = last ? w * win[col] : 1.f;   // launches before the last store unweighted rows
+#pragma unroll
+			for (int r = 0; r < T::NR; r++) {
+				const int n = T::row(r, h);
+				if (n < N) e0[(size_t)n * (C * P) + col] = ww * (t ? a1 : a0)[r];
+			}
+		}
+		if (last && C > 1 && tid < P) {
+			const float ww = w * win[tid];
+			for (int n = 0; n < N; n++)
+				for (int cc = 0; cc < C - 1; cc++) est[((size_t)(row0 + n) * C + cc) * P + tid] *= ww;
+		}
+		__syncthreads();   // the next group rewrites zs and s_v
 	}
 }
 
@@ -3131,6 +3305,14 @@ FILTER2_INST(4, 32)
 FILTER2_INST(8, 8)
 FILTER2_INST(8, 16)
 FILTER2_INST(8, 32)
+template __global__ void filter2_fast_kernel<7, 8, false>(FILTER2_ARGS);
+template __global__ void filter2_fast_kernel<7, 16, false>(FILTER2_ARGS);
+template __global__ void filter2_fast_kernel<7, 32, false>(FILTER2_ARGS);
+#define FILTER2W_ARGS const float *, const float *, const uint32_t *, const uint32_t *, \
+	const uint32_t *, const uint32_t *, StepConst, int, int, const float *, const float *, \
+	const float *, float *, float *, uint32_t *, uint8_t *, float *, uint32_t *, int, int, int64_t, float *
+template __global__ void filter2_wide_kernel<16>(FILTER2W_ARGS);
+template __global__ void filter2_wide_kernel<32>(FILTER2W_ARGS);
 
 // ---------------------------------------------------------------------------
 // Aggregation in the reference's order.
