@@ -125,7 +125,7 @@ __global__ void rs_scatter_kernel(const uint32_t *, const uint32_t *, const uint
 #define AGGB_ARGS const uint32_t *, const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, \
 	StepConst, int, int, float *, float *
 __global__ void bin_order_kernel(const uint32_t *, int, uint32_t *);
-template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS>
+template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS, bool SPLIT>
 __global__ void agg_region_fold_kernel(AGGB_ARGS);
 __global__ void band_bounds_kernel(const uint32_t *, const uint32_t *, int, int, uint32_t *);
 __global__ void normalize_kernel(const float *, const float *, const float *, StepConst,
@@ -831,29 +831,45 @@ BinGrid bin_grid(const StepConst &sc)
 	return bin_grid_of(sc, sc.sPx == 8 ? BinShape{3, 3, 2} : BinShape{4, 4, 0});
 }
 
-// The fold of a step's bins and its LDS bytes (one frame of sums per frame
-// of the region the video has).
+// Regions of 4x4x4 patches over many frames.
+static bool bin_long(const StepConst &sc, const BinShape &s) { return sc.sPx == 4 && sc.sPt == 4 && s.lt > 2; }
+
+// The fold of a step's bins, its LDS bytes (one frame of sums per frame of
+// the region the video has) and its waves per region.
 struct Fold {
 	void (*kernel)(AGGB_ARGS);
 	size_t lds;
+	int waves;
 };
-template <int CC> Fold fold_of(const StepConst &sc, const BinShape &s)
+template <int CC, bool S> Fold fold_shape(const StepConst &sc, const BinShape &s)
 {
 	Fold f;
 	int fs = 384;
 	if (sc.sPx == 4 && sc.sPt == 4) {
-		f.kernel = s.lt > 2 ? agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68>
-		                    : agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68>;
+		f.kernel = bin_long(sc, s) ? agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68, false>
+		                           : agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68, S>;
 		fs = 68;
 	} else if (sc.sPx == 8) {
-		f.kernel = agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64>;
+		f.kernel = agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64, S>;
 		fs = 64;
 	} else
-		f.kernel = sc.P <= 64    ? agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384>
-		           : sc.P <= 128 ? agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384>
-		                         : agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384>;
+		f.kernel = sc.P <= 64    ? agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384, S>
+		           : sc.P <= 128 ? agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384, S>
+		                         : agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384, S>;
 	f.lds = (size_t)std::min(1 << s.lt, sc.F) * fs * (CC == 1 ? 8 : CC == 3 ? 16 : 32);
+	f.waves = S ? 4 : 1;
 	return f;
+}
+// Up to three waves a SIMD the time is that of the longest lists, and four
+// waves a region shorten them (320x240x5, 2400 regions, step 2: 1.12 -> .58
+// ms; 64x48x6: .18 -> .09; 512x512 with 11x11 patches: .33 -> .26); with more
+// regions the rows that two quarters share cost more than that gives
+// (960x540x20: 7.8 -> 14.0 ms), as with those of many frames, whose longest
+// lists are of one place (480x270x12 of 8 bits: 1.62 -> 1.88 ms).
+constexpr int FOLD_SPLIT_MAX = 3000;
+template <int CC> Fold fold_of(const StepConst &sc, const BinGrid &g)
+{
+	return g.nbins < FOLD_SPLIT_MAX && !bin_long(sc, g.s) ? fold_shape<CC, true>(sc, g.s) : fold_shape<CC, false>(sc, g.s);
 }
 
 // Device buffers of the bin lists for Mub rows: the first pass's digit
@@ -946,8 +962,8 @@ void aggregate_chunk(bm4dof_ctx *ctx, const StepConst &sc, const std::vector<uin
 			// the bin lists were built on the side stream (agg_bin_lists)
 			const BinGrid bg = bin_grid(sc);
 			const BinBufs q = bin_bufs(ctx, sc, Mub);
-			const Fold f = sc.C == 1 ? fold_of<1>(sc, bg.s) : sc.C == 3 ? fold_of<3>(sc, bg.s) : fold_of<4>(sc, bg.s);
-			hipLaunchKernelGGL(f.kernel, dim3((unsigned)bg.nbins), dim3(64), f.lds, ctx->stream, q.boff, q.order, q.v0,
+			const Fold f = sc.C == 1 ? fold_of<1>(sc, bg) : sc.C == 3 ? fold_of<3>(sc, bg) : fold_of<4>(sc, bg);
+			hipLaunchKernelGGL(f.kernel, dim3((unsigned)(bg.nbins * f.waves)), dim3(64), f.lds, ctx->stream, q.boff, q.order, q.v0,
 			                   d_erec, est, win, sc, bg.nbx, bg.nby, num, wsum);
 			HIPCHK(hipGetLastError());
 			ctx->agg_blocks += (uint64_t)bg.nbins;

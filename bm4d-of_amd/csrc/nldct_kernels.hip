@@ -4384,21 +4384,6 @@ template <int CC> struct __align__(CC == 1 ? 8 : 16) RegionAcc {
 
 // One wave per region of RX x RY pixels x RT frames; lane = sample of a
 // patch (sample lane + 64 u in slot u < PS).  The region's sums live in LDS,
-// (CC + 1) planes of RT frames at stride FS, rows at stride RS; a row of the
-// region's list is one LDS add of each covered sample per plane.  A wave's
-// LDS operations execute in order and an add rounds to nearest even like
-// v_add_f32, so every pixel's sum takes its rows in list order, one float
-// addition each: the sums computeAggregationStep{1,2} forms.
-//
-// Nothing in the row loop waits for a sum, only for the samples, which are
-// requested 16 rows ahead; per row it issues five lane reads of what the
-// chunk of 64 records holds (mask, LDS offset, row, weight), the load, and
-// CC + 1 adds.  Lanes outside the region or the row's tile are off: their
-// buffer offset is past the row's end, so they fetch nothing.
-// Strides: 4x4x4 patches meet every LDS bank once per half wave with RS = 20,
-// FS = 16 mod 64; rows of 8 samples with RS = 8 mod 16.
-// One wave per region of RX x RY pixels x RT frames; lane = sample of a
-// patch (sample lane + 64 u in slot u < PS).  The region's sums live in LDS,
 // a pixel's weight and channel sums side by side, rows at stride RS, frames
 // at FS; every row of the region's list reads, adds to and writes the sums of
 // the samples it covers.  A wave's LDS accesses execute in order, so each
@@ -4421,14 +4406,20 @@ template <int CC> struct __align__(CC == 1 ? 8 : 16) RegionAcc {
 // 6.0 -> 3.3 ms.  Adding with LDS float atomics instead took 82 ms (about
 // 160 cycles per instruction), pairs of rows without a common pixel read
 // together 9.3 ms.
-template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS>
+//
+// SPLIT: four waves share a region's list, each folds a quarter of its pixels
+// (the quarters of its width and height) and passes over the rows that miss
+// it: of a list of 8 x 8 pixels and 4 x 4 patches two in five rows are left.
+// For videos of few regions, where the time is that of the longest list.
+template <int CC, int PS, int PX, int PT, bool WIN, int LX, int LY, int LT, int RS, int FS, bool SPLIT>
 __global__ __launch_bounds__(64)
 void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *__restrict__ order,
                             const uint32_t *__restrict__ blist, const uint4 *__restrict__ erec,
                             const float *__restrict__ est, const float *__restrict__ win, StepConst sc, int nbx,
                             int nby, float *__restrict__ num, float *__restrict__ wsum)
 {
-	constexpr int RX = 1 << LX, RY = 1 << LY, RT = 1 << LT;
+	constexpr int SL = SPLIT ? 1 : 0;
+	constexpr int RX = 1 << (LX - SL), RY = 1 << (LY - SL), RT = 1 << LT;
 	constexpr int U = PS == 1 && CC == 1 ? 16 : 8;   // rows requested ahead
 	using Acc = RegionAcc<CC>;
 	static_assert(RS >= RX && FS >= RY * RS, "the region fits its array");
@@ -4436,16 +4427,17 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 	extern __shared__ char region_lds[];
 	Acc *const acc = reinterpret_cast<Acc *>(region_lds);
 	const int lane = threadIdx.x;
-	const uint32_t b = order[blockIdx.x];
+	const uint32_t b = order[blockIdx.x >> (2 * SL)];
 	const uint32_t k0 = boff[b], k1 = boff[b + 1];
 	if (k0 >= k1) return;
-	const int bx = (int)(b % (uint32_t)nbx);
+	const int bx = (int)(b % (uint32_t)nbx), part = SPLIT ? (int)blockIdx.x & 3 : 0;
 	const uint32_t rb = b / (uint32_t)nbx;
-	const int x0 = bx << LX, y0 = (int)(rb % (uint32_t)nby) << LY, t0 = (int)(rb / (uint32_t)nby) << LT;
+	const int x0 = (bx << LX) + (part & 1) * RX, y0 = ((int)(rb % (uint32_t)nby) << LY) + (part >> 1) * RY;
+	const int t0 = (int)(rb / (uint32_t)nby) << LT;
 	const int xe = min(x0 + RX, sc.W), ye = min(y0 + RY, sc.H), te = min(t0 + RT, sc.F);
 	const int px = PX ? PX : sc.sPx, pt = PT ? PT : sc.sPt, P = px * px * pt;
 	for (int i = lane; i < min(RT, sc.F) * RY * RX; i += 64) {
-		const int lx = i & (RX - 1), ly = (i >> LX) & (RY - 1), lt = i >> (LX + LY);
+		const int lx = i & (RX - 1), ly = (i >> (LX - SL)) & (RY - 1), lt = i >> (LX + LY - 2 * SL);
 		const int x = x0 + lx, y = y0 + ly, t = t0 + lt, o = lt * FS + ly * RS + lx;
 		const bool in = x < xe && y < ye && t < te;
 		Acc a;
@@ -4479,9 +4471,9 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 		const int x = (int)(rec.x - (uint32_t)t * (uint32_t)sc.WH - (uint32_t)y * (uint32_t)sc.W);
 		// the region and the interior of the row's tile, in patch samples
 		const int ty = (int)rec.y / sc.nW, tx = (int)rec.y - ty * sc.nW;
-		const int ax = max(max(x0, tx * sc.wTmp) - x, 0), ex = min(min(xe, (tx + 1) * sc.wTmp) - x, px);
-		const int ay = max(max(y0, ty * sc.hTmp) - y, 0), ey = min(min(ye, (ty + 1) * sc.hTmp) - y, px);
-		const int at = max(t0 - t, 0), et = min(te - t, pt);
+		const int ax = min(max(max(x0, tx * sc.wTmp) - x, 0), px), ex = max(min(min(xe, (tx + 1) * sc.wTmp) - x, px), 0);
+		const int ay = min(max(max(y0, ty * sc.hTmp) - y, 0), px), ey = max(min(min(ye, (ty + 1) * sc.hTmp) - y, px), 0);
+		const int at = min(max(t0 - t, 0), pt), et = max(min(te - t, pt), 0);
 		const bool live = kc + lane < k1 && ex > ax && ey > ay && et > at;
 		Meta r;
 		r.e = e;
@@ -4558,14 +4550,68 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 	auto entry = [&](uint32_t kc) { return blist[min(kc + (uint32_t)lane, k1 - 1u)]; };
 	uint32_t eN = entry(k0);
 	uint4 rN = erec[eN];
-	Meta mc = meta(k0, eN, rN);
-	eN = entry(k0 + 64);
-	rN = erec[eN];
-	uint32_t eNN = entry(k0 + 128);
+	uint32_t eNN = entry(k0 + 64), kc = k0;
+	auto chunk = [&]() {
+		const Meta m = meta(kc, eN, rN);
+		kc += 64;
+		eN = eNN;
+		rN = erec[eN];
+		eNN = entry(kc + 64);
+		return m;
+	};
+	// SPLIT: the next 64 rows that meet the quarter (fewer at the list's end),
+	// by way of a queue; the other rows' masks are empty
+	constexpr int QN = SPLIT ? 128 : 1;
+	__shared__ uint32_t q_e[QN], q_lo[PS][QN], q_hi[PS][QN];
+	__shared__ int q_o[QN];
+	__shared__ float q_w[QN];
+	int head = 0, have = 0;
+	auto queued = [&]() {
+		while (have < 64 && kc < k1) {
+			const Meta m = chunk();
+			bool any = false;
+#pragma unroll
+			for (int u = 0; u < PS; u++) any |= (m.lo[u] | m.hi[u]) != 0u;
+			const uint64_t live = __ballot(any);
+			const int at = (head + have + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32),
+			                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0u))) & (QN - 1);
+			if (any) {
+				q_e[at] = m.e;
+				q_o[at] = m.o;
+				q_w[at] = m.w;
+#pragma unroll
+				for (int u = 0; u < PS; u++) q_lo[u][at] = m.lo[u], q_hi[u][at] = m.hi[u];
+			}
+			have += __popcll(live);
+		}
+		wave_sync();
+		const int at = (head + lane) & (QN - 1);
+		Meta r;
+		r.e = lane < have ? q_e[at] : 0u;
+		r.o = lane < have ? q_o[at] : 0;
+		r.w = lane < have ? q_w[at] : 0.f;
+#pragma unroll
+		for (int u = 0; u < PS; u++) {
+			r.lo[u] = lane < have ? q_lo[u][at] : 0u;
+			r.hi[u] = lane < have ? q_hi[u][at] : 0u;
+		}
+		wave_sync();
+		const int n = min(have, 64);
+		head = (head + n) & (QN - 1);
+		have -= n;
+		return r;
+	};
+	auto next = [&]() {
+		if constexpr (SPLIT) return queued();
+		else return chunk();
+	};
+	auto more = [&]() { return SPLIT ? have > 0 || kc < k1 : kc < k1; };
+	Meta mc = next();
 	__syncthreads();   // the sums' first values are in LDS
 	Rows qa, qb;
 	request(mc, 0, qa);
-	for (uint32_t kc = k0; kc < k1; kc += 64) {
+	for (bool go = true; go;) {
+		go = more();
 		static_assert((64 / U) % 2 == 0, "packets in pairs");
 #pragma unroll
 		for (int r = 0; r < 64; r += 2 * U) {
@@ -4575,11 +4621,8 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 				request(mc, r + 2 * U, qa);
 				add(mc, r + U, qb);
 			} else {
-				const Meta mn = meta(kc + 64, eN, rN);
+				const Meta mn = next();
 				request(mn, 0, qa);
-				eN = eNN;
-				rN = erec[eN];
-				eNN = entry(kc + 192);
 				add(mc, r + U, qb);
 				mc = mn;
 			}
@@ -4587,7 +4630,7 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 	}
 	__syncthreads();
 	for (int i = lane; i < min(RT, sc.F) * RY * RX; i += 64) {
-		const int lx = i & (RX - 1), ly = (i >> LX) & (RY - 1), lt = i >> (LX + LY);
+		const int lx = i & (RX - 1), ly = (i >> (LX - SL)) & (RY - 1), lt = i >> (LX + LY - 2 * SL);
 		const int x = x0 + lx, y = y0 + ly, t = t0 + lt, o = lt * FS + ly * RS + lx;
 		if (!(x < xe && y < ye && t < te)) continue;
 		const Acc a = acc[o];
@@ -4599,13 +4642,15 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 
 #define AGGB_ARGS const uint32_t *, const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, \
 	StepConst, int, int, float *, float *
-#define AGGB_INST(CC)                                                                                       \
-	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68>(AGGB_ARGS);          \
-	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68>(AGGB_ARGS); \
-	template __global__ void agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64>(AGGB_ARGS);           \
-	template __global__ void agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);         \
-	template __global__ void agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);         \
-	template __global__ void agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384>(AGGB_ARGS);
+#define AGGB_SHAPES(CC, S)                                                                                         \
+	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, 2, 8, 68, S>(AGGB_ARGS);              \
+	template __global__ void agg_region_fold_kernel<CC, 1, 8, 1, true, 3, 3, 2, 8, 64, S>(AGGB_ARGS);               \
+	template __global__ void agg_region_fold_kernel<CC, 1, 0, 1, true, 4, 4, 0, 24, 384, S>(AGGB_ARGS);             \
+	template __global__ void agg_region_fold_kernel<CC, 2, 0, 1, true, 4, 4, 0, 24, 384, S>(AGGB_ARGS);             \
+	template __global__ void agg_region_fold_kernel<CC, 4, 0, 1, true, 4, 4, 0, 24, 384, S>(AGGB_ARGS);
+#define AGGB_INST(CC)                                                                                              \
+	AGGB_SHAPES(CC, false) AGGB_SHAPES(CC, true)                                                                    \
+	template __global__ void agg_region_fold_kernel<CC, 1, 4, 4, false, 3, 3, CC == 1 ? 5 : 4, 8, 68, false>(AGGB_ARGS);
 AGGB_INST(1)
 AGGB_INST(3)
 AGGB_INST(4)

@@ -38,3 +38,24 @@ def test_region_fold_equals_the_chunked_aggregation(ctx, w, h, f, c, nparts, px,
     big = w * h > 300 * 300
     assert ctx.stats()["agg_bt"] == ((16 if c > 1 else 32) if big else 1)
     assert np.array_equal(b0, b1, equal_nan=True) and np.array_equal(f0, f1, equal_nan=True)
+
+
+@pytest.mark.parametrize("w,h,f,c,px,pt,np_", [
+    (41, 33, 4, 1, 4, 4, 32), (57, 39, 7, 3, 4, 4, 8), (33, 30, 1, 1, 8, 1, 16), (73, 41, 5, 4, 8, 1, 8),
+    (37, 50, 2, 1, 7, 1, 8), (47, 35, 1, 3, 11, 1, 8), (49, 33, 1, 1, 15, 1, 4),      # four waves a region
+    (296, 296, 9, 1, 4, 4, 8), (441, 440, 1, 1, 8, 1, 8), (460, 430, 4, 1, 7, 1, 4)])  # one
+@pytest.mark.parametrize("flat", [False, True])
+def test_split_regions_equal_the_chunked_aggregation(ctx, w, h, f, c, px, pt, np_, flat):
+    """Few regions: four waves share a region's list; flat areas make lists of
+    one place, and rows that miss a quarter."""
+    noisy = synth.add_noise(synth.video(w, h, f, channels=c, n_shapes=6, seed=px), 20, px + 1)
+    if flat:
+        noisy[:, :, 5:, : w // 2] = np.float32(40.0)
+    a1, a2 = (A.cli_params(s, 20, noisy.shape, px=px, pt=pt, wx=7, np_=np_) for s in (1, 2))
+    try:
+        ctx.set_option("agg_binned", 0)
+        b0, f0, _ = ctx.run(a1, a2, noisy, nparts=2)
+    finally:
+        ctx.set_option("agg_binned", 1)
+    b1, f1, _ = ctx.run(a1, a2, noisy, nparts=2)
+    assert np.array_equal(b0, b1, equal_nan=True) and np.array_equal(f0, f1, equal_nan=True)
