@@ -42,12 +42,11 @@ struct AggRegion { int RX, RY, RT, tb0; };
 // frames; a patch overlaps at most 8 of them.
 struct BinShape { int lx, ly, lt; };
 
-// stable radix sort passes (sortscan.hip): threads per block, pairs per
-// thread and per block (tile)
+// stable radix sort passes (sortscan.hip): threads per block, most pairs per
+// thread
 #define RS_THREADS 64
 #define RS_IPT 256
-#define RS_TILE (RS_THREADS * RS_IPT)
-// rows per tile of the first bin-sort pass (at most 8 pairs per row)
+// most rows per tile of the first bin-sort pass (at most 8 pairs per row)
 #define BIN_RT 4096
 
 // Decode a 3-index position t*WH + y*W + x.

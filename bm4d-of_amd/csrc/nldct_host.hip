@@ -114,13 +114,13 @@ template <int CC> __global__ void agg_exact_kernel(AGG_ARGS);
 __global__ void pack_rows_kernel(const uint32_t *, const uint32_t *, const float *, int64_t, uint32_t, uint32_t,
                                  uint4 *);
 template <int CC, int CAP, int WP> __global__ void agg_chunk_kernel(AGG2_ARGS);
-__global__ void bin_hist1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int,
+__global__ void bin_hist1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int, int,
                                  uint32_t *);
-__global__ void bin_scatter1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int,
+__global__ void bin_scatter1_kernel(const uint32_t *, const uint32_t *, int64_t, StepConst, BinShape, int, int, int, int,
                                     const uint32_t *, uint32_t *, uint32_t *);
 __global__ void bin_bounds_kernel(const uint32_t *, const uint32_t *, int64_t, int, uint32_t *);
-__global__ void rs_hist_kernel(const uint32_t *, const uint32_t *, int, int, uint32_t *);
-__global__ void rs_scatter_kernel(const uint32_t *, const uint32_t *, const uint32_t *, int, int, const uint32_t *,
+__global__ void rs_hist_kernel(const uint32_t *, const uint32_t *, int, int, int, uint32_t *);
+__global__ void rs_scatter_kernel(const uint32_t *, const uint32_t *, const uint32_t *, int, int, int, const uint32_t *,
                                   uint32_t *, uint32_t *);
 #define AGGB_ARGS const uint32_t *, const uint32_t *, const uint32_t *, const uint4 *, const float *, const float *, \
 	StepConst, int, int, float *, float *
@@ -796,7 +796,7 @@ bool agg_binned_ok(const bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
 	return ctx->agg_binned && ctx->agg_chunked && sc.wTmp >= 8 && sc.hTmp >= 8 &&
 	       ((sc.sPx == 4 && sc.sPt == 4) || (sc.sPt == 1 && sc.sPx <= 16)) &&
 	       (sc.C == 1 || sc.C == 3 || sc.C == 4) && sc.H < 65536 && sc.F < 65536 &&
-	       8 * Mub < ((int64_t)1 << 32) - RS_TILE;
+	       8 * Mub < ((int64_t)1 << 32) - RS_THREADS * RS_IPT;
 }
 
 struct BinGrid {
@@ -879,21 +879,37 @@ template <int CC> Fold fold_of(const StepConst &sc, const BinGrid &g)
 struct BinBufs {
 	uint32_t *off1, *k0, *v0, *k1, *v1, *hist, *hoff, *boff, *order;
 	int nt1, nblk;   // tiles of the first pass (rows) and of the later ones (pairs)
+	int rt, ipt;     // rows of a tile, pairs per thread of one
 };
+// Tiles of the sort: a wave works through one round by round (some 2.7 us per
+// 64 rows), so small inputs take small tiles, up to SORT_TILES of them (64x48x6:
+// 223 -> 20 us the first pass); large ones stop at sizes whose counts, 256 a
+// tile, cost little beside the pairs.
+constexpr int SORT_TILES = 1024;
+static int sort_tile(int64_t n, int least, int most)
+{
+	int t = least;
+	while (t < most && n > (int64_t)t * SORT_TILES) t *= 2;
+	return t;
+}
 BinBufs bin_bufs(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
 {
 	const BinGrid bg = bin_grid(sc);
 	const size_t npair = (size_t)8 * Mub;
 	BinBufs q;
-	q.nblk = (int)((npair + RS_TILE - 1) / RS_TILE);
-	q.nt1 = (int)((Mub + BIN_RT - 1) / BIN_RT);
-	q.off1 = ctx->bin_cnt.as<uint32_t>((size_t)256 * q.nt1 + 1);
+	q.rt = sort_tile(Mub, 256, BIN_RT);
+	q.ipt = sort_tile((int64_t)(npair / RS_THREADS), 16, RS_IPT);
+	q.nblk = (int)((npair + RS_THREADS * q.ipt - 1) / (RS_THREADS * q.ipt));
+	q.nt1 = (int)((Mub + q.rt - 1) / q.rt);
+	// fewer rows may take more tiles, up to SORT_TILES
+	const size_t m1 = std::max(q.nt1, SORT_TILES), mb = std::max(q.nblk, SORT_TILES);
+	q.off1 = ctx->bin_cnt.as<uint32_t>(256 * m1 + 1);
 	q.k0 = ctx->bin_k0.as<uint32_t>(npair);
 	q.v0 = ctx->bin_list.as<uint32_t>(npair);
 	q.k1 = ctx->bin_k1.as<uint32_t>(npair);
 	q.v1 = ctx->bin_v1.as<uint32_t>(npair);
-	q.hist = ctx->bin_hist.as<uint32_t>((size_t)256 * q.nblk);
-	q.hoff = ctx->bin_hoff.as<uint32_t>((size_t)256 * q.nblk + 1);
+	q.hist = ctx->bin_hist.as<uint32_t>(256 * std::max(m1, mb));
+	q.hoff = ctx->bin_hoff.as<uint32_t>(256 * mb + 1);
 	q.boff = ctx->bin_off.as<uint32_t>((size_t)2 * bg.nbins + 1);
 	q.order = q.boff + bg.nbins + 1;
 	return q;
@@ -913,21 +929,21 @@ void agg_bin_lists(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub, const uint
 	uint32_t *kout = passes % 2 ? q.k0 : q.k1, *vout = passes % 2 ? q.v0 : q.v1;
 	// pass 0 from the rows; off1[256 nt1] = the pair count
 	hipLaunchKernelGGL(bin_hist1_kernel, dim3(side_grid(ctx, q.nt1)), dim3(64), 0, st, epos, Mp, Mub, sc, bg.s,
-	                   bg.nbx, bg.nby, q.nt1, q.hist);
+	                   bg.nbx, bg.nby, q.nt1, q.rt, q.hist);
 	dscan(ctx, 0, q.hist, (int64_t)256 * q.nt1, (int64_t)256 * q.nt1 + 1, q.off1, true);
 	const uint32_t *np = q.off1 + (size_t)256 * q.nt1;
 	hipLaunchKernelGGL(bin_scatter1_kernel, dim3(side_grid(ctx, q.nt1)), dim3(64), 0, st, epos, Mp, Mub, sc,
-	                   bg.s, bg.nbx, bg.nby, q.nt1, q.off1, kout, vout);
+	                   bg.s, bg.nbx, bg.nby, q.nt1, q.rt, q.off1, kout, vout);
 	HIPCHK(hipGetLastError());
 	uint32_t *kin = kout, *vin = vout;
 	kout = kin == q.k0 ? q.k1 : q.k0;
 	vout = vin == q.v0 ? q.v1 : q.v0;
 	for (int ps = 1; ps < passes; ps++) {
 		hipLaunchKernelGGL(rs_hist_kernel, dim3(side_grid(ctx, q.nblk)), dim3(RS_THREADS), 0, st, kin, np, 8 * ps,
-		                   q.nblk, q.hist);
+		                   q.nblk, q.ipt, q.hist);
 		dscan(ctx, 0, q.hist, (int64_t)256 * q.nblk, (int64_t)256 * q.nblk, q.hoff, true);
 		hipLaunchKernelGGL(rs_scatter_kernel, dim3(side_grid(ctx, q.nblk)), dim3(RS_THREADS), 0, st, kin, vin, np, 8 * ps, q.nblk,
-		                   q.hoff, kout, vout);
+		                   q.ipt, q.hoff, kout, vout);
 		HIPCHK(hipGetLastError());
 		std::swap(kin, kout);
 		std::swap(vin, vout);
@@ -1229,7 +1245,7 @@ void reserve_step(bm4dof_ctx *ctx, const StepPlan &pl)
 	int64_t nscan = std::max(pl.WHF + 1, G + 1);
 	if (agg_binned_ok(ctx, pl.sc, (int64_t)Mub)) {
 		const BinBufs q = bin_bufs(ctx, pl.sc, (int64_t)Mub);   // the bin sort's scans
-		nscan = std::max<int64_t>(nscan, (int64_t)256 * std::max(q.nt1, q.nblk) + 1);
+		nscan = std::max<int64_t>(nscan, (int64_t)256 * std::max({q.nt1, q.nblk, SORT_TILES}) + 1);
 	}
 	reserve_scan(ctx, nscan);
 }

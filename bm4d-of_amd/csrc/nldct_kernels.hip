@@ -4206,12 +4206,12 @@ __device__ __forceinline__ void bin_span(uint32_t q, const StepConst &sc, const 
 	}
 
 // First radix pass straight from the rows (no pair list in memory): tiles
-// of BIN_RT rows, one wave each (grid-stride over the tiles).
+// of rt rows (a multiple of 256), one wave each (grid-stride over the tiles).
 // bin_hist1_kernel: the low-digit counts of each tile's pairs, digit-major
 // (hist[d * ntiles + tile]).
 __global__ __launch_bounds__(64)
 void bin_hist1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restrict__ Mp, int64_t Mub,
-                      StepConst sc, BinShape bs, int nbx, int nby, int ntiles, uint32_t *__restrict__ hist)
+                      StepConst sc, BinShape bs, int nbx, int nby, int ntiles, int rt, uint32_t *__restrict__ hist)
 {
 	__shared__ uint32_t h[256];
 	const int lane = threadIdx.x;
@@ -4220,8 +4220,8 @@ void bin_hist1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restr
 #pragma unroll
 		for (int i = 0; i < 4; i++) h[lane + 64 * i] = 0;
 		__syncthreads();
-		const int64_t e0 = (int64_t)tile * BIN_RT;
-		for (int r0 = 0; r0 < BIN_RT && e0 + r0 < M; r0 += 256) {   // four rows per lane, loads together
+		const int64_t e0 = (int64_t)tile * rt;
+		for (int r0 = 0; r0 < rt && e0 + r0 < M; r0 += 256) {   // four rows per lane, loads together
 			uint32_t q[4];
 #pragma unroll
 			for (int u = 0; u < 4; u++) {
@@ -4246,7 +4246,7 @@ void bin_hist1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restr
 // digit's offset), as rs_scatter_kernel does for the later passes.
 __global__ __launch_bounds__(64)
 void bin_scatter1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__restrict__ Mp, int64_t Mub,
-                         StepConst sc, BinShape bs, int nbx, int nby, int ntiles, const uint32_t *__restrict__ offs,
+                         StepConst sc, BinShape bs, int nbx, int nby, int ntiles, int rt, const uint32_t *__restrict__ offs,
                          uint32_t *__restrict__ kout, uint32_t *__restrict__ vout)
 {
 	__shared__ uint32_t base[256];
@@ -4255,16 +4255,16 @@ void bin_scatter1_kernel(const uint32_t *__restrict__ epos, const uint32_t *__re
 	const uint64_t lt = (1ull << lane) - 1ull;
 	const int64_t M = min<int64_t>(Mub, (int64_t)*Mp);
 	for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-		const int64_t e0 = (int64_t)tile * BIN_RT;
+		const int64_t e0 = (int64_t)tile * rt;
 		if (e0 >= M) break;
 #pragma unroll
 		for (int i = 0; i < 4; i++) base[lane + 64 * i] = offs[(size_t)(lane + 64 * i) * ntiles + tile];
 		uint32_t qn = e0 + lane < M ? epos[e0 + lane] : 0u;   // the next round's position
 		__syncthreads();
-		for (int r0 = 0; r0 < BIN_RT && e0 + r0 < M; r0 += 64) {
+		for (int r0 = 0; r0 < rt && e0 + r0 < M; r0 += 64) {
 			const int64_t e = e0 + r0 + lane;
 			const uint32_t q = qn;
-			qn = r0 + 64 < BIN_RT && e + 64 < M ? epos[e + 64] : 0u;
+			qn = r0 + 64 < rt && e + 64 < M ? epos[e + 64] : 0u;
 			int c = 0;
 			if (e < M) BIN_FOR_PAIRS(q, key, (void)key; c++);
 			const int incl = wave_incl_scan(c);

@@ -309,14 +309,14 @@ __global__ void drop_groups_kernel(const uint32_t *__restrict__ drop, int n, uin
 
 // ------------------------------------------------------- stable radix sort
 // One LSD pass of 8-bit digits (bits [shift, shift + 8)) over (key, value)
-// pairs; the pair count n is on the device, nblk tiles of RS_TILE pairs
-// bound it.  rs_hist_kernel: digit counts per tile, digit-major
+// pairs; the pair count n is on the device, nblk tiles of ipt pairs per
+// thread (a multiple of 16) bound it.  rs_hist_kernel: digit counts per tile, digit-major
 // (hist[d * nblk + tile]); an exclusive scan of them gives every tile's
 // first output slot per digit; rs_scatter_kernel: each tile writes its
 // pairs there in input order (equal digits keep their order: stable).
 __global__ __launch_bounds__(RS_THREADS)
 void rs_hist_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ np, int shift, int nblk,
-                    uint32_t *__restrict__ hist)
+                    int ipt, uint32_t *__restrict__ hist)
 {
 	constexpr int DPT = 256 / RS_THREADS;   // digits per thread
 	__shared__ uint32_t h[256];
@@ -325,9 +325,9 @@ void rs_hist_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restric
 #pragma unroll
 		for (int i = 0; i < DPT; i++) h[threadIdx.x + i * RS_THREADS] = 0;
 		__syncthreads();
-		const uint64_t b0 = (uint64_t)tile * RS_TILE;
+		const uint64_t b0 = (uint64_t)tile * ipt * RS_THREADS;
 		if (b0 < n)
-			for (int i0 = 0; i0 < RS_IPT; i0 += 16) {   // sixteen loads in flight, then their counts
+			for (int i0 = 0; i0 < ipt; i0 += 16) {   // sixteen loads in flight, then their counts
 				uint32_t kv[16];
 #pragma unroll
 				for (int i = 0; i < 16; i++) {
@@ -355,7 +355,7 @@ void rs_hist_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restric
 // running offset, and the lowest of them advances it.
 __global__ __launch_bounds__(RS_THREADS)
 void rs_scatter_kernel(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                       const uint32_t *__restrict__ np, int shift, int nblk, const uint32_t *__restrict__ offs,
+                       const uint32_t *__restrict__ np, int shift, int nblk, int ipt, const uint32_t *__restrict__ offs,
                        uint32_t *__restrict__ kout, uint32_t *__restrict__ vout)
 {
 	static_assert(RS_THREADS == 64, "one wave per tile");
@@ -364,13 +364,13 @@ void rs_scatter_kernel(const uint32_t *__restrict__ kin, const uint32_t *__restr
 	const int lane = threadIdx.x;
 	const uint64_t n = *np;
 	for (int tile = blockIdx.x; tile < nblk; tile += gridDim.x) {
-		const uint64_t b0 = (uint64_t)tile * RS_TILE;
+		const uint64_t b0 = (uint64_t)tile * ipt * RS_THREADS;
 		if (b0 >= n) break;
 #pragma unroll
 		for (int i = 0; i < DPT; i++) base[lane + i * 64] = offs[(size_t)(lane + i * 64) * nblk + tile];
 		__syncthreads();
 		const uint64_t lt = (1ull << lane) - 1ull;
-		for (int r0 = 0; r0 < RS_IPT; r0 += BATCH) {
+		for (int r0 = 0; r0 < ipt; r0 += BATCH) {
 			if (b0 + (uint64_t)r0 * 64 >= n) break;
 			uint32_t key[BATCH], val[BATCH];
 #pragma unroll
