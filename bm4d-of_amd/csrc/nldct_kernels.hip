@@ -3027,7 +3027,6 @@ void filter2_wide_kernel(const float *__restrict__ noisy, const float *__restric
 // ---------------------------------------------------------------------------
 
 typedef _Float16 tr_f16x4 __attribute__((ext_vector_type(4)));
-constexpr int TR_ZS = 68;   // padded LDS row stride of the inverse's operand
 
 __device__ __forceinline__ void tr_split(float4 x, tr_f16x4 &hi, tr_f16x4 &lo)
 {
@@ -3104,41 +3103,6 @@ __device__ __forceinline__ void mfma_forward(const float *__restrict__ img, cons
 	}
 }
 
-// est[(row0+n)*rs + ro + p] = (w * win[p]) * sum_k Z[n][k] Bi[k][p] for n < N,
-// Z from LDS rows of stride TR_ZS.  One wave; every lane must call it.
-__device__ __forceinline__ void mfma_inverse(const float *__restrict__ zp, const uint16_t *__restrict__ bsp,
-                                             int N, float w, const float *__restrict__ win, uint32_t row0,
-                                             float *__restrict__ est, int rs, int ro)
-{
-	const int l = threadIdx.x, h = l >> 5, j = l & 31;
-	float4 z[8];
-#pragma unroll
-	for (int s = 0; s < 8; s++) z[s] = *reinterpret_cast<const float4 *>(zp + j * TR_ZS + 8 * s + 4 * h);
-	const int sh = tr_scale_exp(z);
-	tr_f16x4 ah[8], al[8];
-#pragma unroll
-	for (int s = 0; s < 8; s++) tr_split_scaled(z[s], sh, ah[s], al[s]);
-#pragma unroll
-	for (int t = 0; t < 2; t++) {
-		mlp_f32x16 c = {};
-		const uint16_t *bh = bsp + 2 * FAST_P * FAST_P + (32 * t + j) * FAST_P + 4 * h;
-		const uint16_t *bl = bh + FAST_P * FAST_P;
-#pragma unroll
-		for (int s = 0; s < 8; s++) {
-			const tr_f16x4 b_hi = tr_load4(bh + 8 * s), b_lo = tr_load4(bl + 8 * s);
-			c = __builtin_amdgcn_mfma_f32_32x32x8f16(ah[s], b_hi, c, 0, 0, 0);
-			c = __builtin_amdgcn_mfma_f32_32x32x8f16(ah[s], b_lo, c, 0, 0, 0);
-			c = __builtin_amdgcn_mfma_f32_32x32x8f16(al[s], b_hi, c, 0, 0, 0);
-		}
-		const float ww = w * win[32 * t + j];
-#pragma unroll
-		for (int r = 0; r < 16; r++) {
-			const int n = 8 * (r >> 2) + 4 * h + (r & 3);
-			if (n < N) est[(size_t)(row0 + n) * rs + ro + 32 * t + j] = ww * ldexpf(c[r], -sh);
-		}
-	}
-}
-
 // Haar-domain coefficients of a group into the lane registers z[n] (lane k),
 // and each row's distance statistic: log1p of its energy over 64 sigma^2
 // (for a detail row, the squared differences between the patch sub-means
@@ -3167,24 +3131,79 @@ __device__ __forceinline__ void learned_coeffs(const float *__restrict__ img, co
 	__syncthreads();
 }
 
-// bf16 feature rows [32][MLP_XS] from the lane registers (rows >= N zero)
-__device__ __forceinline__ void learned_features_lds(const float (&z)[FAST_NMAX], int N, float sigma,
-                                                     const float *__restrict__ rstat, uint16_t *__restrict__ xb)
+// The learned filter keeps a group in registers from its samples to its
+// rows.  The Haar transform along the group is taken before the patch
+// transform and, on the way back, after it (the two act on different axes),
+// so that it runs on lane = sample, as the rows are read and written; and
+// every product's result is the next one's operand where it lies:
+//   lane (h, j) = (l / 32, l % 32) of a 32 x 32 x 16 instruction takes row j of
+//   A and column j of B at eight terms and holds D[8 (r / 4) + 4 h + r % 4][j]
+//   in element r.  With the terms dealt as 16 s + 8 (v / 4) + 4 h + v % 4 to
+//   step s, value v, the elements of D for patch j are, in order, the operand
+//   of the next product over D's rows.
+// Lane (h, j) thus holds patch j's coefficients 8 q + 4 h + i in element
+// 4 q + i: z, the features, the hidden units and the gains alike.  Only the
+// first step, from lane = sample, goes through LDS; the way back to lane =
+// sample is a swap of the two halves' elements.
+//
+// Bound: vector instructions, some 2600 a group (the sigmoids a quarter of
+// them, the fp16 splits a fifth), beside 116 matrix instructions of 32 cycles;
+// the tables of a block, 100 KB, leave a CU two waves a SIMD.  960x540x20 (991
+// thousand groups): 20.8 ms with a wave of its own per block, weights from L2
+// and the hidden rows through LDS (61 % of the time waiting), now 9.1 ms.
+// Against 64 bits the pass is off by 9.4e-5 on average (1.03e-4 before;
+// without the first patch's mean taken off 1.06e-4: in the sample domain every
+// value then carries it through the Haar sums).
+typedef _Float16 lf_f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 lf_bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int LF_WAVES = 8;                // waves of a block: two a SIMD
+constexpr int LF_XS = 36;                  // LDS row stride of the samples on their way
+constexpr int LF_S1 = (MLP_IN + 15) / 16;  // steps of the first layer
+
+// The weights and split tables as operands in LDS, 16 bytes a lane.
+struct LearnedTables {
+	uint4 w1[4 * LF_S1 * 64], w2[4 * 8 * 64], w3[2 * 8 * 64];   // [tile][step][lane]
+	uint4 fwd[2][2 * 4 * 64], inv[2][2 * 4 * 64];               // hi, lo: [tile][step][lane]
+	float b1[MLP_H], b2[MLP_H], b3[MLP_OUT];
+	float one[FAST_P];                                          // coefficients of the constant patch 1
+};
+// Rows of `len` 16-bit values (0 past them) as operands of `steps` steps.
+__device__ __forceinline__ void lf_stage(const uint16_t *__restrict__ m, int len, int tiles, int steps,
+                                         uint4 *__restrict__ out)
 {
-	const int lane = threadIdx.x;
-	const float is = 1.f / sigma;
-#pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) xb[n * MLP_XS + lane] = f32_to_bf16(n < N ? z[n] * is : 0.f);
-	if (lane < 32) {
-		const bool live = lane < N;
-		xb[lane * MLP_XS + 64] = f32_to_bf16(live ? logf(sigma / 20.f) : 0.f);
-		xb[lane * MLP_XS + 65] = f32_to_bf16(rstat[lane]);
-		for (int k = 66; k < MLP_XS; k++) xb[lane * MLP_XS + k] = 0;
+	for (int i = threadIdx.x; i < tiles * steps * 64; i += 64 * LF_WAVES) {
+		const int l = i & 63, s = (i >> 6) % steps, t = (i >> 6) / steps;
+		const uint16_t *row = m + (32 * t + (l & 31)) * len;
+		const int k = 16 * s + 4 * (l >> 5);
+		uint2 a = {0u, 0u}, b = {0u, 0u};
+		if (k < len) __builtin_memcpy(&a, row + k, 8);
+		if (k + 8 < len) __builtin_memcpy(&b, row + k + 8, 8);
+		out[i] = make_uint4(a.x, a.y, b.x, b.y);
 	}
+}
+__device__ __forceinline__ float lf_scale(float m, int &e)   // as tr_scale_exp, m: the lane's largest |value|
+{
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+	(void)frexpf(m, &e);
+	e = 14 - e;
+	return m;
+}
+// v 2^sh in fp16 hi + lo
+__device__ __forceinline__ void lf_split(const float (&v)[32], int sh, lf_f16x8 (&hi)[4], lf_f16x8 (&lo)[4])
+{
+#pragma unroll
+	for (int s = 0; s < 4; s++)
+#pragma unroll
+		for (int u = 0; u < 8; u++) {
+			const float x = ldexpf(v[8 * s + u], sh);
+			hi[s][u] = (_Float16)x;
+			lo[s][u] = (_Float16)(x - (float)hi[s][u]);
+		}
 }
 
 template <int PX>
-__global__ __launch_bounds__(64)
+__global__ __launch_bounds__(64 * LF_WAVES)
 void filter_learned_kernel(const float *__restrict__ img, const uint32_t *__restrict__ idx,
                            const uint32_t *__restrict__ nsim, const uint32_t *__restrict__ base,
                            const uint32_t *__restrict__ gtile, StepConst sc, int g0, int Gc,
@@ -3194,69 +3213,229 @@ void filter_learned_kernel(const float *__restrict__ img, const uint32_t *__rest
                            uint8_t *__restrict__ early, float *__restrict__ gweight,
                            uint8_t *__restrict__ gflag, uint32_t *__restrict__ n_flag, int C, int c)
 {
-	// coefficients, then the bf16 feature rows (read by the network's first
-	// layer only), then gains (row stride 64), then the filtered rows (TR_ZS)
-	__shared__ __align__(16) float zs[FAST_NMAX * TR_ZS];
-	uint16_t *xb = reinterpret_cast<uint16_t *>(zs);
-	static_assert(32 * MLP_XS * 2 <= FAST_NMAX * TR_ZS * 4, "feature rows fit the coefficient buffer");
-	__shared__ __align__(16) uint16_t hb[32 * MLP_HS];
-	const int gl = blockIdx.x;
-	if (gl >= Gc) return;
-	const int g = g0 + gl;
-	const int lane = threadIdx.x;
-	const int N = (int)nsim[g];
-	const uint32_t row0 = base[gl];
-	const uint32_t *gidx = idx + (size_t)g * sc.npmax;
-	if (c == 0 && lane < N) etile[row0 + lane] = gtile[g];
-
-	__shared__ float rstat[FAST_NMAX];
-	float z[FAST_NMAX];
-	learned_coeffs<PX>(img, gidx, N, sc, bsp, sigma, zs, z, rstat);
-	learned_features_lds(z, N, sigma, rstat, xb);
-	__syncthreads();
-	mlp_rows32(net, xb, hb, zs, FAST_P);
-	float s2 = 0.f, s1 = 0.f;
+	__shared__ __align__(16) LearnedTables tab;
+	__shared__ __align__(16) float xs[LF_WAVES][32 * LF_XS];
+	lf_stage(net.w1t, MLP_K1, 4, LF_S1, tab.w1);
+	lf_stage(net.w2t, MLP_H, 4, 8, tab.w2);
+	lf_stage(net.w3t, MLP_H, 2, 8, tab.w3);
 #pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) {
-		if (n < N) {
-			const float gn = zs[n * FAST_P + lane];
-			z[n] = z[n] * gn;
-			s1 += gn;
-			s2 += gn * gn;
+	for (int q = 0; q < 2; q++) {
+		lf_stage(bsp + q * FAST_P * FAST_P, FAST_P, 2, 4, tab.fwd[q]);
+		lf_stage(bsp + (2 + q) * FAST_P * FAST_P, FAST_P, 2, 4, tab.inv[q]);
+	}
+	for (int i = threadIdx.x; i < MLP_H; i += 64 * LF_WAVES) {
+		tab.b1[i] = net.b1[i];
+		tab.b2[i] = net.b2[i];
+		if (i < MLP_OUT) tab.b3[i] = net.b3[i];
+		if (i < FAST_P) {
+			double v = 0.0;
+			for (int p = 0; p < FAST_P; p++) {
+				_Float16 q[2];
+				__builtin_memcpy(&q[0], bsp + i * FAST_P + p, 2);
+				__builtin_memcpy(&q[1], bsp + (FAST_P + i) * FAST_P + p, 2);
+				v += (double)q[0] + (double)q[1];
+			}
+			tab.one[i] = (float)v;
 		}
 	}
-#pragma unroll
-	for (int o = 32; o > 0; o >>= 1) {
-		s1 += __shfl_xor(s1, o, 64);
-		s2 += __shfl_xor(s2, o, 64);
-	}
-	haar_lane(z, N, false);
 	__syncthreads();
-	// filtered rows for the inverse (rows n >= N are zero)
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int h = lane >> 5, j = lane & 31;
+	float *zs = xs[wave];
+	const int off = PX == 4 ? (lane >> 4) * sc.WH + ((lane >> 2) & 3) * sc.W + (lane & 3) : (lane >> 3) * sc.W + (lane & 7);
+	const float is = 1.f / sigma, ls = logf(sigma / 20.f), wv = win[lane];
+	// element r of tile t of a product over the outputs, started from a bias
+	auto bias = [&](const float *__restrict__ b, int t) {
+		mlp_f32x16 a;
 #pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) zs[n * TR_ZS + lane] = z[n];
-	const float cnt = (float)(64 * N);
-	const float gvar = s2 / cnt - (s1 / cnt) * (s1 / cnt);
-	// one weight for all channels of a group, as the reference aggregates
-	// colour groups (nldct.cpp:2293-2299), here from the first channel's
-	// gains; a group is flagged when any channel's gain variance exceeds the
-	// threshold
-	const float w = c == 0 ? (float)(1. / ((double)sigma * sigma) / (double)s2) : gweight[g];
-	const uint8_t f = gvar > gvar_thr ? 1 : 0;
-	if (lane == 0) {
-		if (c == 0) {
-			gweight[g] = w;
-			early[g] = 0;
-			gflag[g] = f;
-			if (f) atomicAdd(n_flag, 1u);
-		} else if (f && !gflag[g]) {
-			gflag[g] = 1;
-			atomicAdd(n_flag, 1u);
+		for (int q = 0; q < 4; q++) {
+			const float4 v = *reinterpret_cast<const float4 *>(b + 32 * t + 8 * q + 4 * h);
+			a[4 * q] = v.x;
+			a[4 * q + 1] = v.y;
+			a[4 * q + 2] = v.z;
+			a[4 * q + 3] = v.w;
 		}
+		return a;
+	};
+	auto layer = [&](const uint4 *__restrict__ w, const lf_bf16x8 *x, int steps, int t, mlp_f32x16 a) {
+#pragma unroll
+		for (int s = 0; s < steps; s++)
+			a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(lf_bf16x8, w[(t * steps + s) * 64 + lane]), x[s], a,
+			                                            0, 0, 0);
+		return a;
+	};
+	auto relu = [](const mlp_f32x16 &a, lf_bf16x8 *x) {   // NaN gives 0
+#pragma unroll
+		for (int r = 0; r < 16; r++) x[r >> 3][r & 7] = (__bf16)__builtin_amdgcn_fmed3f(a[r], 0.f, INFINITY);
+	};
+	for (int gl = blockIdx.x * LF_WAVES + wave; gl < Gc; gl += gridDim.x * LF_WAVES) {
+		const int g = g0 + gl;
+		const int N = (int)nsim[g];
+		const uint32_t row0 = base[gl];
+		const uint32_t *gidx = idx + (size_t)g * sc.npmax;
+		if (c == 0 && lane < N) etile[row0 + lane] = gtile[g];
+		float y[FAST_NMAX], z[32];
+		{
+			const uint32_t my_idx = lane < N ? gidx[lane] : 0u;
+#pragma unroll
+			for (int n = 0; n < FAST_NMAX; n++) {
+				const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)my_idx, n);
+				y[n] = n < N ? img[(size_t)r + off] : 0.f;
+			}
+		}
+		// the first patch's mean is taken off before the transforms and put back
+		// after them, so that their roundings are of the patches' differences:
+		// mean0 1 (lane j = 0) is what it has in the group's coefficients
+		float mean = y[0];
+#pragma unroll
+		for (int o = 32; o > 0; o >>= 1) mean += __shfl_xor(mean, o, 64);
+		mean *= 1.f / 64.f;
+#pragma unroll
+		for (int n = 0; n < FAST_NMAX; n++) y[n] = n < N ? y[n] - mean : 0.f;
+		float mean0 = mean;
+		for (int n = 2; n <= N; n *= 2) mean0 *= 2.f * 0.70710678118654752440f;
+		mean0 = j == 0 ? mean0 : 0.f;
+		haar_lane(y, N, true);
+		// to lane (h, j): samples 0 .. 31, then 32 .. 63
+#pragma unroll
+		for (int p = 0; p < 2; p++) {
+			if (h == p) {
+#pragma unroll
+				for (int n = 0; n < FAST_NMAX; n += 4)
+					*reinterpret_cast<float4 *>(zs + j * LF_XS + n) = make_float4(y[n], y[n + 1], y[n + 2], y[n + 3]);
+			}
+			wave_sync();
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+#pragma unroll
+				for (int i = 0; i < 4; i++) z[16 * p + 4 * q + i] = zs[(8 * q + 4 * h + i) * LF_XS + j];
+			wave_sync();
+		}
+		lf_f16x8 vh[4], vl[4];
+		int sh;
+		{
+			float m = 0.f;
+#pragma unroll
+			for (int k = 0; k < 32; k++) m = fmaxf(m, fabsf(z[k]));
+			lf_scale(m, sh);
+			lf_split(z, sh, vh, vl);
+		}
+#pragma unroll
+		for (int t = 0; t < 2; t++) {
+			mlp_f32x16 a = {};
+#pragma unroll
+			for (int s = 0; s < 4; s++) {
+				const lf_f16x8 bh = __builtin_bit_cast(lf_f16x8, tab.fwd[0][(t * 4 + s) * 64 + lane]);
+				const lf_f16x8 bl = __builtin_bit_cast(lf_f16x8, tab.fwd[1][(t * 4 + s) * 64 + lane]);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, vh[s], a, 0, 0, 0);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl, vh[s], a, 0, 0, 0);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, vl[s], a, 0, 0, 0);
+			}
+#pragma unroll
+			for (int r = 0; r < 16; r++) z[16 * t + r] = ldexpf(a[r], -sh);
+			const mlp_f32x16 b = bias(tab.one, t);
+#pragma unroll
+			for (int r = 0; r < 16; r++) z[16 * t + r] = __builtin_fmaf(mean0, b[r], z[16 * t + r]);
+		}
+		// features: z / sigma, log(sigma / 20), log1p of the row's energy
+		lf_bf16x8 x0[8], x1[8];
+		{
+			float e = 0.f;
+#pragma unroll
+			for (int k = 0; k < 32; k++) {
+				e += z[k] * z[k];
+				x0[k >> 3][k & 7] = (__bf16)(z[k] * is);
+			}
+			e += __shfl_xor(e, 32, 64);
+			const float rs = j < N ? log1pf(e / (64.f * sigma * sigma)) : 0.f;
+			lf_bf16x8 f = {};
+			f[0] = (__bf16)(h == 0 && j < N ? ls : 0.f);
+			f[1] = (__bf16)(h == 0 ? rs : 0.f);
+			x0[4] = f;
+		}
+#pragma unroll
+		for (int t = 0; t < 4; t++) relu(layer(tab.w1, x0, LF_S1, t, bias(tab.b1, t)), x1 + 2 * t);
+#pragma unroll
+		for (int t = 0; t < 4; t++) relu(layer(tab.w2, x1, 8, t, bias(tab.b2, t)), x0 + 2 * t);
+		float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+		for (int t = 0; t < 2; t++) {
+			const mlp_f32x16 a = layer(tab.w3, x0, 8, t, bias(tab.b3, t));
+#pragma unroll
+			for (int r = 0; r < 16; r++) {
+				const float gn = 1.f / (1.f + expf(-a[r]));
+				z[16 * t + r] = j < N ? z[16 * t + r] * gn : 0.f;
+				s1 += j < N ? gn : 0.f;
+				s2 += j < N ? gn * gn : 0.f;
+			}
+		}
+#pragma unroll
+		for (int o = 32; o > 0; o >>= 1) {
+			s1 += __shfl_xor(s1, o, 64);
+			s2 += __shfl_xor(s2, o, 64);
+		}
+		const float cnt = (float)(64 * N);
+		const float gvar = s2 / cnt - (s1 / cnt) * (s1 / cnt);
+		// one weight for all channels of a group, as the reference aggregates
+		// colour groups (nldct.cpp:2293-2299), here from the first channel's
+		// gains; a group is flagged when any channel's gain variance exceeds the
+		// threshold
+		const float w = c == 0 ? (float)(1. / ((double)sigma * sigma) / (double)s2) : gweight[g];
+		const uint8_t f = gvar > gvar_thr ? 1 : 0;
+		if (lane == 0) {
+			if (c == 0) {
+				gweight[g] = w;
+				early[g] = 0;
+				gflag[g] = f;
+				if (f) atomicAdd(n_flag, 1u);
+			} else if (f && !gflag[g]) {
+				gflag[g] = 1;
+				atomicAdd(n_flag, 1u);
+			}
+		}
+		if (c == 0 && lane < N) entry_w[row0 + lane] = w;
+#pragma unroll
+		for (int t = 0; t < 2; t++) {
+			const mlp_f32x16 b = bias(tab.one, t);
+#pragma unroll
+			for (int r = 0; r < 16; r++) z[16 * t + r] = __builtin_fmaf(-mean0, b[r], z[16 * t + r]);
+		}
+		{
+			float m = 0.f;
+#pragma unroll
+			for (int k = 0; k < 32; k++) m = fmaxf(m, fabsf(z[k]));
+			lf_scale(m, sh);
+			lf_split(z, sh, vh, vl);
+		}
+		mlp_f32x16 d[2];
+#pragma unroll
+		for (int t = 0; t < 2; t++) {
+			mlp_f32x16 a = {};
+#pragma unroll
+			for (int s = 0; s < 4; s++) {
+				const lf_f16x8 bh = __builtin_bit_cast(lf_f16x8, tab.inv[0][(t * 4 + s) * 64 + lane]);
+				const lf_f16x8 bl = __builtin_bit_cast(lf_f16x8, tab.inv[1][(t * 4 + s) * 64 + lane]);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], bh, a, 0, 0, 0);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], bl, a, 0, 0, 0);
+				a = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[s], bh, a, 0, 0, 0);
+			}
+			d[t] = a;
+		}
+		// to lane = sample: the halves hold rows 8 q + 4 h + i of both tiles
+#pragma unroll
+		for (int r = 0; r < 16; r++) {
+			const auto o = __builtin_amdgcn_permlane32_swap(__float_as_uint(d[0][r]), __float_as_uint(d[1][r]), false, false);
+			const int n = 8 * (r >> 2) + (r & 3);
+			y[n] = ldexpf(__uint_as_float(o[0]), -sh);
+			y[n + 4] = ldexpf(__uint_as_float(o[1]), -sh);
+		}
+		haar_lane(y, N, false);
+		float *e0 = est + (size_t)row0 * (C * FAST_P) + c * FAST_P + lane;
+		const float ww = w * wv;
+#pragma unroll
+		for (int n = 0; n < FAST_NMAX; n++)
+			if (n < N) e0[(size_t)n * (C * FAST_P)] = ww * (y[n] + mean);
 	}
-	if (c == 0 && lane < N) entry_w[row0 + lane] = w;
-	__syncthreads();
-	mfma_inverse(zs, bsp, N, w, win, row0, est, C * FAST_P, c * FAST_P);
 }
 
 // Split tables of the matrix-core transforms from the fp32 bases
