@@ -60,7 +60,7 @@ __global__ void filter2_kernel(const float *, const float *, const uint32_t *, c
 	const uint32_t *, const uint32_t *, StepConst, int, int, const float *, const float *, \
 	const float *, float *, float *, uint32_t *, uint8_t *, float *, uint32_t *, int, int, int64_t, float *, \
 	const float *, const float *
-template <int PX> __global__ void filter1_fast_kernel(FILTER1_ARGS);
+template <int PX, int NMAX, bool TAB> __global__ void filter1_fast_kernel(FILTER1_ARGS);
 template <int PX> __global__ void coef_kernel(const float *, int, int, int, const float *, float *);
 template <int PX, int NMAX, bool TAB> __global__ void filter2_fast_kernel(FILTER2_ARGS);
 #define FILTER2W_ARGS const float *, const float *, const uint32_t *, const uint32_t *, \
@@ -1289,6 +1289,18 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 	}
 }
 
+using Filter1 = void (*)(FILTER1_ARGS);
+template <int PX, bool TAB> Filter1 filter1_rows(int np)
+{
+	return np < 16 ? filter1_fast_kernel<PX, 8, TAB> : np < 32 ? filter1_fast_kernel<PX, 16, TAB>
+	                                                            : filter1_fast_kernel<PX, 32, TAB>;
+}
+// The step-1 filter for a patch shape and the rows its groups can have.
+Filter1 filter1_of(const StepConst &sc, bool tab)
+{
+	if (sc.sPx == 4) return tab ? filter1_rows<4, true>(sc.npmax) : filter1_rows<4, false>(sc.npmax);
+	return tab ? filter1_rows<8, true>(sc.npmax) : filter1_rows<8, false>(sc.npmax);
+}
 using Filter2 = void (*)(FILTER2_ARGS);
 template <int PX> Filter2 filter2_rows_no_table(int np)
 {
@@ -1434,12 +1446,15 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 				                   dim3((unsigned)std::min(nblk(Gc, 8), 256)), dim3(512), 0, ctx->stream, d_nplanes + (size_t)c * WHF, d_idx, d_nsim, d_base,
 				                   dv.gtile, sc, g0, Gc, dv.bsp, dv.win, la->net, la->sigma,
 				                   la->gvar_thr, d_est, d_ew, d_etile, d_early, d_gw, d_gflag, la->nflag, C, c);
-		else if (pl.fast && step1)
+		else if (pl.fast && step1) {
+			// blocks loop, as those of the step-2 filter
+			const auto kern = filter1_of(sc, d_coef_n != nullptr);
+			const unsigned blocks = (unsigned)std::min(nblk(Gc, 4), d_coef_n ? 25600 : 2048);
 			for (int c = 0; c < C; c++)   // channel planes; the last launch weights all
-				hipLaunchKernelGGL(sc.sPx == 4 ? filter1_fast_kernel<4> : filter1_fast_kernel<8>, dim3(Gc),
-				                   dim3(64), 0, ctx->stream, d_nplanes, d_idx, d_nsim, d_base, dv.gtile, sc, g0,
-				                   Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile, d_early, d_gw, d_cnt, C, c,
-				                   (int64_t)WHF, d_gacc, d_coef_n);
+				hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, ctx->stream, d_nplanes, d_idx, d_nsim, d_base,
+				                   dv.gtile, sc, g0, Gc, dv.basis, dv.binv, dv.win, d_est, d_ew, d_etile, d_early,
+				                   d_gw, d_cnt, C, c, (int64_t)WHF, d_gacc, d_coef_n);
+		}
 		else if (pl.wide && pl.fast) {
 			const auto kern = np < 32 ? filter2_wide_kernel<16> : filter2_wide_kernel<32>;
 			for (int c = 0; c < C; c++)

@@ -2143,8 +2143,8 @@ template <int NMAX> __device__ __forceinline__ void haar_lane(float (&z)[NMAX], 
 // ---------------------------------------------------------------------------
 // Dense patch transforms on the fp32 matrix instructions.  v_mfma_f32_32x32x2
 // and _16x16x4 add their products to the accumulator one term after another,
-// each as one fused multiply-add: bit for bit the sequential sums of
-// fast_forward, at twice the vector unit's rate and beside its work.
+// each as one fused multiply-add: bit for bit a sequential sum, at twice the
+// vector unit's rate and beside its work.
 // Operands of the instruction that takes terms 2 s, 2 s + 1 (ROWS = 32; lane
 // l: h = l / 32, j = l % 32) or 4 s .. 4 s + 3 (ROWS = 16; h = l / 16, j =
 // l % 16): A[row j][term TS s + h], B[term TS s + h][column j].
@@ -2174,6 +2174,7 @@ template <> struct MmTile<16> {
 	static __device__ __forceinline__ int row(int r, int h) { return 4 * h + r; }
 };
 constexpr int MM_ZS = 68;   // LDS row stride of an A operand
+constexpr int MM_HS = 36;   // the same for half the terms
 
 // The P x P matrix m[term * ts + column * cs] as B operands in LDS: float4 q
 // of lane l and column tile t holds the operands of instructions 4 q .. 4 q + 3.
@@ -2214,9 +2215,9 @@ __device__ __forceinline__ void mm_load_a(const float *__restrict__ zs, float4 (
 
 // Column tile t of the product A B, terms in order (those from P on are zeros
 // and left out).
-template <int ROWS, int P>
+template <int ROWS, int P, bool SPARSE = false>
 __device__ __forceinline__ typename MmTile<ROWS>::Acc mm_product(const float4 (&a)[FAST_P / 4 / MmTile<ROWS>::TS],
-                                                                 const float4 *__restrict__ bf, int t)
+                                                                 const float4 *__restrict__ bf, int t, uint64_t kmask = 0)
 {
 	using T = MmTile<ROWS>;
 	constexpr int Q = FAST_P / 4 / T::TS;
@@ -2224,6 +2225,7 @@ __device__ __forceinline__ typename MmTile<ROWS>::Acc mm_product(const float4 (&
 	typename T::Acc c = {};
 #pragma unroll
 	for (int q = 0; q < Q; q++) {
+		if (SPARSE && !((kmask >> (4 * T::TS * q)) & ((1ull << (4 * T::TS)) - 1))) continue;
 		const float4 b = bf[(t * Q + q) * 64 + l];
 		if (T::TS * (4 * q) < P) c = T::mac(a[q].x, b.x, c);
 		if (T::TS * (4 * q + 1) < P) c = T::mac(a[q].y, b.y, c);
@@ -2289,168 +2291,10 @@ __device__ __forceinline__ int wave_sum_int(int v)
 	return v;
 }
 
-// Forward transform of the N patches at anchors gidx[0..N) of `img`
-// (one channel, anchor address = position) into zs[n*64 + lane].
-// PAIRS: two patches per round (two independent sums in flight) or one.
-template <int PX, bool PAIRS = true>
-__device__ __forceinline__ void fast_forward(const float *__restrict__ img, const uint32_t *__restrict__ gidx,
-                                             int N, int W, int WH, const float (&brow)[FAST_P],
-                                             float *__restrict__ zs)
-{
-	constexpr int PT = FAST_P / (PX * PX);
-	int n = 0;
-	for (; PAIRS && n + 1 < N; n += 2) {
-		const float *src0 = img + gidx[n], *src1 = img + gidx[n + 1];
-		float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-		for (int ht = 0; ht < PT; ht++)
-#pragma unroll
-			for (int hy = 0; hy < PX; hy++) {
-				const float *r0 = src0 + ht * WH + hy * W, *r1 = src1 + ht * WH + hy * W;
-#pragma unroll
-				for (int hx = 0; hx < PX; hx++) {
-					const float b = brow[(ht * PX + hy) * PX + hx];
-					acc0 = __builtin_fmaf(r0[hx], b, acc0);
-					acc1 = __builtin_fmaf(r1[hx], b, acc1);
-				}
-			}
-		zs[n * FAST_P + threadIdx.x] = acc0;
-		zs[(n + 1) * FAST_P + threadIdx.x] = acc1;
-	}
-	for (; n < N; n++) {
-		const float *src = img + gidx[n];
-		float acc = 0.f;
-#pragma unroll
-		for (int ht = 0; ht < PT; ht++)
-#pragma unroll
-			for (int hy = 0; hy < PX; hy++) {
-				const float *r = src + ht * WH + hy * W;
-#pragma unroll
-				for (int hx = 0; hx < PX; hx++) acc = __builtin_fmaf(r[hx], brow[(ht * PX + hy) * PX + hx], acc);
-			}
-		zs[n * FAST_P + threadIdx.x] = acc;
-	}
-}
-
-// Inverse transform of the coefficients zs[n*64 + k] and the weighted est
-// rows: est[(row0+n)*rs + ro + pix] = (w*win[pix]) * sum_k z[k][n] Bi[k][pix]
-// (rs = floats per est row, ro = offset of this channel in the row).
-template <bool PAIRS = true>
-__device__ __forceinline__ void fast_inverse(const float *__restrict__ zs, const float *__restrict__ binv,
-                                             int N, float ww, uint32_t row0, float *__restrict__ est,
-                                             int rs = FAST_P, int ro = 0)
-{
-	float bcol[FAST_P];
-#pragma unroll
-	for (int k = 0; k < FAST_P; k++) bcol[k] = binv[k * FAST_P + threadIdx.x];
-	int n = 0;
-	for (; PAIRS && n + 1 < N; n += 2) {
-		const float4 *zr0 = reinterpret_cast<const float4 *>(zs + n * FAST_P);
-		const float4 *zr1 = reinterpret_cast<const float4 *>(zs + (n + 1) * FAST_P);
-		float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-		for (int q = 0; q < FAST_P / 4; q++) {
-			const float4 z0 = zr0[q], z1 = zr1[q];
-			acc0 = __builtin_fmaf(z0.x, bcol[4 * q + 0], acc0);
-			acc1 = __builtin_fmaf(z1.x, bcol[4 * q + 0], acc1);
-			acc0 = __builtin_fmaf(z0.y, bcol[4 * q + 1], acc0);
-			acc1 = __builtin_fmaf(z1.y, bcol[4 * q + 1], acc1);
-			acc0 = __builtin_fmaf(z0.z, bcol[4 * q + 2], acc0);
-			acc1 = __builtin_fmaf(z1.z, bcol[4 * q + 2], acc1);
-			acc0 = __builtin_fmaf(z0.w, bcol[4 * q + 3], acc0);
-			acc1 = __builtin_fmaf(z1.w, bcol[4 * q + 3], acc1);
-		}
-		est[(size_t)(row0 + n) * rs + ro + threadIdx.x] = ww * acc0;
-		est[(size_t)(row0 + n + 1) * rs + ro + threadIdx.x] = ww * acc1;
-	}
-	for (; n < N; n++) {
-		const float4 *zr = reinterpret_cast<const float4 *>(zs + n * FAST_P);
-		float acc = 0.f;
-#pragma unroll
-		for (int q = 0; q < FAST_P / 4; q++) {
-			const float4 z = zr[q];
-			acc = __builtin_fmaf(z.x, bcol[4 * q + 0], acc);
-			acc = __builtin_fmaf(z.y, bcol[4 * q + 1], acc);
-			acc = __builtin_fmaf(z.z, bcol[4 * q + 2], acc);
-			acc = __builtin_fmaf(z.w, bcol[4 * q + 3], acc);
-		}
-		est[(size_t)(row0 + n) * rs + ro + threadIdx.x] = ww * acc;
-	}
-}
-
-// The inverse over the columns k set in kmask only, for groups whose other
-// columns are zero in every row (step 1 after the hard threshold): a
-// skipped term is fma(+0, Bi, acc) = acc bit for bit for every acc but -0,
-// and a sum that starts at +0 reaches -0 only by an underflow below 2^-149,
-// which sums of image data times basis entries do not come near, so the
-// result equals fast_inverse's.  Lane k holds z[0..N) of column k on entry
-// (registers); the compacted rows are written over zs.
-__device__ __forceinline__ void fast_inverse_sparse(const float (&z)[FAST_NMAX], float *__restrict__ zs,
-                                                    const float *__restrict__ binv, int N, float ww,
-                                                    uint32_t row0, float *__restrict__ est, uint64_t kmask,
-                                                    int rs = FAST_P, int ro = 0)
-{
-	const int lane = threadIdx.x;
-	const int kc = __popcll(kmask);
-	// compacted column index of this lane's column
-	if ((kmask >> lane) & 1ull) {
-		const int j = __popcll(kmask & ((1ull << lane) - 1ull));
-#pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) if (n < N) zs[n * FAST_P + j] = z[n];
-	}
-	// inverse basis rows of the kept columns, in column order
-	float bsel[FAST_P];
-	uint64_t m = kmask;
-#pragma unroll
-	for (int j = 0; j < FAST_P; j++) {
-		bsel[j] = 0.f;
-		if (j < kc) {
-			const int k = __ffsll((unsigned long long)m) - 1;
-			m &= m - 1ull;
-			bsel[j] = binv[k * FAST_P + lane];
-		}
-	}
-	__syncthreads();
-	int n = 0;
-	for (; n + 1 < N; n += 2) {
-		const float *z0 = zs + n * FAST_P, *z1 = zs + (n + 1) * FAST_P;
-		float acc0 = 0.f, acc1 = 0.f;
-#pragma unroll
-		for (int j = 0; j < FAST_P; j += 4) {
-			if (j < kc) {
-				const float4 a = *reinterpret_cast<const float4 *>(z0 + j);
-				const float4 b = *reinterpret_cast<const float4 *>(z1 + j);
-				acc0 = __builtin_fmaf(a.x, bsel[j], acc0);
-				acc1 = __builtin_fmaf(b.x, bsel[j], acc1);
-				if (j + 1 < kc) { acc0 = __builtin_fmaf(a.y, bsel[j + 1], acc0); acc1 = __builtin_fmaf(b.y, bsel[j + 1], acc1); }
-				if (j + 2 < kc) { acc0 = __builtin_fmaf(a.z, bsel[j + 2], acc0); acc1 = __builtin_fmaf(b.z, bsel[j + 2], acc1); }
-				if (j + 3 < kc) { acc0 = __builtin_fmaf(a.w, bsel[j + 3], acc0); acc1 = __builtin_fmaf(b.w, bsel[j + 3], acc1); }
-			}
-		}
-		est[(size_t)(row0 + n) * rs + ro + lane] = ww * acc0;
-		est[(size_t)(row0 + n + 1) * rs + ro + lane] = ww * acc1;
-	}
-	for (; n < N; n++) {
-		const float *z0 = zs + n * FAST_P;
-		float acc = 0.f;
-#pragma unroll
-		for (int j = 0; j < FAST_P; j += 4) {
-			if (j < kc) {
-				const float4 a = *reinterpret_cast<const float4 *>(z0 + j);
-				acc = __builtin_fmaf(a.x, bsel[j], acc);
-				if (j + 1 < kc) acc = __builtin_fmaf(a.y, bsel[j + 1], acc);
-				if (j + 2 < kc) acc = __builtin_fmaf(a.z, bsel[j + 2], acc);
-				if (j + 3 < kc) acc = __builtin_fmaf(a.w, bsel[j + 3], acc);
-			}
-		}
-		est[(size_t)(row0 + n) * rs + ro + lane] = ww * acc;
-	}
-}
-
 // Forward transform of every patch anchor of a one-channel plane, once:
-// coef[pos*64 + k] = sum_p B[k][p] x[pos + off(p)] in the order of
-// fast_forward (the same dot product whatever group the patch is in, so the
-// filters' rows read it bit for bit).  One wave per run of anchors along x,
+// coef[pos*64 + k] = sum_p B[k][p] x[pos + off(p)] in the order of p (the same
+// dot product whatever group the patch is in, so the filters' rows read it bit
+// for bit).  One wave per run of anchors along x,
 // lane = coefficient, basis row in registers, four anchors per round (their
 // patches overlap: one load of a row segment serves all four).
 template <int PX>
@@ -2600,78 +2444,6 @@ __device__ __forceinline__ void fast_scale_channels(int N, int C, float ww, uint
 		}
 }
 
-template <int PX>
-__global__ __launch_bounds__(64)
-void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restrict__ idx,
-                         const uint32_t *__restrict__ nsim, const uint32_t *__restrict__ base,
-                         const uint32_t *__restrict__ gtile, StepConst sc, int g0, int Gc,
-                         const float *__restrict__ basis, const float *__restrict__ binv,
-                         const float *__restrict__ win, float *__restrict__ est,
-                         float *__restrict__ entry_w, uint32_t *__restrict__ etile,
-                         uint8_t *__restrict__ early, float *__restrict__ gweight,
-                         uint32_t *__restrict__ n_early, int C, int c, int64_t cstride,
-                         float *__restrict__ gacc, const float *__restrict__ coef)
-{
-	__shared__ __align__(16) float zs[FAST_NMAX * FAST_P];
-	const int gl = blockIdx.x;
-	if (gl >= Gc) return;
-	const int g = g0 + gl;
-	const int lane = threadIdx.x;
-	const int N = (int)nsim[g];
-	const uint32_t row0 = base[gl];
-	const uint32_t *gidx = idx + (size_t)g * sc.npmax;
-	float z[FAST_NMAX];
-	if (coef) fast_rows<FAST_P, true>(coef + c * cstride * FAST_P, gidx, N, z);
-	if (c == 0) {
-		if (lane < N) etile[row0 + lane] = gtile[g];
-		if ((!coef || fast_rows_equal(z, N)) &&
-		    fast_early_out<PX>(img, gidx, N, sc.W, sc.WH, C, cstride, g, row0, est, early, gweight, n_early))
-			return;
-	} else if (early[g])
-		return;
-
-	if (!coef) {
-		{
-			float brow[FAST_P];
-#pragma unroll
-			for (int p = 0; p < FAST_P; p++) brow[p] = basis[lane * FAST_P + p];
-			fast_forward<PX>(img + c * cstride, gidx, N, sc.W, sc.WH, brow, zs);
-		}
-		__syncthreads();
-#pragma unroll
-		for (int n = 0; n < FAST_NMAX; n++) z[n] = n < N ? zs[n * FAST_P + lane] : 0.f;
-	}
-	haar_lane(z, N, true);
-	// rows n >= N are +0: 0 > (beta sigma)^2 fails, so they count nothing
-	// and stay +0 without a guard
-	int cnt = 0;
-#pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) {
-		if (z[n] * z[n] > sc.beta_sigma2 || (lane == 0 && n == 0)) cnt++;
-		else z[n] = 0.f;
-	}
-	haar_lane(z, N, false);
-	// columns with a coefficient left in any row (the others are +0 throughout)
-	bool nzc = false;
-#pragma unroll
-	for (int n = 0; n < FAST_NMAX; n++) nzc |= z[n] != 0.f;
-	const uint64_t kmask = __ballot(nzc);
-	const int nnz_i = wave_sum_int(cnt) + (c ? (int)gacc[g] : 0);
-	const float nnz = (float)nnz_i;
-	const float w = 1 / sc.sigma2 / nnz;
-	const bool last = c == C - 1;
-	if (lane == 0) {
-		if (!last) gacc[g] = (float)nnz_i;
-		else gweight[g] = w;
-		early[g] = 0;
-	}
-	if (last && lane < N) entry_w[row0 + lane] = w;
-	// launches before the last store unweighted rows
-	const float ww = last ? w * win[lane] : 1.f;
-	fast_inverse_sparse(z, zs, binv, N, ww, row0, est, kmask, C * FAST_P, c * FAST_P);
-	if (last && C > 1) fast_scale_channels<FAST_P>(N, C, w * win[lane], row0, est);
-}
-
 // Orders a wave's LDS writes before its lanes' later reads (LDS accesses of a
 // wave execute in order: this only holds the compiler).
 __device__ __forceinline__ void wave_sync()
@@ -2712,24 +2484,46 @@ __device__ __forceinline__ void mm_forward(const float *__restrict__ img, const 
 // Inverse transform of the coefficients z[n] (lane = coefficient) and the
 // weighted est rows: est[(row0 + n) rs + ro + p] = (w win[p]) * sample p of
 // patch n.  One wave; zs: ROWS rows of MM_ZS floats.
-template <int P, int NMAX, int ROWS>
+// SPARSE: the coefficients outside kmask are +0 in every row, and the four
+// instructions whose terms all are are left out.  A term left out is
+// fma(+0, b, acc) = acc bit for bit for every acc but -0, and a sum that
+// starts at +0 reaches -0 only by an underflow below 2^-149, which sums of
+// image data times basis entries do not come near.
+template <int P, int NMAX, int ROWS, bool SPARSE = false>
 __device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__restrict__ zs,
                                            const float4 *__restrict__ bf, int N, float w,
                                            const float *__restrict__ win, uint32_t row0, float *__restrict__ est,
-                                           int rs, int ro)
+                                           int rs, int ro, uint64_t kmask = 0)
 {
 	using T = MmTile<ROWS>;
 	const int l = threadIdx.x & 63, h = l / ROWS, j = l % ROWS;
-	const int at = mm_pos<ROWS>(l);
-#pragma unroll
-	for (int n = 0; n < NMAX; n++) zs[n * MM_ZS + at] = z[n];
-	wave_sync();
 	float4 a[FAST_P / 4 / T::TS];
-	mm_load_a<ROWS>(zs, a);
+	if (SPARSE) {   // one half of the terms after the other through half the LDS
+		constexpr int U = FAST_P / 2 / T::TS;   // a lane's terms of a half
+		const int k = l & 31;
+#pragma unroll
+		for (int half = 0; half < 2; half++) {
+			if (l >> 5 == half) {
+#pragma unroll
+				for (int n = 0; n < NMAX; n++) zs[n * MM_HS + k % T::TS * U + k / T::TS] = z[n];
+			}
+			wave_sync();
+#pragma unroll
+			for (int q = 0; q < U / 4; q++)
+				a[half * (U / 4) + q] = *reinterpret_cast<const float4 *>(zs + j * MM_HS + h * U + 4 * q);
+			wave_sync();
+		}
+	} else {
+		const int at = mm_pos<ROWS>(l);
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) zs[n * MM_ZS + at] = z[n];
+		wave_sync();
+		mm_load_a<ROWS>(zs, a);
+	}
 	float *e0 = est + (size_t)row0 * rs + ro;
 #pragma unroll
 	for (int t = 0; t < FAST_P / ROWS; t++) {
-		const auto c = mm_product<ROWS, P>(a, bf, t);
+		const auto c = mm_product<ROWS, P, SPARSE>(a, bf, t, kmask);
 		const int col = ROWS * t + j;
 		if (P < FAST_P && col >= P) continue;
 		const float ww = win ? w * win[col] : 1.f;
@@ -2740,6 +2534,86 @@ __device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__rest
 		}
 	}
 	wave_sync();
+}
+
+// Step-1 filter: hard threshold, one wave per group (grid-stride), lane =
+// coefficient of every row.  NMAX: rows held (8, 16, 32).
+// Bound: the memory's latency, 4 GB of table rows and 8.2 GB of est per launch
+// at 960x540x20 with 16 waves a CU (the registers' limit, and why the
+// inverse's rows go through LDS in halves: whole rows leave 12 waves, 4.98
+// ms).  There the inverse over the kept columns by vector instructions took
+// two thirds of 2340 a group: 5.46 ms, now 4.75.  Asking for the next group's
+// rows before this one's stores spills: 10.5 ms.
+template <int PX, int NMAX, bool TAB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAB ? 4 : 2)))
+void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restrict__ idx,
+                         const uint32_t *__restrict__ nsim, const uint32_t *__restrict__ base,
+                         const uint32_t *__restrict__ gtile, StepConst sc, int g0, int Gc,
+                         const float *__restrict__ basis, const float *__restrict__ binv,
+                         const float *__restrict__ win, float *__restrict__ est,
+                         float *__restrict__ entry_w, uint32_t *__restrict__ etile,
+                         uint8_t *__restrict__ early, float *__restrict__ gweight,
+                         uint32_t *__restrict__ n_early, int C, int c, int64_t cstride,
+                         float *__restrict__ gacc, const float *__restrict__ coef)
+{
+	constexpr int P = FAST_P, ROWS = NMAX > 16 ? 32 : 16, NW = 4;
+	__shared__ __align__(16) float4 bf[FAST_P * FAST_P / 4];                // inverse basis
+	__shared__ __align__(16) float4 bfwd[TAB ? 1 : FAST_P * FAST_P / 4];    // basis
+	__shared__ __align__(16) float zsm[NW * ROWS * (TAB ? MM_HS : MM_ZS)];
+	mm_load_b<ROWS>(binv, P, 1, P, bf);
+	if (!TAB) mm_load_b<ROWS>(basis, 1, P, P, bfwd);
+	__syncthreads();
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	float *zs = zsm + wave * ROWS * (TAB ? MM_HS : MM_ZS);
+	for (int gl = blockIdx.x * NW + wave; gl < Gc; gl += gridDim.x * NW) {
+		const int g = g0 + gl;
+		const int N = (int)nsim[g];
+		const uint32_t row0 = base[gl];
+		const uint32_t *gidx = idx + (size_t)g * sc.npmax;
+		float z[NMAX];
+		if (TAB) fast_rows<P, true>(coef + c * cstride * FAST_P, gidx, N, z);
+		if (c == 0) {
+			if (lane < N) etile[row0 + lane] = gtile[g];
+			if ((!TAB || fast_rows_equal(z, N)) &&
+			    fast_early_out<PX>(img, gidx, N, sc.W, sc.WH, C, cstride, g, row0, est, early, gweight, n_early))
+				continue;
+		} else if (early[g])
+			continue;
+		if (!TAB) {
+			if (N > 0) mm_forward<PX, ROWS>(img + c * cstride, gidx, N, sc.W, sc.WH, bfwd, zs);
+			wave_sync();
+#pragma unroll
+			for (int n = 0; n < NMAX; n++) z[n] = n < N ? zs[n * MM_ZS + lane] : 0.f;
+			wave_sync();
+		}
+		haar_lane(z, N, true);
+		// rows n >= N are +0: 0 > (beta sigma)^2 fails, so they count nothing
+		// and stay +0 without a guard
+		int cnt = 0;
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) {
+			if (z[n] * z[n] > sc.beta_sigma2 || (lane == 0 && n == 0)) cnt++;
+			else z[n] = 0.f;
+		}
+		haar_lane(z, N, false);
+		// columns with a coefficient left in any row (the others are +0 throughout)
+		bool nzc = false;
+#pragma unroll
+		for (int n = 0; n < NMAX; n++) nzc |= z[n] != 0.f;
+		const uint64_t kmask = __ballot(nzc);
+		const int nnz_i = wave_sum_int(cnt) + (c ? (int)gacc[g] : 0);
+		const float w = 1 / sc.sigma2 / (float)nnz_i;
+		const bool last = c == C - 1;
+		if (lane == 0) {
+			if (!last) gacc[g] = (float)nnz_i;
+			else gweight[g] = w;
+			early[g] = 0;
+		}
+		if (last && lane < N) entry_w[row0 + lane] = w;
+		// launches before the last store unweighted rows
+		mm_inverse<P, NMAX, ROWS, true>(z, zs, bf, N, w, last ? win : nullptr, row0, est, C * P, c * P, kmask);
+		if (last && C > 1) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
+	}
 }
 
 // Step-2 filter, one wave per group (grid-stride), lane = coefficient of
@@ -3555,8 +3429,15 @@ template __global__ void learned_pairs_kernel<8>(PAIRS_ARGS);
 	const uint32_t *, const uint32_t *, StepConst, int, int, const float *, const float *, \
 	const float *, float *, float *, uint32_t *, uint8_t *, float *, uint32_t *, int, int, int64_t, float *, \
 	const float *, const float *
-template __global__ void filter1_fast_kernel<4>(FILTER1_ARGS);
-template __global__ void filter1_fast_kernel<8>(FILTER1_ARGS);
+#define FILTER1_INST(PX, N)                                                                                \
+	template __global__ void filter1_fast_kernel<PX, N, true>(FILTER1_ARGS);                                \
+	template __global__ void filter1_fast_kernel<PX, N, false>(FILTER1_ARGS);
+FILTER1_INST(4, 8)
+FILTER1_INST(4, 16)
+FILTER1_INST(4, 32)
+FILTER1_INST(8, 8)
+FILTER1_INST(8, 16)
+FILTER1_INST(8, 32)
 #define FILTER2_INST(PX, N)                                                                                \
 	template __global__ void filter2_fast_kernel<PX, N, true>(FILTER2_ARGS);                                \
 	template __global__ void filter2_fast_kernel<PX, N, false>(FILTER2_ARGS);
