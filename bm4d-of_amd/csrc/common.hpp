@@ -32,6 +32,9 @@ struct StepConst {
 	// the first, matches kept per frame, distance bias dsub^2*255
 	int pred_w, pred_np;
 	float pred_dsub;
+	// channels at the head of an est row that hold samples without the row's
+	// weight, which the region fold then applies (0, or C - 1)
+	int est_raw;
 };
 
 // Pixel block of the ordered aggregation: RX x RY x RT pixels, frame blocks

@@ -97,7 +97,7 @@ __global__ void sort_runs_kernel(const uint32_t *, int64_t, uint32_t *);
 __global__ void add_rows_kernel(const uint32_t *, unsigned long long *);
 __global__ void early_fix_kernel(const uint8_t *, const uint32_t *, const float *, const uint32_t *,
                                  const uint32_t *, const uint32_t *, const uint32_t *, int, int, const float *,
-                                 int, int, float *, float *);
+                                 int, int, int, float *, float *);
 __global__ void filtered_index_kernel(const uint8_t *, int, uint32_t *);
 __global__ void first_moved_kernel(const uint32_t *, const uint32_t *, int, int, uint32_t *);
 __global__ void bm_pred_kernel(const float *, const float *, const float *, const uint32_t *, const uint32_t *,
@@ -486,6 +486,7 @@ StepConst make_const(const bm4dof_params &p, int W, int H, int F, int C, bool us
                      const Tiling &t)
 {
 	StepConst sc;
+	sc.est_raw = 0;   // set by chunk (enqueue_step)
 	sc.W = W; sc.H = H; sc.F = F; sc.C = C;
 	sc.WH = W * H;
 	sc.WHC = W * H * C;
@@ -1331,7 +1332,7 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
                   const LearnedArgs *la, int parts = 3)
 {
 	const bool step1 = pl.step1;
-	const StepConst &sc = pl.sc;
+	StepConst sc = pl.sc;
 	const int G = pl.G, np = pl.np, C = pl.C;
 	const size_t WHF = pl.WHF, N_all = pl.N_all;
 	auto mark = [&](const char *a, const char *b1, const char *b2) {
@@ -1405,6 +1406,11 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 	for (int g0 = 0; g0 < G; g0 += pl.chunk_groups) {
 		const int Gc = std::min(pl.chunk_groups, G - g0);
 		const int64_t Mub = (int64_t)Gc * np;
+		// the filters of one channel a launch leave the weight of all channels
+		// but the last to the region fold, which holds it: the last launch
+		// would read and write those rows again (641x361x9, 3 channels, 48
+		// patches: filters 3.5 and 9.4 ms so, 1.9 and 5.5 without; folds as before)
+		sc.est_raw = C > 1 && pl.fast && !la && agg_binned_ok(ctx, sc, Mub) ? C - 1 : 0;
 		// row offsets of the chunk's groups; base[Gc] = rows of the chunk
 		uint32_t *d_base = ctx->base.as<uint32_t>((size_t)Gc + 1);
 		dscan(ctx, 0, d_nsim + g0, Gc, (int64_t)Gc + 1, d_base);
@@ -1494,7 +1500,7 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 			                   gend, d_fidx);
 			dscan(ctx, 1, d_fidx, gend, gend, d_lastf);
 			hipLaunchKernelGGL(early_fix_kernel, dim3(nblk(Gc, 64)), dim3(64), 0, ctx->stream, d_early, d_nsim, d_gw,
-			                   d_lastf, dv.gtile, dv.tile_first, d_base, g0, Gc, dv.win, C, sc.P, d_est, d_ew);
+			                   d_lastf, dv.gtile, dv.tile_first, d_base, g0, Gc, dv.win, C, sc.P, sc.est_raw, d_est, d_ew);
 			HIPCHK(hipGetLastError());
 		}
 		mark("l_filter", "s1_filter", "s2_filter");

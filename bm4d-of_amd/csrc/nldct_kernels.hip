@@ -2432,8 +2432,9 @@ __device__ __forceinline__ bool fast_early_out(const float *__restrict__ img, co
 // channel planes cstride apart).  The group weight counts every channel
 // (nldct.cpp:1820-1936, 2038-2168), so gacc[g] carries the running count or
 // sum from launch to launch; launches before the last store the inverse
-// transform unweighted and the last one scales them by its weight: the same
-// products (w * window) * value as one pass over all channels.
+// transform unweighted.  Where the region fold reads the rows it scales them by
+// the group's weight (sc.est_raw); for the other folds the last launch does:
+// the same products (w * window) * value as one pass over all channels.
 template <int P>
 __device__ __forceinline__ void fast_scale_channels(int N, int C, float ww, uint32_t row0, float *__restrict__ est)
 {
@@ -2612,7 +2613,7 @@ void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restri
 		if (last && lane < N) entry_w[row0 + lane] = w;
 		// launches before the last store unweighted rows
 		mm_inverse<P, NMAX, ROWS, true>(z, zs, bf, N, w, last ? win : nullptr, row0, est, C * P, c * P, kmask);
-		if (last && C > 1) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
+		if (last && C > 1 && !sc.est_raw) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
 	}
 }
 
@@ -2702,7 +2703,7 @@ void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restric
 		if (last && lane < N) entry_w[row0 + lane] = w;
 		// launches before the last store unweighted rows
 		mm_inverse<P, NMAX, ROWS>(z, zs, bf, N, w, last ? win : nullptr, row0, est, C * P, c * P);
-		if (last && C > 1 && lane < P) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
+		if (last && C > 1 && !sc.est_raw && lane < P) fast_scale_channels<P>(N, C, w * win[lane], row0, est);
 	}
 }
 
@@ -2870,7 +2871,7 @@ void filter2_wide_kernel(const float *__restrict__ noisy, const float *__restric
 				if (n < N) e0[(size_t)n * (C * P) + col] = ww * (t ? a1 : a0)[r];
 			}
 		}
-		if (last && C > 1 && tid < P) {
+		if (last && C > 1 && !sc.est_raw && tid < P) {
 			const float ww = w * win[tid];
 			for (int n = 0; n < N; n++)
 				for (int cc = 0; cc < C - 1; cc++) est[((size_t)(row0 + n) * C + cc) * P + tid] *= ww;
@@ -4600,7 +4601,8 @@ void agg_region_fold_kernel(const uint32_t *__restrict__ boff, const uint32_t *_
 					Acc a = acc[o + soff[s]];
 					a.w = a.w + wt;
 #pragma unroll
-					for (int c = 0; c < CC; c++) a.n[c] = a.n[c] + q.v[u][s][c];
+					for (int c = 0; c < CC; c++)
+						a.n[c] = a.n[c] + (c < CC - 1 ? (sc.est_raw ? wt : 1.f) * q.v[u][s][c] : q.v[u][s][c]);
 					acc[o + soff[s]] = a;
 				}
 			}

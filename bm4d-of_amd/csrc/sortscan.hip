@@ -256,7 +256,7 @@ __global__ void early_fix_kernel(const uint8_t *__restrict__ early, const uint32
                                  const float *__restrict__ gweight, const uint32_t *__restrict__ lastf,
                                  const uint32_t *__restrict__ gtile, const uint32_t *__restrict__ tile_first,
                                  const uint32_t *__restrict__ base, int g0, int Gc, const float *__restrict__ win,
-                                 int C, int P, float *__restrict__ est, float *__restrict__ entry_w)
+                                 int C, int P, int raw, float *__restrict__ est, float *__restrict__ entry_w)
 {
 	const int gl = blockIdx.x * blockDim.x + threadIdx.x;
 	if (gl >= Gc) return;
@@ -271,7 +271,7 @@ __global__ void early_fix_kernel(const uint8_t *__restrict__ early, const uint32
 		if (gp >= tf) w = gweight[gp];
 		const uint32_t row = base[gl] + (uint32_t)n;
 		float *r = est + (size_t)row * C * P;
-		for (int i = 0; i < C * P; i++) r[i] = (w * win[i % P]) * r[i];
+		for (int i = raw * P; i < C * P; i++) r[i] = (w * win[i % P]) * r[i];   // raw: sc.est_raw
 		entry_w[row] = w;
 	}
 }
