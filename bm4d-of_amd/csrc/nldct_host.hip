@@ -1174,8 +1174,8 @@ StepDev upload_plan(bm4dof_ctx *ctx, const StepPlan &pl, DevBuf &geo_buf)
 
 // Grows every shared work buffer a plan's launches use, so that enqueueing
 // the step allocates nothing (required while a stream is being captured).
-// Threads of coef_kernel over one channel plane (one wave per 16 anchors
-// along x), 0 when the patch does not fit the video.
+// Runs of 16 anchors along x over one channel plane, 0 when the patch does not
+// fit the video.
 int64_t coef_waves(const StepConst &sc)
 {
 	const int nx = sc.W - sc.sPx + 1, ny = sc.H - sc.sPx + 1, nt = sc.F - sc.sPt + 1;
@@ -1264,7 +1264,8 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 	const size_t WHF = pl.WHF;
 	const int nimg = step1 ? 1 : 2;
 	const size_t per = coef_floats(pl, ctx->coef_budget);
-	const int64_t waves = coef_waves(sc);
+	// blocks of four waves, 32 anchors a wave and round
+	const unsigned blocks = (unsigned)std::min<int64_t>((coef_waves(sc) + 7) / 8, 4096);
 	d_coef_n = d_coef_b = nullptr;
 	if (per > 0 && ctx->coef_n.n >= per * sizeof(float) && (step1 || ctx->coef_b.n >= per * sizeof(float))) {
 		const bool have_n = !step1 && ctx->coef_n_keep && ctx->coef_n_ok && ctx->coef_n_whf == WHF &&
@@ -1277,8 +1278,8 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 			(i ? d_coef_b : d_coef_n) = tab;
 			if (i == 0 && have_n) continue;   // the first step's table of the same planes
 			for (int c = 0; c < C; c++)
-				hipLaunchKernelGGL(sc.sPx == 4 ? coef_kernel<4> : coef_kernel<8>, dim3((unsigned)waves), dim3(64), 0,
-				                   st, src + (size_t)c * WHF, sc.W, sc.H, sc.F, dv.basis, tab + (size_t)c * WHF * sc.P);
+				hipLaunchKernelGGL(sc.sPx == 4 ? coef_kernel<4> : coef_kernel<8>, dim3(blocks), dim3(256), 0, st, src + (size_t)c * WHF, sc.W, sc.H, sc.F,
+				                   dv.basis, tab + (size_t)c * WHF * sc.P);
 		}
 		HIPCHK(hipGetLastError());
 		ctx->coef_n_ok = true;

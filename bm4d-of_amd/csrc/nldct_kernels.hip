@@ -2294,64 +2294,55 @@ __device__ __forceinline__ int wave_sum_int(int v)
 // Forward transform of every patch anchor of a one-channel plane, once:
 // coef[pos*64 + k] = sum_p B[k][p] x[pos + off(p)] in the order of p (the same
 // dot product whatever group the patch is in, so the filters' rows read it bit
-// for bit).  One wave per run of anchors along x,
-// lane = coefficient, basis row in registers, four anchors per round (their
-// patches overlap: one load of a row segment serves all four).
+// for bit).  One wave per 32 anchors along x (grid-stride), row = anchor of the
+// fp32 matrix instructions, the basis in LDS for the block's four waves.
+// Bound: HBM writes, 2.24 GB at 960x540x20, and the loads' latency at three
+// waves a SIMD (the operands' registers; four spill).  On vector instructions,
+// lane = coefficient and four anchors a round, 1.9 ms; now the matching beside
+// it takes 0.8 ms less in step 1 and a table of 641x361x9 0.17 ms, before 0.29.
 template <int PX>
-__global__ __launch_bounds__(64)
+__global__ __launch_bounds__(256)
 void coef_kernel(const float *__restrict__ img, int W, int H, int F, const float *__restrict__ basis,
                  float *__restrict__ coef)
 {
-	constexpr int PT = FAST_P / (PX * PX);
-	constexpr int RUN = 16;   // anchors per wave
+	using T = MmTile<32>;
+	constexpr int PT = FAST_P / (PX * PX), P = FAST_P, Q = P / 4 / T::TS;
+	__shared__ __align__(16) float4 bf[P * P / 4];
+	mm_load_b<32>(basis, 1, P, P, bf);
+	__syncthreads();
 	const int nx = W - PX + 1, ny = H - PX + 1, nt = F - PT + 1;
-	const int runs_x = (nx + RUN - 1) / RUN;
-	const int64_t wid = blockIdx.x;
-	if (wid >= (int64_t)runs_x * ny * nt) return;
-	const int rx = (int)(wid % runs_x);
-	const int64_t rest = wid / runs_x;
-	const int y = (int)(rest % ny), t = (int)(rest / ny);
-	const int x0 = rx * RUN, x1 = min(x0 + RUN, nx);
-	const int lane = threadIdx.x;
-	const int64_t WH = (int64_t)W * H;
-	float brow[FAST_P];
+	const int runs_x = (nx + 31) / 32;
+	const int64_t WH = (int64_t)W * H, runs = (int64_t)runs_x * ny * nt;
+	const int lane = threadIdx.x & 63, h = lane >> 5, j = lane & 31;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	for (int64_t r0 = (int64_t)blockIdx.x * 4 + wave; r0 < runs; r0 += (int64_t)gridDim.x * 4) {
+		const int x0 = (int)(r0 % runs_x) * 32, n = min(32, nx - x0);
+		const int64_t rest = r0 / runs_x;
+		const int64_t pos0 = rest / ny * WH + rest % ny * W + x0;
+		// sample p = 2 s + h of a row of PX (even): h places from sample 2 s
+		const float *src = img + pos0;
+		const int at = min(j, n - 1) + h;
+		float4 a[Q];
 #pragma unroll
-	for (int p = 0; p < FAST_P; p++) brow[p] = basis[lane * FAST_P + p];
-	const int64_t pos0 = (int64_t)t * WH + (int64_t)y * W;
-	int x = x0;
-	for (; x + 3 < x1; x += 4) {
-		const float *s0 = img + pos0 + x;
-		float acc[4] = {0.f, 0.f, 0.f, 0.f};
+		for (int q = 0; q < Q; q++) {
+			float v[4];
 #pragma unroll
-		for (int ht = 0; ht < PT; ht++)
-#pragma unroll
-			for (int hy = 0; hy < PX; hy++) {
-				const float *r = s0 + ht * WH + hy * W;
-				float seg[PX + 3];
-#pragma unroll
-				for (int i = 0; i < PX + 3; i++) seg[i] = r[i];
-#pragma unroll
-				for (int hx = 0; hx < PX; hx++) {
-					const float b = brow[(ht * PX + hy) * PX + hx];
-#pragma unroll
-					for (int a = 0; a < 4; a++) acc[a] = __builtin_fmaf(seg[hx + a], b, acc[a]);
-				}
+			for (int u = 0; u < 4; u++) {
+				const int p = T::TS * (4 * q + u);
+				v[u] = (src + p / (PX * PX) * WH + p / PX % PX * W + p % PX)[at];
 			}
+			a[q] = make_float4(v[0], v[1], v[2], v[3]);
+		}
+		float *out = coef + pos0 * P;
 #pragma unroll
-		for (int a = 0; a < 4; a++) coef[(pos0 + x + a) * FAST_P + lane] = acc[a];
-	}
-	for (; x < x1; x++) {
-		const float *s0 = img + pos0 + x;
-		float acc = 0.f;
+		for (int t = 0; t < P / 32; t++) {
+			const auto c = mm_product<32, P>(a, bf, t);
 #pragma unroll
-		for (int ht = 0; ht < PT; ht++)
-#pragma unroll
-			for (int hy = 0; hy < PX; hy++) {
-				const float *r = s0 + ht * WH + hy * W;
-#pragma unroll
-				for (int hx = 0; hx < PX; hx++) acc = __builtin_fmaf(r[hx], brow[(ht * PX + hy) * PX + hx], acc);
+			for (int r = 0; r < T::NR; r++) {
+				const int row = T::row(r, h);
+				if (row < n) out[row * P + 32 * t + j] = c[r];
 			}
-		coef[(pos0 + x) * FAST_P + lane] = acc;
+		}
 	}
 }
 template __global__ void coef_kernel<4>(const float *, int, int, int, const float *, float *);
@@ -2539,14 +2530,15 @@ __device__ __forceinline__ void mm_inverse(const float (&z)[NMAX], float *__rest
 
 // Step-1 filter: hard threshold, one wave per group (grid-stride), lane =
 // coefficient of every row.  NMAX: rows held (8, 16, 32).
-// Bound: the memory's latency, 4 GB of table rows and 8.2 GB of est per launch
-// at 960x540x20 with 16 waves a CU (the registers' limit, and why the
-// inverse's rows go through LDS in halves: whole rows leave 12 waves, 4.98
-// ms).  There the inverse over the kept columns by vector instructions took
-// two thirds of 2340 a group: 5.46 ms, now 4.75.  Asking for the next group's
-// rows before this one's stores spills: 10.5 ms.
+// Bound: HBM, 7.5 GB of table rows and 8.5 GB of est per launch
+// at 960x540x20 (3.5 TB/s with the sort beside it).  There the inverse over
+// the kept columns by vector instructions took two thirds of 2340 a group:
+// 5.46 ms, now 4.7.  Its rows go through LDS in halves, so that LDS does not
+// bound the waves (4.98 ms with whole rows); with 32 rows three waves a SIMD
+// keep the registers out of scratch.  Asking for the next group's rows before
+// this one's stores spills: 10.5 ms.
 template <int PX, int NMAX, bool TAB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAB ? 4 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAB ? NMAX > 16 ? 3 : 4 : 2)))
 void filter1_fast_kernel(const float *__restrict__ img, const uint32_t *__restrict__ idx,
                          const uint32_t *__restrict__ nsim, const uint32_t *__restrict__ base,
                          const uint32_t *__restrict__ gtile, StepConst sc, int g0, int Gc,
