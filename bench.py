@@ -443,10 +443,11 @@ def main():
 
     # dominant kernel among the transform/filter, matching and aggregation stages
     # kernels this workload runs (one channel, 4x4x4 patches, 32 neighbours)
-    kern = {"s1_bm": "bm_reg_kernel<4, 4, false>", "s2_bm": "bm_reg_kernel<4, 4, false>",
+    fold = "agg_region_fold_kernel<1, 1, 4, 4, false, 3, 3, 5, 8, 68, false>"
+    kern = {"s1_bm": "bm_bound_kernel<4, 4, false, false>", "s2_bm": "bm_bound_kernel<4, 4, false, false>",
             "s1_coef": "coef_kernel<4>", "s2_coef": "coef_kernel<4>",
-            "s1_filter": "filter1_fast_kernel<4>", "s2_filter": "filter2_fast_kernel<4>",
-            "s1_aggregate": "agg_bin_fold_kernel<1, 32, 16, 4>", "s2_aggregate": "agg_bin_fold_kernel<1, 32, 16, 4>"}
+            "s1_filter": "filter1_fast_kernel<4, 32, true>", "s2_filter": "filter2_fast_kernel<4, 32, true>",
+            "s1_aggregate": fold, "s2_aggregate": fold}
     work = _stage_work(stats, (W - 3) * (H - 3) * (F - 3), W * H * F)
     ranked = sorted((k for k in stage_ms if k in kern), key=lambda k: -stage_ms[k])
     roofline = _roofline(ranked[0], stage_ms, launches, args.steps, work, kern)
