@@ -29,6 +29,10 @@ struct ArgError : std::runtime_error {
 			throw HipError(std::string(#x) + ": " + hipGetErrorString(e_));               \
 	} while (0)
 
+// Frees the current device's idle table blocks (nldct_host.hip); false when
+// there were none.
+bool idle_trim();
+
 // Grow-only device buffer.
 struct DevBuf {
 	void *p = nullptr;
@@ -39,8 +43,10 @@ struct DevBuf {
 		p = nullptr;
 		n = 0;
 		if (bytes == 0) bytes = 256;
-		if (hipMalloc(&p, bytes) != hipSuccess) {
+		while (hipMalloc(&p, bytes) != hipSuccess) {
 			(void)hipGetLastError();
+			p = nullptr;
+			if (idle_trim()) continue;
 			throw ArgError("device allocation of " + std::to_string(bytes) + " bytes failed",
 			               BM4DOF_ENOMEM);
 		}
@@ -89,8 +95,11 @@ struct bm4dof_ctx {
 	// bytes of per-anchor coefficient tables a step may hold (0: none); at
 	// context creation the smaller of 96 GiB and 2/5 of the free device memory
 	size_t coef_budget = (size_t)96 << 30;
-	// keep the tables allocated between calls (else released at each call's end)
+	// keep the tables with the context between calls (else they go to the
+	// device's idle blocks at each call's end, of which it keeps idle_max bytes)
 	bool keep_tables = false;
+	size_t idle_max = 0;
+	bool counted = false;   // among the device's contexts (idle blocks)
 	// the noisy coefficient table of the last step that filled it (patch
 	// shape, channels, size, basis), and whether the next step of the same
 	// run may read it: set around the second step when both steps see the

@@ -10,6 +10,7 @@
 #include <string>
 #include <vector>
 #include <memory>
+#include <mutex>
 #include <algorithm>
 #include <stdexcept>
 
@@ -1192,6 +1193,82 @@ size_t coef_floats(const StepPlan &pl, size_t budget)
 	return per * sizeof(float) * (pl.step1 ? 1 : 2) <= budget ? per : 0;
 }
 
+// Idle table blocks.  A step's coefficient tables are hundreds of megabytes to
+// gigabytes.  Freed at a call's end and allocated in the next, they cost a call
+// between half a millisecond and, when the driver has not cleared what was
+// freed, hundreds of them (480x270x12 of 8 bits: 8.9 ms a call, up to 25 with
+// it; 641x360x9 in colour 19.8 and 67 to 188).  So a call's end leaves them here, for
+// the next call on any context of the device, up to an eighth of its memory;
+// they are freed when an allocation of the library fails, when a context's
+// coef_budget is set, and with the device's last context.
+struct IdleBlock {
+	int device;
+	void *p;
+	size_t n;
+};
+std::mutex g_idle_mu;
+std::vector<IdleBlock> g_idle;       // oldest first
+std::vector<int> g_idle_contexts;    // devices of the live contexts
+
+// Frees the blocks of `device`, the oldest first, until at most `left` bytes
+// of them are left (with g_idle_mu held).
+bool idle_free(int device, size_t left)
+{
+	size_t sum = 0;
+	for (const IdleBlock &b : g_idle) sum += b.device == device ? b.n : 0;
+	bool any = false;
+	for (size_t i = 0; i < g_idle.size() && sum > left;) {
+		if (g_idle[i].device != device) { i++; continue; }
+		sum -= g_idle[i].n;
+		(void)hipFree(g_idle[i].p);
+		g_idle.erase(g_idle.begin() + i);
+		any = true;
+	}
+	return any;
+}
+size_t idle_bytes(int device)
+{
+	std::lock_guard<std::mutex> lk(g_idle_mu);
+	size_t sum = 0;
+	for (const IdleBlock &b : g_idle) sum += b.device == device ? b.n : 0;
+	return sum;
+}
+// A table of at least `bytes`: the smallest idle block that holds it, else a
+// new one.
+void table_get(bm4dof_ctx *ctx, DevBuf &b, size_t bytes)
+{
+	if (b.p && b.n >= bytes) return;
+	if (b.p) HIPCHK(hipFree(b.p));
+	b.p = nullptr;
+	b.n = 0;
+	{
+		std::lock_guard<std::mutex> lk(g_idle_mu);
+		auto best = g_idle.end();
+		for (auto i = g_idle.begin(); i != g_idle.end(); ++i)
+			if (i->device == ctx->device && i->n >= bytes && (best == g_idle.end() || i->n < best->n)) best = i;
+		if (best != g_idle.end()) {
+			b.p = best->p;
+			b.n = best->n;
+			g_idle.erase(best);
+		}
+	}
+	(void)b.get(bytes);
+}
+// The table to the idle blocks.  No launch that uses it is left.
+void table_put(bm4dof_ctx *ctx, DevBuf &b)
+{
+	if (!b.p) return;
+	if (b.n > ctx->idle_max) {
+		b.release();
+		return;
+	}
+	std::lock_guard<std::mutex> lk(g_idle_mu);
+	idle_free(ctx->device, ctx->idle_max - b.n);
+	g_idle.push_back({ctx->device, b.p, b.n});
+	b.p = nullptr;
+	b.n = 0;
+}
+
 void reserve_step(bm4dof_ctx *ctx, const StepPlan &pl)
 {
 	const size_t G = (size_t)std::max(pl.G, 1), np = (size_t)pl.np;
@@ -1235,8 +1312,8 @@ void reserve_step(bm4dof_ctx *ctx, const StepPlan &pl)
 	const size_t per = coef_floats(pl, ctx->coef_budget);
 	if (per > 0) {
 		try {
-			(void)ctx->coef_n.as<float>(per);
-			if (!pl.step1) (void)ctx->coef_b.as<float>(per);
+			table_get(ctx, ctx->coef_n, per * sizeof(float));
+			if (!pl.step1) table_get(ctx, ctx->coef_b, per * sizeof(float));
 		} catch (const ArgError &e) {
 			if (e.code != BM4DOF_ENOMEM) throw;
 			ctx->coef_n.release();
@@ -2047,15 +2124,24 @@ void batch_capture(bm4dof_batch *b)
 
 } // namespace
 
+bool bm4dof::idle_trim()
+{
+	int device = 0;
+	if (hipGetDevice(&device) != hipSuccess) return false;
+	std::lock_guard<std::mutex> lk(g_idle_mu);
+	return idle_free(device, 0);
+}
+
 namespace {
 
-// End of a denoiser call: the coefficient tables (several GB) go back to the
-// device unless the caller asked to keep them for the next call.
+// End of a denoiser call, its streams idle: the coefficient tables (several
+// GB) go to the device's idle blocks unless the caller asked to keep them
+// with the context.
 void end_run(bm4dof_ctx *ctx)
 {
 	if (!ctx->keep_tables) {
-		ctx->coef_n.release();
-		ctx->coef_b.release();
+		table_put(ctx, ctx->coef_n);
+		table_put(ctx, ctx->coef_b);
 	}
 	ctx->coef_n_ok = false;
 }
@@ -2132,10 +2218,16 @@ int bm4dof_ctx_create(bm4dof_ctx **out, int device)
 		else
 			ctx->tv_pin = nullptr;
 		tv_scratch_init(device);
-		// coefficient tables: at most 2/5 of the device memory free now
+		// coefficient tables: at most 2/5 of the device memory free now (idle
+		// table blocks count as free)
 		size_t free_b = 0, total_b = 0;
 		HIPCHK(hipMemGetInfo(&free_b, &total_b));
+		free_b += idle_bytes(device);
 		ctx->coef_budget = std::min(ctx->coef_budget, free_b / 5 * 2);
+		ctx->idle_max = total_b / 8;
+		std::lock_guard<std::mutex> lk(g_idle_mu);
+		g_idle_contexts.push_back(device);
+		ctx->counted = true;
 	});
 	if (rc) {
 		g_global_err = ctx->err;
@@ -2156,6 +2248,11 @@ void bm4dof_ctx_destroy(bm4dof_ctx *ctx)
 	for (auto e : ctx->ev) (void)hipEventDestroy(e);
 	ctx->plan_cache.reset();
 	for (DevBuf *b : ctx->buffers()) b->release();
+	if (ctx->counted) {
+		std::lock_guard<std::mutex> lk(g_idle_mu);
+		g_idle_contexts.erase(std::find(g_idle_contexts.begin(), g_idle_contexts.end(), ctx->device));
+		if (!std::count(g_idle_contexts.begin(), g_idle_contexts.end(), ctx->device)) idle_free(ctx->device, 0);
+	}
 	if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
 	if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
 	if (ctx->ev_coef) (void)hipEventDestroy(ctx->ev_coef);
@@ -2190,6 +2287,8 @@ int bm4dof_ctx_set_option(bm4dof_ctx *ctx, const char *key, long long value)
 		} else if (k == "coef_budget") {
 			if (value < 0) throw ArgError("coef_budget must be >= 0");
 			ctx->coef_budget = (size_t)value;
+			std::lock_guard<std::mutex> lk(g_idle_mu);
+			idle_free(ctx->device, 0);
 		} else if (k == "keep_tables") {
 			ctx->keep_tables = value != 0;
 		} else if (k == "vbm3d_search") {

@@ -149,11 +149,15 @@ const char *bm4dof_global_error(void);
  *                  1368-1589), driven by the parameters' sizeSearchWindowPred,
  *                  nSimilarPatchesPred and dsub.  This one changes results:
  *                  it selects the search a differently built reference runs.
- *   "keep_tables"  0 (default): the tables are freed at the end of every
- *                  bm4dof_run / _run_dev / _run_learned(_dev) call; 1: they
- *                  stay allocated for the next call on the context (saves
- *                  their allocation when videos of one shape are denoised
- *                  repeatedly).
+ *   "keep_tables"  0 (default): at the end of every bm4dof_run / _run_dev /
+ *                  _run_learned(_dev) call the tables' memory becomes idle,
+ *                  for the next call on any context of the device to take;
+ *                  the library keeps at most an eighth of the device's memory
+ *                  idle (the oldest blocks are freed beyond that, and larger
+ *                  tables at once) and frees it when one of its allocations
+ *                  fails, when a context's "coef_budget" is set (to any
+ *                  value) and with the device's last context; 1: the tables
+ *                  stay with the context.
  * Returns BM4DOF_EINVAL for an unknown key.
  */
 int bm4dof_ctx_set_option(bm4dof_ctx *ctx, const char *key, long long value);

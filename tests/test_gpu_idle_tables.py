@@ -1,0 +1,70 @@
+"""The coefficient tables' memory between calls: it stays allocated and idle
+(a call allocates nothing once its shape has run), any context of the device
+takes it, and setting a coef_budget gives it back.  Device memory is read as
+the runtime reports it, in steps of 2 MiB and per buffer; the tables are 36 MB
+each."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import bm4dof_amd as A, synth
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = (6, 1, 136, 176)
+TABLE = 6 * 136 * 176 * 64 * 4
+SLACK = 16 << 20
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_tables_stay_idle_between_calls_and_go_back():
+    noisy = synth.add_noise(synth.video(176, 136, 6, n_shapes=6, seed=2), 20.0, 3)
+    assert noisy.shape == SHAPE
+    p1, p2 = (A.cli_params(s, 20.0, noisy.shape, px=4, pt=4, wx=7, np_=8) for s in (1, 2))
+    made = []
+
+    def context(budget=None):
+        c = A.Context(0)
+        made.append(c)
+        if budget is not None:
+            c.set_option("coef_budget", budget)       # nothing idle from here on
+        return c
+
+    try:
+        warm = context(0)                             # code objects, flow scratch
+        b0, f0, _ = warm.run(p1, p2, noisy, nparts=2)
+        c = context(0)
+        before = _free()
+        c.run(p1, p2, noisy, nparts=2)
+        other = before - _free()                      # what a run takes beside the tables
+
+        a = context()
+        before = _free()
+        b1, f1, _ = a.run(p1, p2, noisy, nparts=2)
+        first = _free()
+        assert before - first >= other + 2 * TABLE - SLACK
+        for _ in range(3):
+            a.run(p1, p2, noisy, nparts=2)
+            assert _free() == first
+        b = context()
+        before = _free()
+        b2, f2, _ = b.run(p1, p2, noisy, nparts=2)
+        assert before - _free() <= other + SLACK      # the same tables
+        before = _free()
+        a.set_option("coef_budget", 96 << 30)
+        assert _free() - before >= 2 * TABLE - SLACK
+        b3, f3, _ = a.run(p1, p2, noisy, nparts=2)
+        for x, y in ((b1, f1), (b2, f2), (b3, f3)):
+            assert np.array_equal(b0, x) and np.array_equal(f0, y)
+        a.set_option("keep_tables", 1)                # with the context: not idle
+        a.run(p1, p2, noisy, nparts=2)
+        before = _free()
+        b.set_option("coef_budget", 96 << 30)
+        assert _free() - before < SLACK
+    finally:
+        for c in made:
+            c.close()
