@@ -2676,8 +2676,11 @@ void filter2_fast_kernel(const float *__restrict__ noisy, const float *__restric
 		for (int n = 0; n < NMAX; n++) {
 			if (n < N) {
 				const float w = y[n] * y[n] / (y[n] * y[n] + sc.beta_sigma2);
-				z[n] = z[n] * w;
-				y[n] = P == FAST_P || lane < P ? w * w : 0.f;
+				// past the patch's samples y is 0, and w is not a number when
+				// beta is 0: those terms enter the inverse's products too
+				const bool in = P == FAST_P || lane < P;
+				z[n] = in ? z[n] * w : 0.f;
+				y[n] = in ? w * w : 0.f;
 			}
 		}
 		// sum of w^2 in the reference's order, channel, coefficient, then
@@ -2819,7 +2822,7 @@ void filter2_wide_kernel(const float *__restrict__ noisy, const float *__restric
 		for (int n = 0; n < NMAX; n++) {
 			if (n < N) {
 				const float w = y[n] * y[n] / (y[n] * y[n] + sc.beta_sigma2);
-				z[n] = z[n] * w;
+				z[n] = tid < P ? z[n] * w : 0.f;   // see filter2_fast_kernel
 				y[n] = tid < P ? w * w : 0.f;
 			}
 		}
