@@ -294,12 +294,15 @@ class Context:
     def stats(self):
         """Statistics of the last run: dict with the ordered aggregation's
         pixel blocks / banded blocks / block shape and the groups and group
-        rows of each step, and the executed TV-L1 iterations x pixels of the
-        last flow computation."""
-        v = (C.c_int64 * 10)()
-        n = self._L.bm4dof_last_stats(self.h, v, 10)
+        rows of each step, the executed TV-L1 iterations x pixels of the last
+        flow computation, and per step the groups that the matching by
+        bounded distances left to another matcher (-1: not taken) and the
+        chunks of groups."""
+        v = (C.c_int64 * 14)()
+        n = self._L.bm4dof_last_stats(self.h, v, 14)
         keys = ("agg_blocks", "agg_banded_blocks", "agg_bx", "agg_by", "agg_bt",
-                "groups1", "rows1", "groups2", "rows2", "tvl1_pixel_iters")
+                "groups1", "rows1", "groups2", "rows2", "tvl1_pixel_iters", "bm_redone1",
+                "bm_redone2", "chunks1", "chunks2")
         return {keys[i]: int(v[i]) for i in range(n)}
 
     def bm(self, p, image, fflow=None, bflow=None, nparts=2):

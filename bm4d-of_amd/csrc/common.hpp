@@ -52,6 +52,42 @@ struct BinShape { int lx, ly, lt; };
 // most rows per tile of the first bin-sort pass (at most 8 pairs per row)
 #define BIN_RT 4096
 
+// Groups that the bounded matching leaves to another matcher: RedoList::N
+// lists, a group in the one of its index modulo N, whose counters lie on lines
+// of their own.  (One counter for all takes 7 ns a group, 7 ms where a million
+// groups are left.)  Without a bound (scale 0) every group is, and nothing is
+// listed.
+struct RedoList {
+	static constexpr int N = 64, LINE = 32;
+	uint32_t *p;              // N counters, LINE words apart, then N lists
+	const float2 *qp;         // (mid, scale) of the integer samples
+	uint32_t *total;          // running total of such groups
+	int G;
+	__host__ __device__ static size_t words(int G) { return (size_t)N * LINE + (size_t)N * ((G + N - 1) / N); }
+	__device__ void add(int g) const
+	{
+		uint32_t *c = p + (g % N) * LINE;
+		const uint32_t i = atomicAdd(c, 1u);
+		p[N * LINE + (size_t)(g % N) * ((G + N - 1) / N) + i] = (uint32_t)g;
+	}
+	// the groups a block of a grid of a multiple of N blocks takes: number
+	// i = first(), first() + step(), ... below count() (called once)
+	__device__ int first() const { return (int)(blockIdx.x / N); }
+	__device__ int step() const { return (int)(gridDim.x / N); }
+	__device__ int count() const
+	{
+		const int l = (int)(blockIdx.x % N);
+		const int n = qp->y > 0.f ? (int)p[l * LINE] : (G - l + N - 1) / N;
+		if (first() == 0 && threadIdx.x == 0) atomicAdd(total, (uint32_t)n);
+		return n;
+	}
+	__device__ int at(int i) const
+	{
+		const int l = (int)(blockIdx.x % N);
+		return qp->y > 0.f ? (int)p[N * LINE + (size_t)l * ((G + N - 1) / N) + i] : l + N * i;
+	}
+};
+
 // Decode a 3-index position t*WH + y*W + x.
 __host__ __device__ inline void pos_decode(uint32_t pos, int W, int WH, int &x, int &y, int &t)
 {

@@ -112,6 +112,11 @@ struct bm4dof_ctx {
 	uint64_t agg_blocks = 0, agg_overflow_blocks = 0;
 	int agg_region[3] = {0, 0, 0};
 	uint64_t step_groups[2] = {0, 0}, step_rows[2] = {0, 0};   // groups / group rows per step
+	// bounded matching: whether a step of the last run took it, and the groups
+	// it left to another matcher; chunks of groups per step
+	bool step_bounded[2] = {false, false};
+	uint32_t step_redone[2] = {0, 0};
+	int step_chunks[2] = {0, 0};
 	bool fast_filter = true;   // register-resident filter where the group shape allows it
 	int fast_bm = 2;           // block matching: 2 register windows, 1 LDS-staged windows, 0 general
 	int bm_frames = 2;         // frames of search window staged per round of the staged matching

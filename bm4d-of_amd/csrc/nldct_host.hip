@@ -31,21 +31,21 @@ __global__ void bm_window_kernel(const float *, const float *, const uint32_t *,
 template <int PX, int PT, bool MC, bool LIST> __global__ void bm_reg_kernel(const float *, const int4 *, const int2 *,
                                                         const uint32_t *, const uint32_t *, const TileBox *,
                                                         StepConst, int, int, uint32_t *, uint32_t *, int,
-                                                        uint32_t *, uint32_t *, int, const uint32_t *);
+                                                        uint32_t *, uint32_t *, int, RedoList);
 template <int PX, int PT, int NF> __global__ void bm_fast_kernel(BMF_ARGS);
 __global__ void bmq_range_kernel(const float *, int, int, int, float2 *);
-__global__ void bmq_scale_kernel(const float2 *, int, float, float2 *);
+__global__ void bmq_scale_kernel(const float2 *, int, float, float, float2 *);
 template <int PT>
 __global__ void bmq_pack_kernel(const float *, int, int, int, int64_t, int64_t, const float2 *, int16_t *);
 template <int PX, int PT>
 __global__ void bmq_norm_kernel(const int16_t *, int, int, int, int64_t, int, uint32_t *);
 #define BMB_ARGS const float *, const int16_t *, const uint32_t *, const float2 *, const int4 *, const int2 *, \
 	const uint32_t *, const uint32_t *, const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int,    \
-	uint32_t *, uint32_t *, uint32_t *, uint32_t *
+	uint32_t *, uint32_t *, RedoList
 template <int PX, int PT, bool MC, bool CH> __global__ void bm_bound_kernel(BMB_ARGS);
 __global__ void bm_list_kernel(const float *, const float *, const float *, const uint32_t *, const uint32_t *,
-                               const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, const uint32_t *,
-                               const uint32_t *, uint32_t *, uint32_t *);
+                               const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, RedoList, uint32_t *,
+                               uint32_t *);
 __global__ void filter1_kernel(const float *, const uint32_t *, const uint32_t *, const uint32_t *,
                                const uint32_t *, StepConst, int, int, const float *, const float *,
                                const float *, float *, float *, uint32_t *, uint8_t *, float *,
@@ -591,7 +591,7 @@ static void bm_bound_reserve(bm4dof_ctx *ctx, const StepConst &sc, int step, int
 	(void)ctx->bmq_part.as<float2>(BMQ_RANGE_BLOCKS + 1);
 	(void)ctx->bmq_img.as<int16_t>((step == 1 ? 1 : sc.C) * WHF * sc.sPt + 32);
 	(void)ctx->bmq_norm.as<uint32_t>(WHF);
-	(void)ctx->bmq_list.as<uint32_t>((size_t)G + 1);
+	(void)ctx->bmq_list.as<uint32_t>(RedoList::words(G));
 }
 static void bm_bound(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, const float *ff,
                      const float *bf, const uint32_t *d_gpos, const uint32_t *d_gtile, const TileBox *d_tiles, int G,
@@ -604,16 +604,24 @@ static void bm_bound(bm4dof_ctx *ctx, const StepConst &sc, int step, const float
 	float2 *part = ctx->bmq_part.as<float2>(BMQ_RANGE_BLOCKS + 1), *qp = part + BMQ_RANGE_BLOCKS;
 	int16_t *qimg = ctx->bmq_img.as<int16_t>((size_t)nch * WHF * sc.sPt + 32);
 	uint32_t *norm = ctx->bmq_norm.as<uint32_t>((size_t)WHF);
-	uint32_t *list = ctx->bmq_list.as<uint32_t>((size_t)G + 1);
+	const RedoList list = {ctx->bmq_list.as<uint32_t>(RedoList::words(G)), qp,
+	                       ctx->counters.as<uint32_t>(16) + 9 + step, G};
+	ctx->step_bounded[step - 1] = true;
 	int4 *d_wins = ctx->bm_wins.as<int4>((size_t)G * sWt);
 	int2 *d_wmeta = ctx->bm_wmeta.as<int2>((size_t)G);
-	fill_u32(ctx, list, 0u, 1);
+	fill_u32(ctx, list.p, 0u, RedoList::N * RedoList::LINE);
 	// the channels the distances run on: the first nch planes of a frame
 	const int nf = sc.WH * nch, rx = std::min(32, nblk(nf, 1024)), ry = std::min(sc.F, BMQ_RANGE_BLOCKS / rx);
 	hipLaunchKernelGGL(bmq_range_kernel, dim3(rx, ry), dim3(256), 0, st, img, sc.WHC, nf, sc.F, part);
 	const int nblocks = rx * ry;
 	const float Q = floorf(sqrtf(2147483648.f / (float)(sc.P * nch))) - 2.f;
-	hipLaunchKernelGGL(bmq_scale_kernel, dim3(1), dim3(64), 0, st, part, nblocks, Q, qp);
+	// integer steps per noise level below which nothing is bounded: one
+	// sample far off the others leaves the rest few steps.  960x540x20, step 1:
+	// at 29 steps 7.2 ms, at 14 12.4, at 2.3 14.0, and 11.4 with no group
+	// bounded; step 2 24.3, 26.1, 29.8 and 23.7.  (7x7x1, whose other matcher is
+	// slower, 640x361x11: at 7.7 steps 2.75 ms, at 2.3 3.29, without 3.16.)
+	const float least = (sc.sPx == 4 || sc.sPx == 8 ? 16.f : 4.f) / sqrtf(sc.sigma2);
+	hipLaunchKernelGGL(bmq_scale_kernel, dim3(1), dim3(64), 0, st, part, nblocks, Q, least, qp);
 	hipLaunchKernelGGL(sc.sPt == 4 ? bmq_pack_kernel<4> : bmq_pack_kernel<1>, dim3(nblk(nch * WHF, 256)), dim3(256), 0, st, img, sc.WH, sc.WHC, sc.F, WHF,
 	                   nch * WHF, qp, qimg);
 	const auto nk = sc.sPx == 4 ? bmq_norm_kernel<4, 4> : sc.sPx == 8 ? bmq_norm_kernel<8, 1>
@@ -634,16 +642,17 @@ static void bm_bound(bm4dof_ctx *ctx, const StepConst &sc, int step, const float
 	const auto kern = sc.sPx == 4 ? bound_of<4, 4>(nch > 1, rchunks > 1) : sc.sPx == 8 ? bound_of<8, 1>(nch > 1, rchunks > 1)
 	                  : sc.sPx == 7 ? bound_of<7, 1>(nch > 1, rchunks > 1) : bound_of<11, 1>(nch > 1, rchunks > 1);
 	hipLaunchKernelGGL(kern, dim3(G), dim3(64), std::max((size_t)maxCand * 4, (size_t)256 * 8), st, img, qimg, norm, qp, d_wins, d_wmeta, d_gpos,
-	                   d_gtile, d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, list, list + 1);
+	                   d_gtile, d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, list);
+	const unsigned rblocks = (unsigned)nblk(std::min(G, 8192), RedoList::N) * RedoList::N;
 	if ((sc.sPx == 4 || sc.sPx == 8) && maxCand * 8 <= 56 * 1024) {
 		const auto reg = nch == 1 ? (sc.sPx == 4 ? bm_reg_kernel<4, 4, false, true> : bm_reg_kernel<8, 1, false, true>)
 		                          : (sc.sPx == 4 ? bm_reg_kernel<4, 4, true, true> : bm_reg_kernel<8, 1, true, true>);
 		const int rc = std::max(1, std::min(sc.sWx, 64 / std::max(1, sWt * sc.sWx)));
-		hipLaunchKernelGGL(reg, dim3((unsigned)std::min(G, 8192)), dim3(64), (size_t)maxCand * 8, st, img, d_wins, d_wmeta,
+		hipLaunchKernelGGL(reg, dim3(rblocks), dim3(64), (size_t)maxCand * 8, st, img, d_wins, d_wmeta,
 		                   d_gpos, d_gtile, d_tiles, sc, rc, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G, list);
 	} else
-		hipLaunchKernelGGL(bm_list_kernel, dim3((unsigned)std::min(G, 2048)), dim3(256), lds, st, img, ff, bf, d_gpos,
-		                   d_gtile, d_tiles, sc, step, maxCand, d_idx, d_nsim, G, list, list + 1, d_ties, d_ties + 1);
+		hipLaunchKernelGGL(bm_list_kernel, dim3(rblocks), dim3(256), lds, st, img, ff, bf, d_gpos,
+		                   d_gtile, d_tiles, sc, step, maxCand, d_idx, d_nsim, G, list, d_ties, d_ties + 1);
 	HIPCHK(hipGetLastError());
 }
 
@@ -701,7 +710,7 @@ void run_bm(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, co
 		auto kern = nch == 1 ? (PX == 4 ? bm_reg_kernel<4, 4, false, false> : bm_reg_kernel<8, 1, false, false>)
 		                     : (PX == 4 ? bm_reg_kernel<4, 4, true, false> : bm_reg_kernel<8, 1, true, false>);
 		hipLaunchKernelGGL(kern, dim3(G), dim3(64), lds_reg, ctx->stream, img, d_wins, d_wmeta, d_gpos, d_gtile,
-		                   d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G, (const uint32_t *)nullptr);
+		                   d_tiles, sc, rchunks, nch, d_idx, d_nsim, G, d_ties, d_ties + 1, G, RedoList{});
 		HIPCHK(hipGetLastError());
 		bm_ties(ctx, sc, step, img, ff, bf, d_gpos, d_gtile, d_tiles, G, d_idx, d_nsim, d_ties, maxCand, lds);
 		return;
@@ -1759,6 +1768,7 @@ uint64_t run_step(bm4dof_ctx *ctx, const bm4dof_params &p, int W, int H, int F, 
 		if (ratio) *ratio += 100.f * (float)n / (float)((size_t)W * H * F);
 	}
 	ctx->step_groups[pl.step1 ? 0 : 1] += groups;
+	ctx->step_chunks[pl.step1 ? 0 : 1] = nblk(std::max(pl.G, 1), pl.chunk_groups);
 	enqueue_step(ctx, pl, cp->dv, noisy_w, basic_w, ffu, bfu, out_w, &tm, la, 2);
 	return groups;
 }
@@ -1768,6 +1778,8 @@ void stats_begin(bm4dof_ctx *ctx)
 {
 	ctx->agg_blocks = ctx->agg_overflow_blocks = 0;
 	ctx->step_groups[0] = ctx->step_groups[1] = ctx->step_rows[0] = ctx->step_rows[1] = 0;
+	ctx->step_bounded[0] = ctx->step_bounded[1] = false;
+	ctx->step_chunks[0] = ctx->step_chunks[1] = 0;
 	fill_u32(ctx, ctx->counters.as<uint32_t>(16), 0u, 16);
 	fill_u32(ctx, (uint32_t *)ctx->stat64.as<unsigned long long>(4), 0u, 8);
 }
@@ -1781,6 +1793,8 @@ void stats_end(bm4dof_ctx *ctx)
 	ctx->step_rows[0] = rows[0];
 	ctx->step_rows[1] = rows[1];
 	ctx->agg_overflow_blocks = cnt[4];
+	ctx->step_redone[0] = cnt[10];
+	ctx->step_redone[1] = cnt[11];
 }
 
 // The two steps of runNlBayes on device buffers (nldct.cpp:352-470), with
@@ -2649,13 +2663,14 @@ __attribute__((visibility("default")))
 int bm4dof_last_stats(const bm4dof_ctx *ctx, int64_t *stats, int max_slots)
 {
 	if (!ctx || !stats) return 0;
-	const int64_t v[10] = {(int64_t)ctx->agg_blocks, (int64_t)ctx->agg_overflow_blocks,
+	const auto redone = [&](int s) { return ctx->step_bounded[s] ? (int64_t)ctx->step_redone[s] : -1; };
+	const int64_t v[14] = {(int64_t)ctx->agg_blocks, (int64_t)ctx->agg_overflow_blocks,
 	                       ctx->agg_region[0], ctx->agg_region[1], ctx->agg_region[2],
 	                       (int64_t)ctx->step_groups[0], (int64_t)ctx->step_rows[0],
 	                       (int64_t)ctx->step_groups[1], (int64_t)ctx->step_rows[1],
-	                       (int64_t)ctx->tv_pixel_iters};
+	                       (int64_t)ctx->tv_pixel_iters, redone(0), redone(1), ctx->step_chunks[0], ctx->step_chunks[1]};
 	int n = 0;
-	for (; n < 10 && n < max_slots; n++) stats[n] = v[n];
+	for (; n < 14 && n < max_slots; n++) stats[n] = v[n];
 	return n;
 }
 

@@ -883,6 +883,7 @@ __device__ void bm_radix_select(const uint32_t *__restrict__ skey, int *__restri
 	for (int j = lane; j < nb; j += 64) {
 		const int r = stie[j];
 		int c = 0;
+#pragma unroll 8
 		for (int i = 0; i < nb; i++) c += stie[i] < r;
 		if (c < (int)remaining) {
 			sel_key[na_expected + c] = T;
@@ -1084,7 +1085,8 @@ __device__ __forceinline__ void bmr_load_row(float (&dst)[PT][PX], const float *
 		}
 }
 
-// LIST: the groups to match are list[1 ..], list[0] of them (grid-stride).
+// LIST: the groups to match are the listed ones, a block loops over some of
+// them; else a block's is its own.
 template <int PX, int PT, bool MC, bool LIST>
 __global__ __launch_bounds__(64)
 void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
@@ -1092,7 +1094,7 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
                    const uint32_t *__restrict__ gtile, const TileBox *__restrict__ tiles,
                    StepConst sc, int rchunks, int nch, uint32_t *__restrict__ out_idx,
                    uint32_t *__restrict__ out_nsim, int G, uint32_t *__restrict__ tie_count,
-                   uint32_t *__restrict__ tie_list, int tie_cap, const uint32_t *__restrict__ list)
+                   uint32_t *__restrict__ tie_list, int tie_cap, RedoList list)
 {
 	constexpr int PP = PX * PX * PT;
 	extern __shared__ unsigned char smem[];
@@ -1105,9 +1107,9 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 	__shared__ int out_rank[64];
 
 	const int lane = threadIdx.x;
-	const int count = LIST ? (int)min(list[0], (uint32_t)G) : G;
-	for (int gi = blockIdx.x; gi < count; gi += gridDim.x) {
-	const int g = LIST ? (int)list[gi + 1] : gi;
+	const int count = LIST ? list.count() : G, step = LIST ? list.step() : (int)gridDim.x;
+	for (int gi = LIST ? list.first() : (int)blockIdx.x; gi < count; gi += step) {
+	const int g = LIST ? list.at(gi) : gi;
 	const uint32_t pos = gpos[g];
 	uint32_t *oidx = out_idx + (size_t)g * sc.npmax;
 	if (sc.npmax <= 1) {
@@ -1287,7 +1289,7 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 }
 
 #define BMR_ARGS const float *, const int4 *, const int2 *, const uint32_t *, const uint32_t *, \
-	const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int, const uint32_t *
+	const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int, uint32_t *, uint32_t *, int, RedoList
 template __global__ void bm_reg_kernel<4, 4, false, false>(BMR_ARGS);
 template __global__ void bm_reg_kernel<4, 4, false, true>(BMR_ARGS);
 template __global__ void bm_reg_kernel<8, 1, false, false>(BMR_ARGS);
@@ -1358,9 +1360,9 @@ void bmq_range_kernel(const float *__restrict__ v, int whc, int n, int F, float2
 }
 
 // (mid, scale) for samples in +-Q, scale 0 when the range is not finite or
-// empty.  One wave.
+// empty, or when the scale comes out below `least`.  One wave.
 __global__ __launch_bounds__(64)
-void bmq_scale_kernel(const float2 *__restrict__ part, int nb, float Q, float2 *__restrict__ out)
+void bmq_scale_kernel(const float2 *__restrict__ part, int nb, float Q, float least, float2 *__restrict__ out)
 {
 	float lo = INFINITY, hi = -INFINITY;
 	for (int i = threadIdx.x; i < nb; i += 64) {
@@ -1378,7 +1380,7 @@ void bmq_scale_kernel(const float2 *__restrict__ part, int nb, float Q, float2 *
 		// ranges whose squares leave the normal floats (then the reference's
 		// distances meet at 0 or infinity) or whose v - mid is coarse
 		const float s = half > 1e-15f && half < 1e15f && half > 1e-4f * fabsf(mid) ? Q / half * 0.9999f : 0.f;
-		*out = make_float2(mid, s);
+		*out = make_float2(mid, s >= least ? s : 0.f);
 	}
 }
 
@@ -1500,7 +1502,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
                      const TileBox *__restrict__ tiles, StepConst sc, int rchunks, int nch,
                      uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_nsim, int G,
                      uint32_t *__restrict__ tie_count, uint32_t *__restrict__ tie_list,
-                     uint32_t *__restrict__ redo_count, uint32_t *__restrict__ redo_list)
+                     RedoList redo)
 {
 	using R = BmqRow<PX, PT>;
 	constexpr int NW = R::NW, NC = R::NC;
@@ -1514,7 +1516,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
 	__shared__ int f_qt[64];             // and the frame
 
 	const int g = blockIdx.x;
-	if (g >= G) return;
+	if (g >= G || !(qp->y > 0.f)) return;
 	const int lane = threadIdx.x;
 	const int sWt = sc.wtf + sc.wtb + 1;
 	const uint32_t pos = gpos[g];
@@ -1647,7 +1649,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
 		for (int o = 0; o < NC; o++) n += __popcll(__ballot(lmin[o] <= v)) + __popcll(__ballot(lmin2[o] <= v));
 		return n;
 	};
-	bool fits = qp->y > 0.f && of_columns(0xfffffffeu) >= kk;
+	bool fits = of_columns(0xfffffffeu) >= kk;
 	int cnt = 0;
 	if (fits) {
 		uint32_t mx = 0;
@@ -1669,7 +1671,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
 		fits = cnt <= BMQ_CAP;
 	}
 	if (!fits) {
-		if (lane == 0) redo_list[atomicAdd(redo_count, 1u)] = (uint32_t)g;
+		if (lane == 0) redo.add(g);
 		return;
 	}
 	__syncthreads();
@@ -1759,13 +1761,12 @@ __global__ __launch_bounds__(BM_THREADS)
 void bm_list_kernel(const float *__restrict__ img, const float *__restrict__ fflow, const float *__restrict__ bflow,
                     const uint32_t *__restrict__ gpos, const uint32_t *__restrict__ gtile,
                     const TileBox *__restrict__ tiles, StepConst sc, int step, int maxCand,
-                    uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_nsim, int G,
-                    const uint32_t *__restrict__ list_count, const uint32_t *__restrict__ list,
+                    uint32_t *__restrict__ out_idx, uint32_t *__restrict__ out_nsim, int G, RedoList list,
                     uint32_t *__restrict__ tie_count, uint32_t *__restrict__ tie_list)
 {
-	const uint32_t n = min(*list_count, (uint32_t)G);
-	for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-		bm_group<false>((int)list[i], img, fflow, bflow, gpos, gtile, tiles, sc, step, maxCand, out_idx, out_nsim, G,
+	const int n = list.count();
+	for (int i = list.first(); i < n; i += list.step()) {
+		bm_group<false>(list.at(i), img, fflow, bflow, gpos, gtile, tiles, sc, step, maxCand, out_idx, out_nsim, G,
 		                tie_count, tie_list, G);
 		__syncthreads();
 	}
@@ -1773,7 +1774,7 @@ void bm_list_kernel(const float *__restrict__ img, const float *__restrict__ ffl
 
 #define BMB_ARGS const float *, const int16_t *, const uint32_t *, const float2 *, const int4 *, const int2 *, \
 	const uint32_t *, const uint32_t *, const TileBox *, StepConst, int, int, uint32_t *, uint32_t *, int,    \
-	uint32_t *, uint32_t *, uint32_t *, uint32_t *
+	uint32_t *, uint32_t *, RedoList
 #define BMB_INST(PX, PT)                                                   \
 	template __global__ void bm_bound_kernel<PX, PT, false, false>(BMB_ARGS); \
 	template __global__ void bm_bound_kernel<PX, PT, false, true>(BMB_ARGS);  \

@@ -232,7 +232,10 @@ int bm4dof_last_timings(const bm4dof_ctx *ctx, float *ms, const char **names, in
  * stats[5..6] = groups and group rows (patches over all groups) of step 1,
  * stats[7..8] = the same for step 2; stats[9] = executed TV-L1 iterations
  * times pixels, summed over pairs, scales and warps, of the last flow
- * computation on the context.  Returns the number of slots filled. */
+ * computation on the context; stats[10..11] = groups of each step that the
+ * matching by bounded distances left to another matcher, -1 where the step did
+ * not take it; stats[12..13] = chunks of groups each step was filtered in.
+ * Returns the number of slots filled. */
 int bm4dof_last_stats(const bm4dof_ctx *ctx, int64_t *stats, int max_slots);
 
 /* ---- batches and the autotuner ----
