@@ -2303,6 +2303,9 @@ int bm4dof_ctx_set_option(bm4dof_ctx *ctx, const char *key, long long value)
 			ctx->coef_budget = (size_t)value;
 			std::lock_guard<std::mutex> lk(g_idle_mu);
 			idle_free(ctx->device, 0);
+		} else if (k == "est_budget") {
+			if (value <= 0) throw ArgError("est_budget must be positive");
+			ctx->est_budget = (size_t)value;
 		} else if (k == "keep_tables") {
 			ctx->keep_tables = value != 0;
 		} else if (k == "vbm3d_search") {

@@ -143,6 +143,10 @@ const char *bm4dof_global_error(void);
  *                  whose tables do not fit the budget or the free device
  *                  memory transform the patches group by group; the output
  *                  is the same either way.  0 disables the tables.
+ *   "est_budget"   bytes of device memory a step may hold in estimated patches
+ *                  (each group's rows, C*P floats a patch; default 24 GiB):
+ *                  groups beyond it are filtered and aggregated in further
+ *                  chunks of consecutive groups.
  *   "vbm3d_search" 0 (default): block matching as the reference builds it;
  *                  1: the predictive search of a build with VBM3D_SEARCH
  *                  defined (src/core/nldct.h:20; nldct.cpp:904-1130,
