@@ -909,10 +909,11 @@ BinBufs bin_bufs(bm4dof_ctx *ctx, const StepConst &sc, int64_t Mub)
 	const size_t npair = (size_t)8 * Mub;
 	BinBufs q;
 	q.rt = sort_tile(Mub, 256, BIN_RT);
-	q.ipt = sort_tile((int64_t)(npair / RS_THREADS), 16, RS_IPT);
+	q.ipt = sort_tile((int64_t)((npair + RS_THREADS - 1) / RS_THREADS), 16, RS_IPT);
 	q.nblk = (int)((npair + RS_THREADS * q.ipt - 1) / (RS_THREADS * q.ipt));
 	q.nt1 = (int)((Mub + q.rt - 1) / q.rt);
-	// fewer rows may take more tiles, up to SORT_TILES
+	// fewer rows may take more tiles, up to SORT_TILES (sort_tile, whose n
+	// counts a rest as a whole)
 	const size_t m1 = std::max(q.nt1, SORT_TILES), mb = std::max(q.nblk, SORT_TILES);
 	q.off1 = ctx->bin_cnt.as<uint32_t>(256 * m1 + 1);
 	q.k0 = ctx->bin_k0.as<uint32_t>(npair);

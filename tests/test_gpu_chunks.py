@@ -39,3 +39,39 @@ def test_chunks_equal_one(px, pt, np_, f, c, opt):
     for b, o in out[1:]:
         assert np.array_equal(out[0][0], b, equal_nan=True) and np.array_equal(out[0][1], o, equal_nan=True)
     assert np.isfinite(out[0][1]).mean() > 0.5     # (colour: no number where no patch lies)
+
+
+def test_last_chunk_of_a_captured_step():
+    """A last chunk of 131075 rows takes as many sort tiles of the smallest
+    size as a chunk may have; the buffers were sized for a larger first chunk,
+    whose tiles are larger and half as many.  Nothing may grow in a capture."""
+    import torch
+    noisy = torch.from_numpy(synth.add_noise(synth.video(81, 81, 1, n_shapes=6, seed=4), 20.0, 5)).cuda()
+    p1, p2 = (A.cli_params(s, 20.0, noisy.shape, px=8, pt=1, wx=9, np_=49) for s in (1, 2))
+    p1.offSet = p2.offSet = 1
+    one = [torch.zeros_like(noisy) for _ in range(2)]
+    many = [torch.zeros_like(noisy) for _ in range(2)]
+    torch.cuda.synchronize()
+    ctx = A.Context(0)
+    try:
+        ctx.run_dev(p1, p2, noisy.data_ptr(), noisy.shape, None, None, one[0].data_ptr(), one[1].data_ptr(), nparts=1)
+        groups = ctx.stats()["groups1"]
+        assert groups == ctx.stats()["groups2"] and 2 * 2675 < groups < 2675 + 5350
+    finally:
+        ctx.close()
+    ctx = A.Context(0)
+    try:
+        ctx.set_option("est_budget", (groups - 2675) * 49 * 64 * 4)
+        seq = A.Seq(noisy.data_ptr(), None, None, many[0].data_ptr(), many[1].data_ptr(), 81, 81, 1)
+        batch = ctx.batch([seq], [p1], [p2], nparts=1, graph=True)
+        for _ in range(3):
+            for m in many:
+                m.zero_()
+            torch.cuda.synchronize()
+            batch.run()
+            torch.cuda.synchronize()
+            for a, b in zip(one, many):
+                assert torch.equal(a, b)
+        batch.close()
+    finally:
+        ctx.close()
