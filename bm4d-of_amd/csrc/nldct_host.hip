@@ -561,6 +561,9 @@ static void bm_ties(bm4dof_ctx *ctx, const StepConst &sc, int step, const float 
 // and against bm_kernel, the only other one for their sizes: 7x7x1, 3e7:
 // .35 / 1.39; 11x11x1, 39x39, 1.2e7: .48 / .82.
 constexpr int BMQ_RANGE_BLOCKS = 512;
+// The window records hold places inside a tile in 16 bits each; larger images
+// take the general matcher.
+static bool windows_fit(const StepConst &sc) { return sc.W <= 65536 && sc.H <= 65536; }
 static bool bm_bound_ok(const StepConst &sc, int step, int G)
 {
 	const int nch = step == 1 ? 1 : sc.C;
@@ -569,7 +572,7 @@ static bool bm_bound_ok(const StepConst &sc, int step, int G)
 	// what the kernels hold: scan indices in 16 bits, places' byte offsets in
 	// 32, a lane per frame; past 512 samples the float sums' own rounding
 	// would leave the bound's slack
-	if (sc.npmax <= 1 || sc.P * nch > 512 || sc.wtf + sc.wtb + 1 > 64 ||
+	if (!windows_fit(sc) || sc.npmax <= 1 || sc.P * nch > 512 || sc.wtf + sc.wtb + 1 > 64 ||
 	    (int64_t)sc.sWx * sc.sWx * (sc.wtf + sc.wtb + 1) >= 65536 || (int64_t)sc.WH * sc.F >= ((int64_t)1 << 28))
 		return false;
 	if (sc.sPx == 4 && sc.sPt == 4) return all >= 4000000;
@@ -687,7 +690,7 @@ void run_bm(bm4dof_ctx *ctx, const StepConst &sc, int step, const float *img, co
 	// step 2 sums all channels (the register kernel takes any channel count,
 	// the LDS-staged one a single channel)
 	const int PX = sc.sPx, PT = sc.sPt;
-	const bool shape_ok = (PX == 4 && PT == 4) || (PX == 8 && PT == 1);
+	const bool shape_ok = windows_fit(sc) && ((PX == 4 && PT == 4) || (PX == 8 && PT == 1));
 	const int NF = ctx->bm_frames;   // frames staged per round: 1, 2 or 4
 	const size_t stage_floats = std::max<size_t>((size_t)NF * (sc.sWx + PX - 1) * (sc.sWx + PX - 1) * PT,
 	                                             (size_t)maxCand);

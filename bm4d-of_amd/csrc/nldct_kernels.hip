@@ -758,6 +758,9 @@ void bm_pred_kernel(const float *__restrict__ img, const float *__restrict__ ffl
 // sequential (ht, hy, hx) sum of the reference (nldct.cpp:1262-1274,
 // 1723-1737).  Selection as bm_kernel.
 // ---------------------------------------------------------------------------
+// Rows of a window's first candidate below its tile's first (16 bits, unsigned).
+__device__ __forceinline__ int win_y(const int4 &f) { return (int)((uint32_t)f.y >> 16); }
+
 __global__ void bm_window_kernel(const float *__restrict__ fflow, const float *__restrict__ bflow,
                                  const uint32_t *__restrict__ gpos, const uint32_t *__restrict__ gtile,
                                  const TileBox *__restrict__ tiles, StepConst sc, int G,
@@ -789,7 +792,7 @@ __global__ void bm_window_kernel(const float *__restrict__ fflow, const float *_
 		const int rx1 = min(Wt - sPx, cx + half - shift_x);
 		const int ry1 = min(Ht - sPx, cy + half - shift_y);
 		const int nx = max(0, rx1 - rx0 + 1), ny = max(0, ry1 - ry0 + 1);
-		wins[(size_t)g * sWt + ii] = make_int4(qt, rx0 | (ry0 << 16), nx | (ny << 16), base);
+		wins[(size_t)g * sWt + ii] = make_int4(qt, (int)((uint32_t)rx0 | ((uint32_t)ry0 << 16)), nx | (ny << 16), base);
 		base += nx * ny;
 		ii++;
 	};
@@ -925,7 +928,7 @@ __device__ void bm_emit(const uint32_t *__restrict__ out_key, const int *__restr
 			const int4 f = gw[ii];
 			const int o = r - f.w;
 			const int nx = f.z & 0xffff;
-			const int qy = (f.y >> 16) + o / nx, qx = (f.y & 0xffff) + o % nx;
+			const int qy = win_y(f) + o / nx, qx = (f.y & 0xffff) + o % nx;
 			q = (uint32_t)f.x * (uint32_t)sc.WH + (uint32_t)(qy + tb.oy) * (uint32_t)sc.W + (uint32_t)(qx + tb.ox);
 		}
 		oidx[lane] = q;
@@ -1004,7 +1007,7 @@ void bm_fast_kernel(const float *__restrict__ img, const int4 *__restrict__ wins
 			const int ht = r / (rw[j] * rh[j]);
 			const int q = r - ht * rw[j] * rh[j];
 			const int yy = q / rw[j], xx = q - yy * rw[j];
-			const int ax = tb.ox + (f[j].y & 0xffff) + xx, ay = tb.oy + (f[j].y >> 16) + yy;
+			const int ax = tb.ox + (f[j].y & 0xffff) + xx, ay = tb.oy + win_y(f[j]) + yy;
 			stage[i] = img[(size_t)(f[j].x + ht) * sc.WHC + (size_t)ay * sc.W + ax];
 		}
 		__syncthreads();
@@ -1035,7 +1038,7 @@ void bm_fast_kernel(const float *__restrict__ img, const int4 *__restrict__ wins
 	int s_self;
 	{
 		const int4 f0 = gw[0];
-		s_self = f0.w + (py - (f0.y >> 16)) * (f0.z & 0xffff) + (px - (f0.y & 0xffff));
+		s_self = f0.w + (py - win_y(f0)) * (f0.z & 0xffff) + (px - (f0.y & 0xffff));
 	}
 	const int nSimP = min(sc.npmax, nsrch);
 	int kk = 1;
@@ -1177,7 +1180,7 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 			const int r = loc / nx, cx = loc - r * nx;
 			const int y0 = r * ny / rchunks, y1 = (r + 1) * ny / rchunks;
 			if (y0 >= y1) continue;
-			const float *p = imc + (size_t)f.x * sc.WHC + (size_t)(tb.oy + (f.y >> 16)) * sc.W +
+			const float *p = imc + (size_t)f.x * sc.WHC + (size_t)(tb.oy + win_y(f)) * sc.W +
 			                 (tb.ox + (f.y & 0xffff) + cx);
 			uint32_t *kout = skey + f.w + cx;
 			float w[PX][PT][PX];
@@ -1213,7 +1216,7 @@ void bm_reg_kernel(const float *__restrict__ img, const int4 *__restrict__ wins,
 	int s_self;
 	{
 		const int4 f0 = gw[0];
-		s_self = f0.w + (py - (f0.y >> 16)) * (f0.z & 0xffff) + (px - (f0.y & 0xffff));
+		s_self = f0.w + (py - win_y(f0)) * (f0.z & 0xffff) + (px - (f0.y & 0xffff));
 	}
 	const int nSimP = min(sc.npmax, nsrch);
 	int kk = 1;
@@ -1534,7 +1537,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
 	const int nx = min(full, tb.ex - tb.ox - PX + 1), ny = min(full, tb.ey - tb.oy - PX + 1);
 	if (lane < nframes) {
 		const int4 f = gw[lane];
-		f_at[lane] = (uint32_t)f.x * (uint32_t)WH + (uint32_t)(tb.oy + (f.y >> 16)) * (uint32_t)W +
+		f_at[lane] = (uint32_t)f.x * (uint32_t)WH + (uint32_t)(tb.oy + win_y(f)) * (uint32_t)W +
 		             (uint32_t)(tb.ox + (f.y & 0xffff));
 		f_qt[lane] = f.x;
 	}
@@ -1712,7 +1715,7 @@ void bm_bound_kernel(const float *__restrict__ img, const int16_t *__restrict__ 
 	int gx, gy, gt;
 	pos_decode(pos, W, WH, gx, gy, gt);
 	const int4 f0 = gw[0];
-	const int s_self = (gy - tb.oy - (f0.y >> 16)) * nx + (gx - tb.ox - (f0.y & 0xffff));
+	const int s_self = (gy - tb.oy - win_y(f0)) * nx + (gx - tb.ox - (f0.y & 0xffff));
 	// the reference's distances of what stays: channels, frames, rows, columns
 	const float *a0 = img + (size_t)gt * sc.WHC + (size_t)gy * W + gx;
 	for (int e = lane; e < cnt; e += 64) {
