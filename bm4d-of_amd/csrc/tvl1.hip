@@ -364,9 +364,9 @@ template <bool POS> __device__ __forceinline__ double sqrt_sum_sq(double s)
 	return __builtin_amdgcn_class(s, 0x260) ? s : g;   // +-0 and +inf give themselves
 }
 
-// a / d for several a and one finite d: a times the reciprocal in double
-// (two Newton steps from the float one, within 2^-51), rounded to float.  The
-// quotient of two floats is 2^-49 or more away, relatively, from where two
+// a / d for several a and one d below 2^126 (whose float reciprocal is then a
+// normal number): a times the reciprocal in double (two Newton steps from the
+// float one, within 2^-51), rounded to float.  The quotient of two floats is 2^-49 or more away, relatively, from where two
 // floats meet, so this is the correctly rounded quotient (of results below
 // 2^-126 the last bit can differ).
 __device__ __forceinline__ double tv_recip(float d)
@@ -379,14 +379,14 @@ __device__ __forceinline__ double tv_recip(float d)
 __device__ __forceinline__ float tv_quot(float a, double y) { return (float)((double)a * y); }
 
 // Phase A of a pixel: TH, divergence (dp1, dp2), u (tvl1flow_lib.c:170-225).
-// yg: tv_recip(g), 0 where g < TV_GRAD_IS_ZERO (the quotient then comes out
-// 0, as the reference sets it).  Returns the squared update.
+// yg: the reciprocal of g; flat: g < TV_GRAD_IS_ZERO, where the reference sets
+// the quotient 0 (also of a rho that is no number).  Returns the squared update.
 __device__ __forceinline__ float tv_pixel_u(float &u1, float &u2, float dp1, float dp2, float wx, float wy, float g,
-                                            double yg, float rc, float l_t, float theta)
+                                            double yg, bool flat, float rc, float l_t, float theta)
 {
 	const float rho = rc + (wx * u1 + wy * u2);
 	const float lg = l_t * g;
-	float fi = tv_quot(-rho, yg);
+	float fi = flat ? 0.f : tv_quot(-rho, yg);
 	fi = rho > lg ? -l_t : fi;
 	fi = rho < -lg ? l_t : fi;
 	const float v1 = u1 + fi * wx, v2 = u2 + fi * wy;
@@ -420,7 +420,7 @@ __device__ __forceinline__ void tv_pixel_p(float &p11, float &p12, float &p21, f
 	p12 = tv_quot(b12, y1);
 	p21 = tv_quot(b21, y2);
 	p22 = tv_quot(b22, y2);
-	if (__builtin_expect(!(ng1 + ng2 < INFINITY), 0)) {
+	if (__builtin_expect(!(ng1 + ng2 < 0x1p126f), 0)) {
 		asm volatile("");   // (a branch, not both sides)
 		ng1 = 1.0f + taut * (float)sqrt_sum_sq<false>((double)u1x * u1x + (double)u1y * u1y);
 		ng2 = 1.0f + taut * (float)sqrt_sum_sq<false>((double)u2x * u2x + (double)u2y * u2y);
@@ -445,6 +445,7 @@ template <int R> struct TVRows {
 	float u1[R], u2[R], p11[R], p12[R], p21[R], p22[R];
 	float wx[R], wy[R], rc[R], g[R];
 	double yg[R];
+	bool flat[R];
 };
 // Rows the waves hand to each other: the first row's u, the last row's p12
 // and p22.
@@ -480,7 +481,8 @@ __device__ __forceinline__ void tv_iterate(TVRows<R> &t, TVEdge<W> &L, int wv, i
 				dp1 = side ? (h1 + t.p12[r]) - a12u : dp1;
 				dp2 = side ? (h2 + t.p22[r]) - a22u : dp2;
 			}
-			const float q = tv_pixel_u(t.u1[r], t.u2[r], dp1, dp2, t.wx[r], t.wy[r], t.g[r], t.yg[r], t.rc[r], l_t, theta);
+			const float q = tv_pixel_u(t.u1[r], t.u2[r], dp1, dp2, t.wx[r], t.wy[r], t.g[r], t.yg[r], t.flat[r],
+			                           t.rc[r], l_t, theta);
 			if (y >= 0 && y < TY) ej += (double)(own ? q : 0.f);
 		}
 #pragma unroll
@@ -558,8 +560,11 @@ void tv_iter_kernel(const float *__restrict__ I1wx, const float *__restrict__ I1
 		t.rc[r] = at(rho_c + off, o);
 	}
 #pragma unroll
-	for (int r = 0; r < R; r++)
-		t.yg[r] = t.g[r] < TV_GRAD_IS_ZERO || t.g[r] == INFINITY ? 0.0 : tv_recip(t.g[r]);
+	for (int r = 0; r < R; r++) {
+		t.flat[r] = t.g[r] < TV_GRAD_IS_ZERO;
+		t.yg[r] = tv_recip(t.g[r]);
+		if (__any(!(t.g[r] < 0x1p126f))) t.yg[r] = 1.0 / (double)t.g[r];
+	}
 	L.p[wv][0][lane] = t.p12[R - 1];
 	L.p[wv][1][lane] = t.p22[R - 1];
 	double err[K];
