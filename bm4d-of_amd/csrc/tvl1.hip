@@ -842,6 +842,20 @@ inline int tv_part_tiles(const TVPlan &pl)
 	return m;
 }
 
+// Partial sums that the account of the fixed scratch counts, which decides the
+// pairs that fit it: one per 32 x 16 pixels, or per 64 x 32 where those are 1024
+// or more.  (The sums' own number depends on the tiles; bm4dof_tvl1_noalloc
+// keeps them elsewhere.)
+inline int tv_account_tiles(const TVPlan &pl)
+{
+	int m = 0;
+	for (int s = 0; s < pl.nscales; s++) {
+		const int l = ((pl.nx[s] + 63) / 64) * ((pl.ny[s] + 31) / 32);
+		m = std::max(m, l >= 1024 ? l : ((pl.nx[s] + 31) / 32) * ((pl.ny[s] + 15) / 16));
+	}
+	return m;
+}
+
 // Byte offsets of the parts of a TVScratch carved from one region, and the
 // region's size (the last entry), each part 256-byte aligned.
 std::array<size_t, 8> tv_scratch_layout(const TVPlan &pl, size_t size0)
@@ -854,7 +868,7 @@ std::array<size_t, 8> tv_scratch_layout(const TVPlan &pl, size_t size0)
 	o[2] = o[1] + al(pl.pyr * 4 * sizeof(float));                      // working planes
 	o[3] = o[2] + al(P * size0 * TV_WORK * sizeof(float));             // min/max
 	o[4] = o[3] + al(P * TV_MMB * 4 * sizeof(float));                  // iteration partial sums
-	o[5] = o[4] + al(P * TV_K * (size_t)tv_part_tiles(pl) * sizeof(double));
+	o[5] = o[4] + al(P * TV_K * (size_t)tv_account_tiles(pl) * sizeof(double));
 	o[6] = o[5] + al((5 * P + 1) * sizeof(int));                       // taps
 	o[7] = o[6] + al(64 * sizeof(double));                             // total
 	return o;
@@ -1141,8 +1155,12 @@ int bm4dof_tvl1_noalloc(bm4dof_ctx *ctx, const bm4dof_tvl1_params *prm, const fl
 			               " bytes of scratch; the fixed scratch holds " +
 			               std::to_string((size_t)BM4DOF_TVL1_NOALLOC_BYTES));
 		char *b = (char *)base;
-		const TVScratch t = tv_scratch_carve(b, lay);
+		TVScratch t = tv_scratch_carve(b, lay);
 		float *fr = (float *)(b + lay[7]);
+		// the partial sums over the frames, which nothing reads after their
+		// normalisation (32 bytes a tile of at least 56 x 8 pixels, or of the
+		// pair where it is smaller; 8 bytes a pixel of at least 9)
+		t.part = (double *)fr;
 		HIPCHK(hipMemcpyAsync(fr, I0, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
 		HIPCHK(hipMemcpyAsync(fr + n, I1, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
 		tv_flow_pairs(ctx, *prm, fr, nx, ny, {0}, {1}, u1, u2, iters, &t);
