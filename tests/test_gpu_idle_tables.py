@@ -68,3 +68,32 @@ def test_tables_stay_idle_between_calls_and_go_back():
     finally:
         for c in made:
             c.close()
+
+
+def test_contexts_on_threads_share_idle_tables():
+    """Two contexts, each on its own thread, on clips of different sizes in turn:
+    the blocks change hands between calls."""
+    import threading
+    clips = [synth.add_noise(synth.video(w, 60, 6, n_shapes=5, seed=w), 20.0, 3) for w in (72, 96, 140)]
+    prm = [[A.cli_params(s, 20.0, v.shape, px=4, pt=4, wx=7, np_=8) for s in (1, 2)] for v in clips]
+    ctxs = [A.Context(0) for _ in range(2)]
+    try:
+        want = [ctxs[0].run(*p, v, nparts=2)[:2] for p, v in zip(prm, clips)]
+        wrong = []
+
+        def go(k):
+            for i in range(12):
+                j = (i * (k + 1) + k) % 3
+                b, f, _ = ctxs[k].run(*prm[j], clips[j], nparts=2)
+                if not (np.array_equal(b, want[j][0]) and np.array_equal(f, want[j][1])):
+                    wrong.append((k, i))
+
+        threads = [threading.Thread(target=go, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(60)
+        assert not wrong and not any(t.is_alive() for t in threads)
+    finally:
+        for c in ctxs:
+            c.close()
