@@ -398,9 +398,6 @@ def main():
     d_final = torch.empty_like(d_noisy)
     torch.cuda.synchronize()
     ctx = A.Context(0)
-    # a caller that denoises videos of one shape repeatedly keeps the
-    # coefficient tables between calls (the default frees them at each end)
-    ctx.set_option("keep_tables", 1)
 
     # flows of the sequence (a first call sizes the buffers; the second is timed)
     ctx.tvl1_sequence_dev(d_noisy.data_ptr(), W, H, F, d_ff.data_ptr(), d_bf.data_ptr())

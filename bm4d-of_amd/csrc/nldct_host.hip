@@ -560,6 +560,7 @@ static void bm_ties(bm4dof_ctx *ctx, const StepConst &sc, int step, const float 
 //     2.28 / 2.34; 7x7x9 (441), 4e7: .72 / .65
 // and against bm_kernel, the only other one for their sizes: 7x7x1, 3e7:
 // .35 / 1.39; 11x11x1, 39x39, 1.2e7: .48 / .82.
+constexpr int GPU_CUS = 256;   // of the MI355X
 constexpr int BMQ_RANGE_BLOCKS = 512;
 // The window records hold places inside a tile in 16 bits each; larger images
 // take the general matcher.
@@ -570,8 +571,8 @@ static bool bm_bound_ok(const StepConst &sc, int step, int G)
 	const int64_t cand = (int64_t)sc.sWx * sc.sWx * std::max(1, std::min(sc.wtf + sc.wtb + 1, sc.F - sc.sPt + 1));
 	const int64_t all = cand * G;
 	// what the kernels hold: scan indices in 16 bits, places' byte offsets in
-	// 32, a lane per frame; past 512 samples the float sums' own rounding
-	// would leave the bound's slack
+	// 32, a lane per frame; the float sums' own rounding has to stay within
+	// the bound's slack, 2 (samples + 2) 2^-24 < 1e-4 (bmq_limit)
 	if (!windows_fit(sc) || sc.npmax <= 1 || sc.P * nch > 512 || sc.wtf + sc.wtb + 1 > 64 ||
 	    (int64_t)sc.sWx * sc.sWx * (sc.wtf + sc.wtb + 1) >= 65536 || (int64_t)sc.WH * sc.F >= ((int64_t)1 << 28))
 		return false;
@@ -1186,22 +1187,19 @@ StepDev upload_plan(bm4dof_ctx *ctx, const StepPlan &pl, DevBuf &geo_buf)
 	return d;
 }
 
-// Grows every shared work buffer a plan's launches use, so that enqueueing
-// the step allocates nothing (required while a stream is being captured).
-// Runs of 16 anchors along x over one channel plane, 0 when the patch does not
-// fit the video.
-int64_t coef_waves(const StepConst &sc)
+// Runs of 32 anchors along x over one channel plane (one wave's round of
+// coef_kernel), 0 when the patch does not fit the video.
+int64_t coef_runs(const StepConst &sc)
 {
 	const int nx = sc.W - sc.sPx + 1, ny = sc.H - sc.sPx + 1, nt = sc.F - sc.sPt + 1;
-	return nx > 0 && ny > 0 && nt > 0 ? (int64_t)((nx + 15) / 16) * ny * nt : 0;
+	return nx > 0 && ny > 0 && nt > 0 ? (int64_t)((nx + 31) / 32) * ny * nt : 0;
 }
 
 // Floats of one image's coefficient table for a step that uses them (the
 // register filters of a plain step, within coef_budget), else 0.
 size_t coef_floats(const StepPlan &pl, size_t budget)
 {
-	const int64_t waves = coef_waves(pl.sc);
-	if (!pl.fast || !pl.fast_shape || pl.learned || waves <= 0 || waves * 64 >= ((int64_t)1 << 32)) return 0;
+	if (!pl.fast || !pl.fast_shape || pl.learned || coef_runs(pl.sc) <= 0) return 0;
 	const size_t per = (size_t)pl.C * pl.WHF * pl.sc.P;
 	return per * sizeof(float) * (pl.step1 ? 1 : 2) <= budget ? per : 0;
 }
@@ -1282,6 +1280,8 @@ void table_put(bm4dof_ctx *ctx, DevBuf &b)
 	b.n = 0;
 }
 
+// Grows every shared work buffer a plan's launches use, so that enqueueing
+// the step allocates nothing (required while a stream is being captured).
 void reserve_step(bm4dof_ctx *ctx, const StepPlan &pl)
 {
 	const size_t G = (size_t)std::max(pl.G, 1), np = (size_t)pl.np;
@@ -1354,8 +1354,8 @@ static void coef_tables(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, 
 	const size_t WHF = pl.WHF;
 	const int nimg = step1 ? 1 : 2;
 	const size_t per = coef_floats(pl, ctx->coef_budget);
-	// blocks of four waves, 32 anchors a wave and round
-	const unsigned blocks = (unsigned)std::min<int64_t>((coef_waves(sc) + 7) / 8, 4096);
+	// blocks of four waves, which loop
+	const unsigned blocks = (unsigned)std::min<int64_t>((coef_runs(sc) + 3) / 4, 4096);
 	d_coef_n = d_coef_b = nullptr;
 	if (per > 0 && ctx->coef_n.n >= per * sizeof(float) && (step1 || ctx->coef_b.n >= per * sizeof(float))) {
 		const bool have_n = !step1 && ctx->coef_n_keep && ctx->coef_n_ok && ctx->coef_n_whf == WHF &&
@@ -1540,7 +1540,7 @@ void enqueue_step(bm4dof_ctx *ctx, const StepPlan &pl, const StepDev &dv, const 
 				// a block lays out 100 KB of tables and fills a CU: one each (1024
 				// blocks: the same at 960x540x20, .96 against .91 ms at 300x200x7)
 				hipLaunchKernelGGL(sc.sPx == 4 ? filter_learned_kernel<4> : filter_learned_kernel<8>,
-				                   dim3((unsigned)std::min(nblk(Gc, 8), 256)), dim3(512), 0, ctx->stream, d_nplanes + (size_t)c * WHF, d_idx, d_nsim, d_base,
+				                   dim3((unsigned)std::min(nblk(Gc, 8), GPU_CUS)), dim3(512), 0, ctx->stream, d_nplanes + (size_t)c * WHF, d_idx, d_nsim, d_base,
 				                   dv.gtile, sc, g0, Gc, dv.bsp, dv.win, la->net, la->sigma,
 				                   la->gvar_thr, d_est, d_ew, d_etile, d_early, d_gw, d_gflag, la->nflag, C, c);
 		else if (pl.fast && step1) {

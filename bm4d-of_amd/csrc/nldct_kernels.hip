@@ -1318,11 +1318,13 @@ template __global__ void bm_reg_kernel<8, 1, true, true>(BMR_ARGS);
 // most 1.001 sqrt(PC).  With T at or above the kk-th smallest D, the kk-th
 // smallest true distance is at most (sqrt(T) + 1.001 sqrt(PC))^2 units, and a
 // candidate with D > (sqrt(T) + 2.002 sqrt(PC))^2 lies above it.  The float
-// sums' own rounding (below 2e-5 of a distance) is in the slack of
-// bmq_limit.  What stays, some 40 to 100 candidates, is summed and ranked
-// exactly as bm_reg_kernel does it.  Groups with more than BMQ_CAP left, with
-// too few candidates to bound, or an image without a finite range are listed
-// and matched again (bm_reg_kernel or bm_list_kernel).
+// sums' own rounding, at most (PC + 2) 2^-24 of a distance each, is in the
+// slack of bmq_limit: 1e-4, which has to exceed twice that (6.2e-5 at the 512
+// samples that bm_bound_ok admits).  What stays, some 40 to 100 candidates, is summed and ranked
+// exactly as bm_reg_kernel does it.  Groups with more than BMQ_CAP left or with
+// too few candidates to bound are listed and matched again (bm_reg_kernel or
+// bm_list_kernel), all groups where the image has no finite range or one that
+// leaves its noise few integer steps (scale 0).
 // ---------------------------------------------------------------------------
 #define BMQ_CAP 256
 
@@ -2105,17 +2107,17 @@ void filter2_kernel(const float *__restrict__ noisy, const float *__restrict__ b
 }
 
 // ---------------------------------------------------------------------------
-// Register-resident filter for one-channel groups of 64-sample patches
-// (px=4/pt=4 or px=8/pt=1) with at most 32 neighbours: one wave per group.
+// Register-resident filters for groups with at most 32 neighbours, one channel
+// a launch, one wave per group: 64-sample patches (px=4/pt=4 or px=8/pt=1),
+// in step 2 also 7x7 pixels of one frame, and with two waves per group patches
+// of 65 to 128 samples (filter2_wide_kernel).
 //
-// Forward transform: lane k holds row k of the basis in registers; the
-// samples of patch n are wave-uniform and arrive through scalar loads, so
-// each coefficient z[k][n] is a register dot product in pixel order.
-// Haar along the group and the threshold / Wiener shrinkage then run inside
-// each lane (lane k owns coefficient k of every patch).  Inverse transform:
-// lane pix holds column pix of the inverse basis; the coefficients of
-// patch n are read from LDS as wave-uniform (broadcast) values, sequential
-// in k.  Same arithmetic, same order as filter1_kernel / filter2_kernel.
+// Lane k owns coefficient k of every patch: the coefficients come from the
+// tables of all anchors (coef_kernel) or from the fp32 matrix instructions,
+// Haar along the group and the threshold / Wiener shrinkage run inside each
+// lane, and the inverse transform is another product on the matrix
+// instructions, whose operands go through LDS.  Same arithmetic, same order as
+// filter1_kernel / filter2_kernel.
 // ---------------------------------------------------------------------------
 
 #define FAST_P 64

@@ -104,14 +104,19 @@ const char *bm4dof_global_error(void);
  * execution is fixed).  All but "vbm3d_search" select between kernels that
  * compute the same result; outputs do not depend on them.  Keys:
  *   "fast_filter"  1 (default): register-resident group filter where the
- *                  group shape allows it (64-sample patches, fewer than 64
- *                  similar patches, no orderInvariance; colour one launch
+ *                  group shape allows it (fewer than 64 similar patches, no
+ *                  orderInvariance; 4x4x4 or 8x8x1 patches, in step 2 also
+ *                  7x7x1 and patches of 65 to 128 samples; colour one launch
  *                  per channel); 0: the general LDS filter for every group.
- *   "fast_bm"      block matching for patches 4x4x4 or 8x8x1: 2 (default):
- *                  one wave per group, candidate windows in registers (any
- *                  channel count); 1: one wave per group on LDS-staged
- *                  search windows (one channel in the distance); 0: the
- *                  general kernel for every shape.
+ *   "fast_bm"      block matching: 2 (default): one wave per group, any channel
+ *                  count; where there are many candidates (4e6 for patches
+ *                  4x4x4 and 8x8x1, for these 640 a group too; 1e6 for 7x7x1
+ *                  and 11x11x1) by a bound of every distance on integer
+ *                  samples first, else with the windows in registers (4x4x4,
+ *                  8x8x1); 1: one wave per group on LDS-staged search windows
+ *                  (4x4x4 or 8x8x1, one channel in the distance); 0: the
+ *                  general kernel, which 1 and 2 use for all other patches and
+ *                  for images of more than 65536 pixels a side.
  *   "bm_frames"    frames of search window staged in LDS per round of the
  *                  LDS-staged block matching: 1, 2 (default) or 4.
  *   "agg_chunked"  1 (default): ordered aggregation by sorted row chunks
@@ -124,7 +129,8 @@ const char *bm4dof_global_error(void);
  *                  each region (8 x 8 pixels x 4 to 32 frames, 16 x 16 x 1
  *                  for one-frame patches other than 8x8) gets its rows as
  *                  one list in row order, built beside the filter, and one
- *                  wave folds the list into the region's sums; 0: the
+ *                  wave (four where there are fewer than 3000 regions) folds
+ *                  the list into the region's sums; 0: the
  *                  chunked aggregation sorts the rows of every 8 x 8 x 1
  *                  block itself.
  *   "coef_beside_bm" 1 (default): a gray step's coefficient tables are
