@@ -1209,8 +1209,8 @@ size_t coef_floats(const StepPlan &pl, size_t budget)
 // between half a millisecond and, when the driver has not cleared what was
 // freed, hundreds of them (480x270x12 of 8 bits: 8.9 ms a call, up to 25 with
 // it; 641x360x9 in colour 19.8 and 67 to 188).  So a call's end leaves them here, for
-// the next call on any context of the device, up to an eighth of its memory;
-// they are freed when an allocation of the library fails, when a context's
+// the next call on any context of the device, up to an eighth of its memory and
+// no more than the context's coef_budget; they are freed when an allocation of the library fails, when a context's
 // coef_budget is set, and with the device's last context.
 struct IdleBlock {
 	int device;
@@ -1269,12 +1269,13 @@ void table_get(bm4dof_ctx *ctx, DevBuf &b, size_t bytes)
 void table_put(bm4dof_ctx *ctx, DevBuf &b)
 {
 	if (!b.p) return;
-	if (b.n > ctx->idle_max) {
+	const size_t most = std::min(ctx->idle_max, ctx->coef_budget);
+	if (b.n > most) {
 		b.release();
 		return;
 	}
 	std::lock_guard<std::mutex> lk(g_idle_mu);
-	idle_free(ctx->device, ctx->idle_max - b.n);
+	idle_free(ctx->device, most - b.n);
 	g_idle.push_back({ctx->device, b.p, b.n});
 	b.p = nullptr;
 	b.n = 0;

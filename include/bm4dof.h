@@ -163,8 +163,9 @@ const char *bm4dof_global_error(void);
  *                  _run_learned(_dev) call the tables' memory becomes idle,
  *                  for the next call on any context of the device to take;
  *                  the library keeps at most an eighth of the device's memory
- *                  idle (the oldest blocks are freed beyond that, and larger
- *                  tables at once) and frees it when one of its allocations
+ *                  idle, and no more than the context's "coef_budget" (the
+ *                  oldest blocks are freed beyond that, and larger tables at
+ *                  once), and frees it when one of its allocations
  *                  fails, when a context's "coef_budget" is set (to any
  *                  value) and with the device's last context; 1: the tables
  *                  stay with the context.

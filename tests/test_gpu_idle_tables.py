@@ -60,6 +60,16 @@ def test_tables_stay_idle_between_calls_and_go_back():
         b3, f3, _ = a.run(p1, p2, noisy, nparts=2)
         for x, y in ((b1, f1), (b2, f2), (b3, f3)):
             assert np.array_equal(b0, x) and np.array_equal(f0, y)
+        a.set_option("coef_budget", 3 * TABLE)        # two tables fit, and may stay idle
+        before = _free()
+        a.run(p1, p2, noisy, nparts=2)
+        assert before - _free() >= 2 * TABLE - SLACK
+        small = synth.add_noise(synth.video(150, 136, 6, n_shapes=6, seed=2), 20.0, 3)
+        before = _free()
+        a.set_option("coef_budget", TABLE * 175 // 100)   # two of the smaller clip's
+        a.run(p1, p2, small, nparts=2)
+        a.run(p1, p2, noisy, nparts=2)                # only step 1's table fits: it displaces those
+        assert abs(_free() - before - TABLE) <= SLACK  # of the two blocks before one is left
         a.set_option("keep_tables", 1)                # with the context: not idle
         a.run(p1, p2, noisy, nparts=2)
         before = _free()
